@@ -20,6 +20,7 @@
 namespace tc {
 
 constexpr int NUFFT_W = 8;
+struct SpreadArgs;  // nufft.hip
 
 class PolarNufft {
  public:
@@ -54,10 +55,16 @@ class PolarNufft {
   // centre, which every ray crosses, are split over many workgroups.
   bool work_ready_ = false;
   int nwork_ = 0, nslots_ = 0, nfix_ = 0, chunk_ = 0;
-  std::vector<int> counts_;  // polar points per fine-grid tile
-  DevBuf work_;  // int4: tile, first point, end point, scratch slot (-1: none)
+  std::vector<int> counts_;      // polar points per fine-grid tile
+  std::vector<int> tile_first_;  // first segment of each tile
+  // ray segments of every tile (device lists, built once per geometry)
+  DevBuf seg_pj_, seg_off_, tile_seg_;
+  // two int4 per item: tile, first point, end point, scratch slot (-1: none);
+  // the tile's segment range
+  DevBuf work_;
   DevBuf fix_;   // int4: tile, first slot, slot count, 0
-  void count_tiles(hipStream_t stream);
+  SpreadArgs spread_args() const;
+  void make_segments(hipStream_t stream);
   void make_work(int chunk);
 };
 

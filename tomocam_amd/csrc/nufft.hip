@@ -65,19 +65,22 @@ static void gauss_legendre(int n, std::vector<double>& x, std::vector<double>& w
 
 // ---------------------------------------------------------------------------
 // spreading (type 1): each workgroup owns a T x T tile of the fine grid and
-// gathers every ray segment whose kernel footprint meets it (rays are
-// enumerated analytically, so no sorting and no global atomics).
+// adds every polar point whose kernel footprint meets it.  The ray segments
+// that meet a tile are enumerated analytically, once per geometry (no sorting
+// and no global atomics).
 // ---------------------------------------------------------------------------
 
 constexpr int SP_T = 32;
-constexpr int SP_SB = 4;
-constexpr int SP_LIST = 2048;
+constexpr int SP_LIST = 2048;  // most projection angles (11 bits of a segment)
 
 struct SpreadArgs {
   const float2* c;  // [nsl][P][N]
   float2* fine;     // [nsl][nf][nf]
   const double* ax;
   const double* ay;
+  const int* seg_pj;    // segments of all tiles: p | jlo << 11 | shift << 27
+  const int* seg_off;   // their first points' numbers within the tile
+  const int* tile_seg;  // [ntiles + 1] first segment of each tile
   int P, N, cidx, nf, nsl, ntx;
   double umax;
   float beta;
@@ -124,77 +127,7 @@ __device__ __forceinline__ int block_scan_incl(int v, int* wsum) {
 // partial tiles a fix-up pass adds.  Small grids (fewer than 4096 tiles, a
 // few workgroups per CU) take 512 so the central tiles, where every ray
 // passes, do not leave a tail; larger grids take 1024 (less fix-up).
-// Measured with the longest-first order below: 8 x 512^2 at 360 angles
-// 0.50 -> 0.44 ms with 512; 32 x 1454^2 at 720 angles 8.42 (1024) vs 8.75.
 static int spread_chunk(int ntiles) { return ntiles < 4096 ? 512 : 1024; }
-
-// Enumerates the ray segments (superset j ranges) of shift (U0, V0) whose
-// kernel footprints meet the tile window; leaves seg_pj[k] = p | jlo << 11
-// and exclusive offsets seg_off[0..nseg] in LDS and returns the number of
-// points.  Called by all 256 threads (contains barriers).
-__device__ int enumerate_segments(const SpreadArgs& a, double U0, double V0,
-                                  double lox, double hix, double loy,
-                                  double hiy, int* seg_pj, int* seg_off,
-                                  int* wsum, int* nseg_sh, int* nsg_out) {
-  const int tid = threadIdx.x;
-  // Deterministic compaction: thread t examines angles t, t+256, ... and
-  // writes its non-empty segments at a block-scanned offset, so every
-  // workgroup of the same tile sees the same segment order.
-  constexpr int MAXA = SP_LIST / 256;
-  int jl[MAXA], jh[MAXA];
-  int local = 0;
-#pragma unroll
-  for (int i = 0; i < MAXA; ++i) {
-    const int p = tid + 256 * i;
-    jl[i] = 1;
-    jh[i] = 0;
-    if (p < a.P) {
-      double tlo = -1e30, thi = 1e30;
-      ray_interval(a.ax[p], U0, lox, hix, tlo, thi);
-      ray_interval(a.ay[p], V0, loy, hiy, tlo, thi);
-      if (tlo <= thi) {
-        tlo = fmax(tlo, -(double)a.N - 2.0);
-        thi = fmin(thi, (double)a.N + 2.0);
-        jl[i] = max(0, (int)floor(tlo) + a.cidx - 1);
-        jh[i] = min(a.N - 1, (int)ceil(thi) + a.cidx + 1);
-      }
-    }
-    local += jl[i] <= jh[i];
-  }
-  __syncthreads();  // previous users of the segment arrays are done
-  const int incl0 = block_scan_incl(local, wsum);
-  int pos = incl0 - local;
-#pragma unroll
-  for (int i = 0; i < MAXA; ++i) {
-    if (jl[i] <= jh[i]) {
-      seg_pj[pos] = (tid + 256 * i) | (jl[i] << 11);
-      seg_off[pos] = jh[i] - jl[i] + 1;
-      ++pos;
-    }
-  }
-  if (tid == 255) *nseg_sh = incl0;
-  __syncthreads();
-  const int nsg = *nseg_sh;
-  const int per = (nsg + 255) >> 8;
-  const int start = tid * per;
-  int lsum = 0;
-  for (int k = 0; k < per; ++k)
-    if (start + k < nsg) lsum += seg_off[start + k];
-  const int incl = block_scan_incl(lsum, wsum);
-  int run = incl - lsum;
-  for (int k = 0; k < per; ++k) {
-    const int idx = start + k;
-    if (idx < nsg) {
-      const int c = seg_off[idx];
-      seg_off[idx] = run;
-      run += c;
-    }
-  }
-  if (tid == 255) seg_off[nsg] = incl;
-  __syncthreads();
-  *nsg_out = nsg;
-  return seg_off[nsg];
-}
 
 struct TileWindow {
   int X0, Y0, X1, Y1;
@@ -225,250 +158,326 @@ __device__ __forceinline__ bool shift_skipped(const SpreadArgs& a,
          V0 + a.umax <= w.loy || V0 - a.umax > w.hiy;
 }
 
-// points per tile (all shifts), for building the work list
-__global__ void __launch_bounds__(256) spread_count_kernel(SpreadArgs a,
-                                                           int* counts) {
-  __shared__ int seg_pj[SP_LIST];
-  __shared__ int seg_off[SP_LIST + 1];
-  __shared__ int wsum[4];
-  __shared__ int nseg;
-  const int tile = blockIdx.x;
-  const TileWindow w = tile_window(a, tile);
-  int tot = 0;
-  for (int ky = -1; ky <= 1; ++ky)
-    for (int kx = -1; kx <= 1; ++kx) {
-      const double U0 = 0.5 * a.nf + kx * (double)a.nf;
-      const double V0 = 0.5 * a.nf + ky * (double)a.nf;
-      if (shift_skipped(a, w, U0, V0)) continue;
-      int nsg;
-      tot += enumerate_segments(a, U0, V0, w.lox, w.hix, w.loy, w.hiy, seg_pj,
-                                seg_off, wsum, &nseg, &nsg);
-    }
-  if (threadIdx.x == 0) counts[tile] = tot;
+// grid origin of periodic copy `shift` (0 .. 8, row-major over ky, kx)
+__device__ __forceinline__ double2 shift_origin(const SpreadArgs& a,
+                                                int shift) {
+  const int ky = shift / 3 - 1, kx = shift - (shift / 3) * 3 - 1;
+  return make_double2(0.5 * a.nf + kx * (double)a.nf,
+                      0.5 * a.nf + ky * (double)a.nf);
 }
 
-// One workgroup per (work item, slice group): accumulates the points
-// [f0, f1) of its tile in LDS and writes the tile to the fine grid (first
-// chunk) or to a scratch slot (further chunks).  Points are taken in batches
-// of SP_BATCH: each thread first prepares one point (cell origin, offsets of
-// the first footprint cell, slice values, the 8-row bands of the tile its
-// footprint meets) in LDS; then wave w adds the batch's points that meet
-// band w (rows [8w, 8w + 8) of the tile, which it owns) with lane (a, b) on
-// footprint cell (a, b).  Owned rows make the read-add-write race-free
-// without atomics (LDS float atomics are ~30x slower than a plain
-// read-add-write here), and each cell sums its points in list order, so the
-// result is deterministic.  The segment list lives in dynamic LDS sized to
-// the number of angles.
-// Accumulator row stride (float2).  33 keeps a workgroup's LDS (41.5 KB
-// static plus 8 bytes per angle) within a third of the CU's 160 KB up to
-// 1639 angles, so three workgroups share a CU: at 1501 angles a 16 x 2908^2
-// backprojection takes 36.2 instead of 43.2 ms with stride 36 (two
-// workgroups per CU); at 720 and 360 angles, where stride 36 fits three as
-// well, strides 33, 34 and 36 time the same.
-constexpr int SP_RS = 33;
-constexpr int SP_BATCH = 128;
-static_assert(SP_SB == 4, "slice values are held as two float4 per point");
+// first footprint cell and its distance from the point, along one axis (fma
+// so that every kernel rounds the coordinate alike)
+__device__ __forceinline__ int first_cell(double origin, double t, double step,
+                                          float& frac) {
+  const double u = fma(t, step, origin);
+  const double c = ceil(u - 0.5 * NUFFT_W);
+  frac = (float)(c - u);
+  return (int)c;
+}
 
+// Segments of one tile, counted (FILL false: counts[tile] = points,
+// counts[ntiles + tile] = segments) or written to the plan's lists.  Thread t
+// examines angles t, t + 256, ... of each periodic copy, in turn; a segment is
+// trimmed to the samples whose footprints really meet the tile.  The order
+// (copy, then a block-scanned order of the angles) is fixed, so every call of
+// the geometry adds a tile's points in the same order.
+template <bool FILL>
+__global__ void __launch_bounds__(256)
+spread_segments_kernel(SpreadArgs a, int* counts, int* seg_pj, int* seg_off) {
+  __shared__ int wsum[4];
+  __shared__ int carry[2];
+  const int tile = blockIdx.x, tid = threadIdx.x;
+  const TileWindow w = tile_window(a, tile);
+  const int s0 = FILL ? a.tile_seg[tile] : 0;
+  int nseg = 0, npts = 0;
+  for (int shift = 0; shift < 9; ++shift) {
+    const double2 o = shift_origin(a, shift);
+    if (shift_skipped(a, w, o.x, o.y)) continue;
+    for (int p0 = 0; p0 < a.P; p0 += 256) {
+      const int p = p0 + tid;
+      int jl = 1, jh = 0;
+      if (p < a.P) {
+        const double ax = a.ax[p], ay = a.ay[p];
+        double tlo = -1e30, thi = 1e30;
+        ray_interval(ax, o.x, w.lox, w.hix, tlo, thi);
+        ray_interval(ay, o.y, w.loy, w.hiy, tlo, thi);
+        if (tlo <= thi) {
+          tlo = fmax(tlo, -(double)a.N - 2.0);
+          thi = fmin(thi, (double)a.N + 2.0);
+          jl = max(0, (int)floor(tlo) + a.cidx - 1);
+          jh = min(a.N - 1, (int)ceil(thi) + a.cidx + 1);
+          auto meets = [&](int j) {
+            float f;
+            const double t = (double)(j - a.cidx);
+            const int lx = first_cell(o.x, t, ax, f);
+            const int ly = first_cell(o.y, t, ay, f);
+            return lx < w.X1 && lx + NUFFT_W > w.X0 && ly < w.Y1 &&
+                   ly + NUFFT_W > w.Y0;
+          };
+          while (jl <= jh && !meets(jl)) ++jl;
+          while (jl <= jh && !meets(jh)) --jh;
+        }
+      }
+      const int len = max(0, jh - jl + 1), has = len > 0;
+      const int iseg = block_scan_incl(has, wsum);
+      const int ipts = block_scan_incl(len, wsum);
+      if (FILL && has) {
+        seg_pj[s0 + nseg + iseg - 1] = p | (jl << 11) | (shift << 27);
+        seg_off[s0 + nseg + iseg - 1] = npts + ipts - len;
+      }
+      if (tid == 255) {
+        carry[0] = iseg;
+        carry[1] = ipts;
+      }
+      __syncthreads();
+      nseg += carry[0];
+      npts += carry[1];
+      __syncthreads();
+    }
+  }
+  if (!FILL && tid == 0) {
+    counts[tile] = npts;
+    counts[gridDim.x + tile] = nseg;
+  }
+}
+
+// One workgroup per (work item, group of SB slices): the points [f0, f1) of
+// its tile as a matrix product on the matrix cores.  The tile is 16 regions
+// of 4 rows x 16 columns, four to a wave.  For a region, a slice pair and
+// four points, v_mfma_f32_16x16x4 multiplies
+//   A[4 r + e][k] = wy_k(row r) c_k(e)   (e: Re, Im of either slice)
+//   B[k][x]       = wx_k(column x)
+// so the region's cells are accumulated in FP32 registers: lane (r, x) holds
+// the four values of cell (r, x).  Points are prepared in batches of SP_BATCH
+// (one thread a point: footprint cell, 8 + 8 kernel weights and the slices'
+// values, to LDS); each wave then lists the points that meet a region, in
+// point order, and takes them four at a time.  Weights outside the footprint
+// are zero.  Every cell adds its points in list order: deterministic.
+//
+// The former kernel added points to LDS cells (read, add, write of 8 bytes per
+// cell, slice and point), about 615 SIMD cycles a point for four slices; here
+// a point costs 16.6 % of 16 regions x 32 cycles for two slices.
+// 8 x 2048^2 at 1501 angles (4374^2 grid): 2.81 -> 0.72 ms, now bound by
+// writing the grid.
+constexpr int SP_BATCH = 128;
+
+// Rows and columns of wave w's region g: each pair of 4-row bands has one
+// region of every wave, and so has each column half over two pairs.  A batch
+// is a few neighbouring rays, which may cross the tile along a few rows or
+// columns; with eight whole rows to a wave, such a batch left most waves idle.
+__device__ __forceinline__ int region_y(int w, int g) {
+  return 8 * g + 4 * (((w - g) & 3) >> 1);
+}
+__device__ __forceinline__ int region_x(int w, int g) {
+  return 16 * ((w - g) & 1);
+}
+using f32x4 = __attribute__((__vector_size__(4 * sizeof(float)))) float;
+
+template <int SB>
 __global__ void __launch_bounds__(256)
 spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
-  __shared__ float2 acc[SP_SB][SP_T * SP_RS];
-  __shared__ int4 pt_geo[SP_BATCH];      // l0x, l0y, bits(a0), bits(b0)
-  __shared__ float4 pt_val[SP_BATCH][2];  // slices (0, 1), (2, 3)
-  __shared__ int pt_band[SP_BATCH];
-  __shared__ short wlist[4][SP_BATCH];
-  __shared__ int wsum[4];
-  __shared__ int nseg;
-  extern __shared__ int seg_dyn[];  // seg_pj[P], seg_off[P + 1]
-  int* seg_pj = seg_dyn;
-  int* seg_off = seg_dyn + a.P;
+  constexpr int Q = SB / 2;  // slice pairs
+  // rows padded so that one thread a row writes 16 bytes without conflicts
+  constexpr int CS = Q == 1 ? 4 : 4 * Q + 4;
+  // x weights at 4 .. 11 and y weights at 16 .. 23, a zero on either side of
+  // each run: a cell outside the footprint reads one of those
+  __shared__ alignas(16) float pt_w[SP_BATCH][28];
+  // [Re, Im of even slices, Re, Im of odd slices][slice pair]
+  __shared__ alignas(16) float pt_c[SP_BATCH][CS];
+  __shared__ short2 pt_geo[SP_BATCH];  // (index | l0x << 8, l0y)
+  __shared__ int wlist[4][SP_BATCH + 12];
+  __shared__ int sg_off[SP_BATCH + 1], sg_pj[SP_BATCH];
+  __shared__ int sg_first;
   static_assert(SP_T == 32, "four 8-row bands per tile");
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int qa = lane >> 3, qb = lane & 7;
-  const int4 item = work[xcd_remap(blockIdx.x, gridDim.x)];
-  const int s0 = blockIdx.y * SP_SB;
-  const int ns = min(SP_SB, a.nsl - s0);
+  const int lm = lane & 15, lk = lane >> 4;
+  const int wi = xcd_remap(blockIdx.x, gridDim.x);
+  const int4 item = work[2 * wi];
+  const int4 segs = work[2 * wi + 1];  // the tile's segments [x, y)
+  const int s0 = blockIdx.y * SB;
+  const int ns = min(SB, a.nsl - s0);
   const TileWindow w = tile_window(a, item.x);
-  const int band0 = w.Y0 + 8 * wave;  // rows this wave owns
-  const int band1 = min(band0 + 8, w.Y1);
-  for (int i = tid; i < SP_SB * SP_T * SP_RS; i += 256)
-    (&acc[0][0])[i] = make_float2(0.f, 0.f);
-  const double hw = 0.5 * NUFFT_W;
   const long sstride = (long)a.P * a.N;
-  const float zscale = 2.0f / NUFFT_W;
-  int base = 0;
-  for (int ky = -1; ky <= 1; ++ky) {
-    for (int kx = -1; kx <= 1; ++kx) {
-      const double U0 = 0.5 * a.nf + kx * (double)a.nf;
-      const double V0 = 0.5 * a.nf + ky * (double)a.nf;
-      if (shift_skipped(a, w, U0, V0)) continue;
-      if (base >= item.z) continue;  // uniform: chunk already complete
-      int nsg;
-      const int total = enumerate_segments(a, U0, V0, w.lox, w.hix, w.loy,
-                                           w.hiy, seg_pj, seg_off, wsum,
-                                           &nseg, &nsg);
-      const int fa = max(item.y, base) - base;
-      const int fb = min(item.z, base + total) - base;
-      for (int fb0 = fa; fb0 < fb; fb0 += SP_BATCH) {
-        const int nb = min(SP_BATCH, fb - fb0);
-        // prepare: thread t -> point fb0 + t
-        if (tid < nb) {
-          const int f = fb0 + tid;
-          int lo = 0, hi = nsg;  // seg_off[lo] <= f < seg_off[hi]
-          while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (seg_off[mid] <= f) lo = mid;
-            else hi = mid;
-          }
-          const int pj = seg_pj[lo];
-          const int p = pj & 2047;
-          const int j = (pj >> 11) + (f - seg_off[lo]);
-          const double t = (double)(j - a.cidx);
-          const double u = U0 + t * a.ax[p];
-          const double v = V0 + t * a.ay[p];
-          const double cxu = ceil(u - hw), cyv = ceil(v - hw);
-          const int l0x = (int)cxu, l0y = (int)cyv;
-          pt_geo[tid] = make_int4(l0x, l0y,
-                                  __builtin_bit_cast(int, (float)(cxu - u)),
-                                  __builtin_bit_cast(int, (float)(cyv - v)));
-          const float2* cp = a.c + (long)s0 * sstride + (long)p * a.N + j;
-          float2 cv[SP_SB];
+  const int seg1 = segs.y;
+  f32x4 acc[4][Q];
 #pragma unroll
-          for (int q = 0; q < SP_SB; ++q)
-            cv[q] = q < ns ? cp[(long)q * sstride] : make_float2(0.f, 0.f);
-          pt_val[tid][0] = make_float4(cv[0].x, cv[0].y, cv[1].x, cv[1].y);
-          pt_val[tid][1] = make_float4(cv[2].x, cv[2].y, cv[3].x, cv[3].y);
-          int bands = 0;
-          if (l0x < w.X1 && l0x + NUFFT_W > w.X0) {
+  for (int g = 0; g < 4; ++g)
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-              const int r0 = w.Y0 + 8 * b, r1 = min(r0 + 8, w.Y1);
-              if (l0y < r1 && l0y + NUFFT_W > r0) bands |= 1 << b;
-            }
-          }
-          pt_band[tid] = bands;
-        }
-        __syncthreads();
-        // this wave's list of points meeting its band, kept in registers
-        int cnt = 0;
-        int lst[SP_BATCH / 64];
-#pragma unroll
-        for (int c = 0; c < SP_BATCH / 64; ++c) {
-          const int idx = c * 64 + lane;
-          const bool hit = idx < nb && ((pt_band[idx] >> wave) & 1);
-          const unsigned long long bal = __ballot(hit);
-          const int pos =
-              cnt + __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
-                                              __builtin_amdgcn_mbcnt_lo(
-                                                  (unsigned)bal, 0u));
-          if (hit) wlist[wave][pos] = (short)idx;
-          cnt += __popcll(bal);
-        }
-#pragma unroll
-        for (int c = 0; c < SP_BATCH / 64; ++c) lst[c] = wlist[wave][c * 64 + lane];
-        // software-pipelined: point k + 1's data is read from LDS while
-        // point k's cells are updated
-        auto entry = [&](int k) {
-          return k < 64 ? __builtin_amdgcn_readlane(lst[0], k)
-                        : __builtin_amdgcn_readlane(lst[1], k - 64);
-        };
-        static_assert(SP_BATCH == 128, "two list registers");
-        int4 g = make_int4(0, 0, 0, 0);
-        float4 v01 = make_float4(0.f, 0.f, 0.f, 0.f), v23 = v01;
-        if (cnt > 0) {
-          const int i = entry(0);
-          g = pt_geo[i];
-          v01 = pt_val[i][0];
-          v23 = pt_val[i][1];
-        }
-        for (int k = 0; k < cnt; ++k) {
-          const int in = entry(min(k + 1, cnt - 1));
-          const int4 gn = pt_geo[in];
-          const float4 v01n = pt_val[in][0];
-          const float4 v23n = pt_val[in][1];
-          const int cx = g.x + qb;
-          const int cy = g.y + qa;
-          // the point's 8 x weights (lanes 0-7) and 8 y weights (lanes
-          // 8-15), one kernel evaluation per lane, fetched by lane (qa, qb)
-          // from lanes qb and 8 + qa; every lane takes part, so this stays
-          // outside the bounds test
-          const int m = lane & 7;
-          const float dl = __builtin_bit_cast(float, lane < 8 ? g.z : g.w) +
-                           (float)m;
-          const float wl = es_kernel(dl * zscale, a.beta);
-          const float wx = __builtin_bit_cast(
-              float, __builtin_amdgcn_ds_bpermute(
-                         qb << 2, __builtin_bit_cast(int, wl)));
-          const float wy = __builtin_bit_cast(
-              float, __builtin_amdgcn_ds_bpermute(
-                         (8 + qa) << 2, __builtin_bit_cast(int, wl)));
-          if (cy >= band0 && cy < band1 && cx >= w.X0 && cx < w.X1) {
-            const float wgt = wx * wy;
-            const int cell = (cy - w.Y0) * SP_RS + (cx - w.X0);
-            float2 a0 = acc[0][cell], a1 = acc[1][cell];
-            float2 a2 = acc[2][cell], a3 = acc[3][cell];
-            a0.x = fmaf(v01.x, wgt, a0.x);
-            a0.y = fmaf(v01.y, wgt, a0.y);
-            a1.x = fmaf(v01.z, wgt, a1.x);
-            a1.y = fmaf(v01.w, wgt, a1.y);
-            a2.x = fmaf(v23.x, wgt, a2.x);
-            a2.y = fmaf(v23.y, wgt, a2.y);
-            a3.x = fmaf(v23.z, wgt, a3.x);
-            a3.y = fmaf(v23.w, wgt, a3.y);
-            acc[0][cell] = a0;
-            acc[1][cell] = a1;
-            acc[2][cell] = a2;
-            acc[3][cell] = a3;
-          }
-          g = gn;
-          v01 = v01n;
-          v23 = v23n;
-        }
-        __syncthreads();  // the batch buffers are rewritten next
-      }
-      base += total;
-    }
+    for (int q = 0; q < Q; ++q) acc[g][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (tid < SP_BATCH) {
+    pt_w[tid][3] = pt_w[tid][12] = 0.f;
+    pt_w[tid][15] = pt_w[tid][24] = 0.f;
   }
-  __syncthreads();
+  int seg = segs.x;
+  if (item.y > 0) {
+    // the segment that holds point f0 (offsets ascend from 0 at segs.x)
+    for (int i = seg + tid; i < seg1; i += 256) {
+      const int nxt = i + 1 < seg1 ? a.seg_off[i + 1] : 0x7fffffff;
+      if (a.seg_off[i] <= item.y && item.y < nxt) sg_first = i;
+    }
+    __syncthreads();
+    seg = sg_first;
+  }
+  // half 0 prepares x (and even slices) of point `pt`, half 1 y (odd slices)
+  const int pt = tid & (SP_BATCH - 1);
+  const int half = __builtin_amdgcn_readfirstlane(tid / SP_BATCH);
+  for (int fb0 = item.y; fb0 < item.z; fb0 += SP_BATCH) {
+    const int nb = min(SP_BATCH, item.z - fb0);
+    // the batch's segments: every segment has a point, so at most nb of them
+    if (tid <= SP_BATCH) {
+      const int i = seg + tid;
+      sg_off[tid] = i < seg1 ? a.seg_off[i] : 0x7fffffff;
+      if (tid < SP_BATCH) sg_pj[tid] = i < seg1 ? a.seg_pj[i] : 0;
+    }
+    __syncthreads();
+    auto segment_of = [&](int f, int n) {  // sg_off[lo] <= f < sg_off[lo + 1]
+      int lo = 0, hi = n;
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (sg_off[mid] <= f) lo = mid;
+        else hi = mid;
+      }
+      return lo;
+    };
+    if (pt < nb) {
+      const int f = fb0 + pt;
+      const int lo = segment_of(f, SP_BATCH);
+      const int pj = sg_pj[lo];
+      const int p = pj & 2047;
+      const int j = ((pj >> 11) & 0xffff) + (f - sg_off[lo]);
+      const float2* cp =
+          a.c + (long)(s0 + half) * sstride + (long)p * a.N + j;
+      float2 cv[Q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        cv[q] = 2 * q + half < ns ? cp[2 * q * sstride] : make_float2(0.f, 0.f);
+      const double2 o = shift_origin(a, pj >> 27);
+      float frac;
+      const int l0 = first_cell(half ? o.y : o.x, (double)(j - a.cidx),
+                                half ? a.ay[p] : a.ax[p], frac) -
+                     (half ? w.Y0 : w.X0);  // -7 .. 31
+      if (half)
+        pt_geo[pt].y = (short)l0;
+      else
+        pt_geo[pt].x = (short)(pt | (l0 << 8));
+      float wt[NUFFT_W];
+#pragma unroll
+      for (int m = 0; m < NUFFT_W; ++m)
+        wt[m] = es_kernel((frac + (float)m) * (2.0f / NUFFT_W), a.beta);
+#pragma unroll
+      for (int m = 0; m < NUFFT_W; ++m) pt_w[pt][12 * half + 4 + m] = wt[m];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        pt_c[pt][(2 * half) * Q + q] = cv[q].x;
+        pt_c[pt][(2 * half + 1) * Q + q] = cv[q].y;
+      }
+      // the segment of the next batch's first point
+      if (tid == nb - 1) sg_first = seg + segment_of(fb0 + nb, SP_BATCH + 1);
+    } else if (half == 0) {
+      pt_geo[pt] = make_short2((short)(pt | (100 << 8)), 100);  // no region
+    }
+    __syncthreads();
+    seg = sg_first;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int ry = region_y(wave, g), rx = region_x(wave, g);
+      // points whose footprints meet the region, in point order: index and
+      // footprint origin in the region, plus 8
+      int cnt = 0;
+#pragma unroll
+      for (int c = 0; c < SP_BATCH / 64; ++c) {
+        const short2 e = pt_geo[c * 64 + lane];
+        const int dx = (e.x >> 8) - rx, dy = e.y - ry;
+        const bool hit = dx > -NUFFT_W && dx < 16 && dy > -NUFFT_W && dy < 4;
+        const unsigned long long bal = __ballot(hit);
+        const int pos =
+            cnt + __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
+                                            __builtin_amdgcn_mbcnt_lo(
+                                                (unsigned)bal, 0u));
+        if (hit)
+          wlist[wave][pos] = (e.x & 0xff) | (dx + 8) << 8 | (dy + 8) << 16;
+        cnt += __popcll(bal);
+      }
+      if (cnt == 0) continue;
+      // the steps and look-ahead past the end take a point of the batch with
+      // its footprint out of reach
+      if (lane < 12) wlist[wave][cnt + lane] = 0xffff00;
+      __builtin_amdgcn_wave_barrier();
+      // Steps of four points; the next step's weights and values and the list
+      // entries of the one after it are read from LDS while this one's
+      // products run.
+      struct Step {
+        float wx, wy, c[Q];
+      };
+      auto fetch = [&](int e) {
+        Step t;
+        const int i = e & 0xff;
+        const int dx = min(max(lm + 8 - ((e >> 8) & 0xff), -1), 8);
+        const int dy = min(max((lm >> 2) + 8 - ((e >> 16) & 0xff), -1), 8);
+        t.wx = pt_w[i][4 + dx];
+        t.wy = pt_w[i][16 + dy];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) t.c[q] = pt_c[i][(lm & 3) * Q + q];
+        return t;
+      };
+      Step cur = fetch(wlist[wave][lk]);
+      int e1 = wlist[wave][4 + lk];
+      for (int k0 = 0; k0 < cnt; k0 += 4) {
+        const Step nxt = fetch(e1);
+        e1 = wlist[wave][k0 + 8 + lk];
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+          acc[g][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              cur.wy * cur.c[q], cur.wx, acc[g][q], 0, 0, 0);
+        cur = nxt;
+      }
+    }
+    __syncthreads();  // the batch buffers are rewritten next
+  }
   float2* dst = item.w < 0 ? nullptr
                            : scratch + ((long)item.w * gridDim.y + blockIdx.y) *
-                                           (SP_SB * SP_T * SP_T);
-  for (int i = tid; i < ns * SP_T * SP_T; i += 256) {
-    const int s = i / (SP_T * SP_T);
-    const int c = i - s * SP_T * SP_T;
-    const int ly = c / SP_T, lx = c - ly * SP_T;
-    const float2 val = acc[s][ly * SP_RS + lx];
-    if (dst) {
-      dst[i] = val;
-    } else if (w.Y0 + ly < w.Y1 && w.X0 + lx < w.X1) {
-      a.fine[((long)(s0 + s) * a.nf + w.Y0 + ly) * a.nf + w.X0 + lx] = val;
+                                           (SB * SP_T * SP_T);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int ly = region_y(wave, g) + lk, lx = region_x(wave, g) + lm;
+    const bool in = w.Y0 + ly < w.Y1 && w.X0 + lx < w.X1;
+#pragma unroll
+    for (int s = 0; s < SB; ++s) {
+      const float2 val = make_float2(acc[g][s >> 1][2 * (s & 1)],
+                                     acc[g][s >> 1][2 * (s & 1) + 1]);
+      if (dst) {
+        dst[(s * SP_T + ly) * SP_T + lx] = val;
+      } else if (in && s < ns) {
+        a.fine[((long)(s0 + s) * a.nf + w.Y0 + ly) * a.nf + w.X0 + lx] = val;
+      }
     }
   }
 }
 
 // Adds the scratch slots of multi-chunk tiles into the fine grid, in slot
-// order (deterministic).
+// order (deterministic).  sb: slices per group of the spreading launch.
 __global__ void __launch_bounds__(256)
 spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix,
-                    const float2* __restrict__ scratch) {
+                    const float2* __restrict__ scratch, int sb) {
   const int4 f = fix[blockIdx.x];
-  const int s0 = blockIdx.y * SP_SB;
-  const int ns = min(SP_SB, a.nsl - s0);
+  const int s0 = blockIdx.y * sb;
+  const int ns = min(sb, a.nsl - s0);
   const int ty = f.x / a.ntx, tx = f.x - (f.x / a.ntx) * a.ntx;
   const int X0 = tx * SP_T, Y0 = ty * SP_T;
   const int X1 = min(X0 + SP_T, a.nf), Y1 = min(Y0 + SP_T, a.nf);
-  // blockIdx.z picks a quarter of the SP_SB x SP_T x SP_T elements, so a
-  // tile's slots are summed by four workgroups; each thread sums its four
-  // elements over the slots four slots at a time (16 loads in flight);
-  // the per-element order is slot order
-  constexpr int PART = SP_SB * SP_T * SP_T / 4;
-  constexpr int PER = PART / 256;
-  const int nel = ns * SP_T * SP_T;
-  const int e0 = blockIdx.z * PART + threadIdx.x;
-  const long slot_stride = (long)gridDim.y * (SP_SB * SP_T * SP_T);
+  // blockIdx.z picks a slice of the group, so a tile's slots are summed by sb
+  // workgroups; each thread sums its four elements over the slots four slots
+  // at a time (16 loads in flight); the per-element order is slot order
+  const int s = blockIdx.z;
+  if (s >= ns) return;
+  constexpr int PER = SP_T * SP_T / 256;
+  const long slot_stride = (long)gridDim.y * sb * (SP_T * SP_T);
   const float2* base = scratch + (long)f.y * slot_stride +
-                       (long)blockIdx.y * (SP_SB * SP_T * SP_T);
+                       ((long)blockIdx.y * sb + s) * (SP_T * SP_T) +
+                       threadIdx.x;
   float2 sum[PER];
 #pragma unroll
   for (int e = 0; e < PER; ++e) sum[e] = make_float2(0.f, 0.f);
@@ -478,11 +487,8 @@ spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix,
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int e = 0; e < PER; ++e) {
-        const int i = e0 + 256 * e;
-        q[u][e] = i < nel ? base[(long)(k + u) * slot_stride + i]
-                          : make_float2(0.f, 0.f);
-      }
+      for (int e = 0; e < PER; ++e)
+        q[u][e] = base[(long)(k + u) * slot_stride + 256 * e];
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -494,21 +500,16 @@ spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix,
   for (; k < f.z; ++k) {
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
-      const int i = e0 + 256 * e;
-      if (i < nel) {
-        const float2 q = base[(long)k * slot_stride + i];
-        sum[e].x += q.x;
-        sum[e].y += q.y;
-      }
+      const float2 q = base[(long)k * slot_stride + 256 * e];
+      sum[e].x += q.x;
+      sum[e].y += q.y;
     }
   }
 #pragma unroll
   for (int e = 0; e < PER; ++e) {
-    const int i = e0 + 256 * e;
-    const int s = i / (SP_T * SP_T);
-    const int cell = i - s * SP_T * SP_T;
+    const int cell = threadIdx.x + 256 * e;
     const int ly = cell / SP_T, lx = cell - ly * SP_T;
-    if (i < nel && Y0 + ly < Y1 && X0 + lx < X1) {
+    if (Y0 + ly < Y1 && X0 + lx < X1) {
       float2* o = a.fine + ((long)(s0 + s) * a.nf + Y0 + ly) * a.nf + X0 + lx;
       const float2 cur = *o;
       *o = make_float2(cur.x + sum[e].x, cur.y + sum[e].y);
@@ -723,28 +724,52 @@ float2* PolarNufft::fine(int batch) {
   return fine_.as<float2>();
 }
 
-// Points per tile of this geometry (a device count, read back once).
-void PolarNufft::count_tiles(hipStream_t stream) {
-  const int ntx = (int)cdiv(nf_, SP_T);
-  const int ntiles = ntx * ntx;
-  const int cidx = N_ / 2;
+SpreadArgs PolarNufft::spread_args() const {
   SpreadArgs a{};
   a.ax = ax_.as<double>();
   a.ay = ay_.as<double>();
+  a.seg_pj = seg_pj_.as<int>();
+  a.seg_off = seg_off_.as<int>();
+  a.tile_seg = tile_seg_.as<int>();
   a.P = P_;
   a.N = N_;
-  a.cidx = cidx;
+  a.cidx = N_ / 2;
   a.nf = nf_;
-  a.ntx = ntx;
-  a.umax = std::max(cidx, N_ - 1 - cidx) * ((double)nf_ / (N_ - 1)) + 1.0;
-  DevBuf dcounts(sizeof(int) * ntiles);
-  hipLaunchKernelGGL(spread_count_kernel, dim3(ntiles), dim3(256), 0, stream,
-                     a, dcounts.as<int>());
+  a.ntx = (int)cdiv(nf_, SP_T);
+  a.umax = std::max(a.cidx, N_ - 1 - a.cidx) * ((double)nf_ / (N_ - 1)) + 1.0;
+  a.beta = beta_;
+  return a;
+}
+
+// The ray segments of every tile of this geometry: counted on the device,
+// read back once (the work list needs the points per tile), then written.
+void PolarNufft::make_segments(hipStream_t stream) {
+  ArenaPause no_arena;  // the plan's lists, offsets filled synchronously
+  const int ntx = (int)cdiv(nf_, SP_T);
+  const int ntiles = ntx * ntx;
+  SpreadArgs a = spread_args();
+  DevBuf dcounts(sizeof(int) * 2 * ntiles);
+  hipLaunchKernelGGL(spread_segments_kernel<false>, dim3(ntiles), dim3(256), 0,
+                     stream, a, dcounts.as<int>(), nullptr, nullptr);
   TC_HIP(hipGetLastError());
-  counts_.assign(ntiles, 0);
-  TC_HIP(hipMemcpyAsync(counts_.data(), dcounts.as<void>(),
-                        sizeof(int) * ntiles, hipMemcpyDeviceToHost, stream));
+  std::vector<int> h(2 * (size_t)ntiles);
+  TC_HIP(hipMemcpyAsync(h.data(), dcounts.as<void>(), sizeof(int) * h.size(),
+                        hipMemcpyDeviceToHost, stream));
   TC_HIP(hipStreamSynchronize(stream));
+  counts_.assign(h.begin(), h.begin() + ntiles);
+  std::vector<int>& first = tile_first_;
+  first.assign(ntiles + 1, 0);
+  for (int t = 0; t < ntiles; ++t) first[t + 1] = first[t] + h[ntiles + t];
+  tile_seg_.alloc(sizeof(int) * first.size());
+  TC_HIP(hipMemcpy(tile_seg_.as<void>(), first.data(),
+                   sizeof(int) * first.size(), hipMemcpyHostToDevice));
+  const size_t nseg = std::max(1, first[ntiles]);
+  seg_pj_.alloc(sizeof(int) * nseg);
+  seg_off_.alloc(sizeof(int) * nseg);
+  a = spread_args();
+  hipLaunchKernelGGL(spread_segments_kernel<true>, dim3(ntiles), dim3(256), 0,
+                     stream, a, nullptr, seg_pj_.as<int>(), seg_off_.as<int>());
+  TC_HIP(hipGetLastError());
 }
 
 // The work and fix-up lists for `chunk` points per item, uploaded to the
@@ -785,12 +810,19 @@ void PolarNufft::make_work(int chunk) {
       work[x * q + (x < rmd ? x : rmd) + t] = byw[b];
     }
   }
+  // each item with its tile's range of segments
+  std::vector<int4> items;
+  items.reserve(2 * work.size());
+  for (const int4& x : work) {
+    items.push_back(x);
+    items.push_back(make_int4(tile_first_[x.x], tile_first_[x.x + 1], 0, 0));
+  }
   nwork_ = (int)work.size();
   nslots_ = slot;
   nfix_ = (int)fix.size();
   chunk_ = chunk;
-  work_.alloc(sizeof(int4) * nwork_);
-  TC_HIP(hipMemcpy(work_.as<void>(), work.data(), sizeof(int4) * nwork_,
+  work_.alloc(sizeof(int4) * items.size());
+  TC_HIP(hipMemcpy(work_.as<void>(), items.data(), sizeof(int4) * items.size(),
                    hipMemcpyHostToDevice));
   if (nfix_) {
     fix_.alloc(sizeof(int4) * nfix_);
@@ -813,10 +845,11 @@ static std::tuple<int, int, int, int, int> chunk_key(int P, int N, int nf,
 }
 
 // Slices per fine-grid batch: about 1 GB of fine grid, in whole groups of
-// SP_SB slices (a spreading workgroup accumulates SP_SB slices; a partial
-// group idles part of its accumulator and repeats the tile's segment
-// enumeration and point set-up for fewer slices), rounding up while that
-// stays within 1.25 GB.
+// SP_SB slices (a spreading workgroup accumulates up to SP_SB slices; a
+// partial group idles part of its matrix products and repeats the tile's
+// point set-up for fewer slices), rounding up while that stays within
+// 1.25 GB.
+constexpr int SP_SB = 8;
 static int fine_batch(int nf, int S) {
   const double per = 8.0 * nf * (double)nf, budget = 1.0e9;
   const int b0 = (int)std::max(1.0, std::floor(budget / per));
@@ -834,46 +867,38 @@ void PolarNufft::type1_real(const float2* c, float* out, int S, float scale,
   TC_REQUIRE(S >= 1, "NUFFT: need at least one slice");
   const int B = fine_batch(nf_, S);
   float2* fg = fine(B);
-  const int ntx = (int)cdiv(nf_, SP_T);
-  const unsigned ngroups_max = cdiv(B, SP_SB);
-  const int cidx = N_ / 2;
-  const double umax =
-      std::max(cidx, N_ - 1 - cidx) * ((double)nf_ / (N_ - 1)) + 1.0;
+  // slices a spreading workgroup takes: a point's weights and footprint serve
+  // all of them, so as many as there are, up to 8 (64 accumulators a lane)
+  auto group = [](int nb) { return nb <= 2 ? 2 : nb <= 4 ? 4 : SP_SB; };
   auto args = [&](int s0, int nb) {
-    SpreadArgs a;
+    SpreadArgs a = spread_args();
     a.c = c + (long)s0 * P_ * N_;
     a.fine = fg;
-    a.ax = ax_.as<double>();
-    a.ay = ay_.as<double>();
-    a.P = P_;
-    a.N = N_;
-    a.cidx = cidx;
-    a.nf = nf_;
     a.nsl = nb;
-    a.ntx = ntx;
-    a.umax = umax;
-    a.beta = beta_;
     return a;
   };
-  const size_t seg_lds = sizeof(int) * (2 * (size_t)P_ + 1);
   // the fine grid of nb slices from the current work lists
   auto spread = [&](const SpreadArgs& a, int nb, float2* scratch) {
-    const unsigned ng = cdiv(nb, SP_SB);
-    hipLaunchKernelGGL(spread_kernel, dim3((unsigned)nwork_, ng), dim3(256),
-                       seg_lds, stream, a, work_.as<int4>(), scratch);
+    const int sb = group(nb);
+    const unsigned ng = cdiv(nb, sb);
+    auto k = sb == 2 ? spread_kernel<2> : sb == 4 ? spread_kernel<4>
+                                                  : spread_kernel<SP_SB>;
+    hipLaunchKernelGGL(k, dim3((unsigned)nwork_, ng), dim3(256), 0, stream, a,
+                       work_.as<int4>(), scratch);
     TC_HIP(hipGetLastError());
     if (nfix_) {
-      hipLaunchKernelGGL(spread_fixup_kernel, dim3((unsigned)nfix_, ng, 4),
-                         dim3(256), 0, stream, a, fix_.as<int4>(), scratch);
+      hipLaunchKernelGGL(spread_fixup_kernel, dim3((unsigned)nfix_, ng, sb),
+                         dim3(256), 0, stream, a, fix_.as<int4>(), scratch, sb);
       TC_HIP(hipGetLastError());
     }
   };
-  auto scratch_bytes = [&](unsigned ngroups) {
-    return sizeof(float2) * (size_t)std::max(nslots_, 1) * ngroups * SP_SB *
+  auto scratch_bytes = [&](int nb) {
+    const int sb = group(nb);
+    return sizeof(float2) * (size_t)std::max(nslots_, 1) * cdiv(nb, sb) * sb *
            SP_T * SP_T;
   };
   if (!work_ready_) {
-    count_tiles(stream);
+    make_segments(stream);
     const int ntiles = (int)counts_.size();
     // Points per work item: TOMOCAM_HIP_SPREAD_CHUNK (>= 64), else the
     // autotuner's choice for this geometry, else (tuning allowed) the
@@ -906,7 +931,7 @@ void PolarNufft::type1_real(const float2* c, float* out, int S, float scale,
       try {
         for (int k : cands) {
           make_work(k);
-          DevBuf scr(scratch_bytes(cdiv(nb, SP_SB)));
+          DevBuf scr(scratch_bytes(nb));
           float ms = 0.f;
           for (int rep = 0; rep < 3; ++rep) {
             TC_HIP(hipEventRecord(e0, stream));
@@ -941,7 +966,7 @@ void PolarNufft::type1_real(const float2* c, float* out, int S, float scale,
     if (chunk != chunk_) make_work(chunk);
     work_ready_ = true;
   }
-  DevBuf scratch(scratch_bytes(ngroups_max));
+  DevBuf scratch(scratch_bytes(B));
   for (int s0 = 0; s0 < S; s0 += B) {
     const int nb = std::min(B, S - s0);
     const SpreadArgs a = args(s0, nb);
