@@ -82,7 +82,7 @@ int tc_gradient(const float* d_x, const float* d_sinoT, float* d_g,
     hipStream_t s = as_stream(stream);
     tc::ArenaScope arena(s);
     tc::PolarNufft& nu = tc::nufft_plan(h_angles, nproj, npix, npix);
-    tc::DevBuf c(sizeof(float2) * (size_t)nslices * nproj * npix);
+    tc::DevBuf c(sizeof(float2) * (size_t)nslices * nproj * nu.nh());
     nu.type2_real(d_x, c.as<float2>(), nslices, s);
     const double n3 = (double)npix * npix * npix;
     nu.type1_real(c.as<float2>(), d_g, nslices, (float)(1.0 / n3), s);

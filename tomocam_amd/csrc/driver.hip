@@ -321,7 +321,7 @@ Mbir2Result mbir_nufft(const float* sino, const float* x0, float* recon, int S,
 
   PolarNufft& nu = nufft_plan(h_angles, P, n2, n2);
   const float inv_n3 = (float)(1.0 / ((double)n2 * n2 * n2));
-  DevBuf bcoef(sizeof(float2) * (size_t)ns2);
+  DevBuf bcoef(sizeof(float2) * (size_t)S * P * nu.nh());
   DevBuf bproj(sizeof(float) * ns2);
   // Re(A^H A v)/n^3 - b (+ R'(v))  (src/gradient.cpp:35-103)
   auto gradient = [&](const float* v, float* g, int nsl, const float* b) {

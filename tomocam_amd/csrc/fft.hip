@@ -1,12 +1,14 @@
 // Host plans and the generic batched line FFT kernel.
 #include <cmath>
 #include <cstdlib>
+#include <functional>
 #include <map>
 #include <memory>
 #include <mutex>
 
-#include "fft_device.h"
+#include "fft_ct.h"
 #include "fft_ops.h"
+#include "lds_launch.h"
 
 namespace tc {
 
@@ -52,9 +54,39 @@ int fft_next_smooth(int n, bool even) {
   }
 }
 
+constexpr int RT_MAX_STAGES = 8;
+
+// The radices of L: as few stages as possible, and of those the largest
+// smallest radix (so that the stages have alike numbers of butterflies).
+static std::vector<int> rt_factor(int L) {
+  static const int kRadices[] = {16, 15, 14, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
+  std::vector<int> best, cur;
+  std::function<void(int, int)> go = [&](int m, int from) {
+    if (!best.empty() && cur.size() >= best.size() && m > 1) return;
+    if (m == 1) {
+      if (best.empty() || cur.size() < best.size() ||
+          (cur.size() == best.size() && cur.back() > best.back()))
+        best = cur;
+      return;
+    }
+    for (int i = from; i < 13; ++i)
+      if (m % kRadices[i] == 0) {
+        cur.push_back(kRadices[i]);
+        go(m / kRadices[i], i);
+        cur.pop_back();
+      }
+  };
+  go(L, 0);
+  TC_REQUIRE(L == 1 || !best.empty(), "FFT length " + std::to_string(L) +
+                                          " is not a product of 2, 3, 5, 7");
+  TC_REQUIRE((int)best.size() <= RT_MAX_STAGES, "FFT length too large");
+  return best;
+}
+
 FFTLength::FFTLength(int L) {
   ArenaPause no_arena;  // process-lifetime table, filled synchronously
   std::vector<int> r = fft_factor(L);
+  radices_ = rt_factor(L);
   plan_.L = L;
   plan_.nst = (int)r.size();
   for (int i = 0; i < plan_.nst; ++i) plan_.radix[i] = r[i];
@@ -99,126 +131,577 @@ const FFTLength& fft_length(int L) {
 }
 
 // ---------------------------------------------------------------------------
-// generic batched line FFT: line l of batch b starts at b*bstride + l*lstride,
-// element i at + i*estride (complex elements).  `nin` leading elements are
-// read (the rest are zero); the first `nout` elements are written.
+// Runtime plans: any 2,3,5,7-smooth length as two to six radices of up to 16,
+// lines in LDS, each stage from one buffer to the other (one barrier a stage).
+// The former form took radices 8, 4, 2, 3, 5, 7 in place: four to six stages
+// of two barriers each (3 x 672 lines of 672 points: 25 -> 17 us for the 337
+// columns of the half grid, 12 us for the packed rows).
+// Lines too long for two buffers (more than about 9900 points) run in place.
 // ---------------------------------------------------------------------------
 
+constexpr int RT_MAX_THREADS = 512;
+
+struct RtPlan {
+  int L, nst, ldl;  // ldl: LDS elements per line and buffer
+  int lines_off;    // elements from one buffer to the other
+  int radix[RT_MAX_STAGES];
+  const float2* tw;  // exp(-2 pi i m / L)
+};
+
+// one unused slot per 32: the first stages' strided stores spread over banks
+__host__ __device__ __forceinline__ int rt_pad(int i) { return i + (i >> 5); }
+
+template <int R, int DIR>
+__device__ __forceinline__ void rt_stage(const float2* in, float2* out,
+                                         int nlines, const RtPlan& P, int Ns,
+                                         int tid, int nthr) {
+  const int nb = P.L / R, step = P.L / (Ns * R);
+  for (int t = tid; t < nlines * nb; t += nthr) {
+    const int line = nlines == 1 ? 0 : t / nb;
+    const int j = t - line * nb;
+    const int k = Ns == 1 ? 0 : j % Ns;
+    const float2* src = in + line * P.ldl;
+    float2 v[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = src[rt_pad(j + r * nb)];
+    if (Ns > 1) {
+#pragma unroll
+      for (int r = 1; r < R; ++r) {
+        const float2 w = P.tw[k * r * step];
+        v[r] = DIR < 0 ? cmul(v[r], w) : cmulc(v[r], w);
+      }
+    }
+    ct::DftC<R, DIR>::run(v);
+    float2* dst = out + line * P.ldl;
+    const int d = (j - k) * R + k;
+#pragma unroll
+    for (int r = 0; r < R; ++r) dst[rt_pad(d + r * Ns)] = v[r];
+  }
+}
+
+// Transforms the lines in the first buffer of `sm` (the second if `second`)
+// and returns the buffer that holds the result.  Called by every thread, with
+// the data behind a barrier; returns behind one.
+template <int DIR>
+__device__ __forceinline__ float2* rt_fft(float2* sm, int nlines,
+                                          const RtPlan& P, int tid, int nthr,
+                                          bool second = false) {
+  float2* a = second ? sm + P.lines_off : sm;
+  float2* b = second ? sm : sm + P.lines_off;
+  int Ns = 1;
+  for (int s = 0; s < P.nst; ++s) {
+    const int R = P.radix[s];
+    switch (R) {
+#define TC_RT(RR)                                         \
+  case RR:                                                \
+    rt_stage<RR, DIR>(a, b, nlines, P, Ns, tid, nthr);    \
+    break;
+      TC_RT(2) TC_RT(3) TC_RT(4) TC_RT(5) TC_RT(6) TC_RT(7) TC_RT(8) TC_RT(9)
+      TC_RT(10) TC_RT(12) TC_RT(14) TC_RT(15) TC_RT(16)
+#undef TC_RT
+    }
+    __syncthreads();
+    Ns *= R;
+    float2* t = a;
+    a = b;
+    b = t;
+  }
+  return a;
+}
+
+struct RtLaunch {
+  RtPlan plan;
+  int lpw, nthr;
+  size_t smem;
+};
+
+// bytes of LDS of lpw lines in two buffers
+static size_t rt_bytes(int L, int lpw) {
+  return 2 * sizeof(float2) * (size_t)lpw * (rt_pad(L) + 1);
+}
+static bool rt_fits(int L) { return rt_bytes(L, 1) <= 160 * 1024; }
+
+// At most `want` lines per workgroup, 64 KB of LDS or one line, and a thread
+// per butterfly of the smallest radix up to 512.
+static RtLaunch rt_launch(int L, long nlines, int want) {
+  TC_REQUIRE(rt_fits(L), "FFT line does not fit in LDS");
+  const FFTLength& F = fft_length(L);
+  RtLaunch l;
+  l.plan.L = L;
+  l.plan.tw = F.plan().tw;
+  l.plan.nst = (int)F.radices().size();
+  for (int i = 0; i < l.plan.nst; ++i) l.plan.radix[i] = F.radices()[i];
+  l.plan.ldl = rt_pad(L) + 1;
+  l.lpw = 1;
+  while (2 * l.lpw <= want && rt_bytes(L, 2 * l.lpw) <= 64 * 1024 &&
+         nlines > l.lpw)
+    l.lpw *= 2;
+  l.plan.lines_off = l.lpw * l.plan.ldl;
+  const int rmin = l.plan.nst ? F.radices().back() : 1;
+  const long nb = (long)l.lpw * L / rmin;
+  l.nthr = (int)std::min<long>(RT_MAX_THREADS, (nb + 63) / 64 * 64);
+  l.smem = rt_bytes(L, l.lpw);
+  return l;
+}
+
+// Line l of batch b starts at b*bstride + l*lstride, element i at + i*estride
+// (complex elements).  Of a line, the elements [0, nin) and [L - nin_hi, L)
+// are read (the others are zero) and [0, nout) and [L - nout_hi, L) written.
+struct LinesMap {
+  int lines_per_batch, nin, nin_hi, nout, nout_hi, colmajor;
+  long total, bstride, lstride, estride;
+  float scale;
+};
+
+__device__ __forceinline__ long line_base(const LinesMap& m, long gl) {
+  const long b = gl / m.lines_per_batch;
+  return b * m.bstride + (gl - b * m.lines_per_batch) * m.lstride;
+}
+
+template <int DIR>
+__global__ void __launch_bounds__(RT_MAX_THREADS)
+rt_lines_kernel(const float2* __restrict__ in, float2* __restrict__ out,
+                RtPlan P, LinesMap m, int lpw) {
+  extern __shared__ float2 sm[];
+  const int tid = threadIdx.x, nthr = blockDim.x, L = P.L;
+  const long l0 = (long)blockIdx.x * lpw;
+  const int nl = (int)min((long)lpw, m.total - l0);
+  for (int t = tid; t < lpw * L; t += nthr) {
+    const int l = m.colmajor ? t % lpw : t / L;
+    const int i = m.colmajor ? t / lpw : t - l * L;
+    float2 v = make_float2(0.f, 0.f);
+    if (l < nl && (i < m.nin || i >= L - m.nin_hi))
+      v = in[line_base(m, l0 + l) + (long)i * m.estride];
+    sm[l * P.ldl + rt_pad(i)] = v;
+  }
+  __syncthreads();
+  const float2* z = rt_fft<DIR>(sm, lpw, P, tid, nthr);
+  const int nw = m.nout + m.nout_hi;  // elements written per line
+  for (int t = tid; t < lpw * nw; t += nthr) {
+    const int l = m.colmajor ? t % lpw : t / nw;
+    int i = m.colmajor ? t / lpw : t - l * nw;
+    if (i >= m.nout) i += L - nw;
+    if (l < nl)
+      out[line_base(m, l0 + l) + (long)i * m.estride] =
+          cscale(z[l * P.ldl + rt_pad(i)], m.scale);
+  }
+}
+
+// lines of more than rt_fits() points: one line per workgroup, in place
 template <int DIR, int NB>
 __global__ void __launch_bounds__(1024)
 fft_lines_kernel(const float2* __restrict__ in, float2* __restrict__ out,
-                 FFTPlan P, int lines_per_batch, int nbatch, long bstride,
-                 long lstride, long estride, int nin, int nout, int lpw,
-                 int ldl, int colmajor, float scale) {
+                 FFTPlan P, LinesMap m) {
   extern __shared__ float2 sm[];
-  const int tid = threadIdx.x;
-  const int nthr = blockDim.x;
-  const long total_lines = (long)lines_per_batch * nbatch;
-  const long l0 = (long)blockIdx.x * lpw;
-  const int nl = (int)((total_lines - l0) < lpw ? (total_lines - l0) : lpw);
-  const int L = P.L;
-
-  // load (zero beyond nin)
-  for (int t = tid; t < lpw * L; t += nthr) {
-    int l, i;
-    if (colmajor) {
-      l = t % lpw;
-      i = t / lpw;
-    } else {
-      l = t / L;
-      i = t - l * L;
-    }
-    float2 v = make_float2(0.f, 0.f);
-    if (l < nl && i < nin) {
-      long gl = l0 + l;
-      long b = gl / lines_per_batch;
-      long ll = gl - b * lines_per_batch;
-      v = in[b * bstride + ll * lstride + (long)i * estride];
-    }
-    sm[l * ldl + i] = v;
-  }
+  const int tid = threadIdx.x, nthr = blockDim.x, L = P.L;
+  const long base = line_base(m, blockIdx.x);
+  for (int i = tid; i < L; i += nthr)
+    sm[i] = (i < m.nin || i >= L - m.nin_hi) ? in[base + (long)i * m.estride]
+                                             : make_float2(0.f, 0.f);
   __syncthreads();
-  fft_lds<DIR, NB>(sm, lpw, ldl, P, tid, nthr);
-  for (int t = tid; t < lpw * nout; t += nthr) {
-    int l, i;
-    if (colmajor) {
-      l = t % lpw;
-      i = t / lpw;
-    } else {
-      l = t / nout;
-      i = t - l * nout;
-    }
-    if (l < nl) {
-      long gl = l0 + l;
-      long b = gl / lines_per_batch;
-      long ll = gl - b * lines_per_batch;
-      out[b * bstride + ll * lstride + (long)i * estride] =
-          cscale(sm[l * ldl + i], scale);
-    }
+  fft_lds<DIR, NB>(sm, 1, L, P, tid, nthr);
+  const int nw = m.nout + m.nout_hi;
+  for (int t = tid; t < nw; t += nthr) {
+    const int i = t < m.nout ? t : t + L - nw;
+    out[base + (long)i * m.estride] = cscale(sm[i], m.scale);
   }
 }
 
-template <int DIR, int NB>
-static void launch_lines_nb(const LineFFTArgs& a, const FFTLength& F, int lpw,
-                            int nthr, size_t smem, unsigned nblk,
-                            hipStream_t stream) {
-  auto k = fft_lines_kernel<DIR, NB>;
-  TC_HIP(hipFuncSetAttribute((const void*)k,
-                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)smem));
-  hipLaunchKernelGGL(k, dim3(nblk), dim3(nthr), smem, stream, a.in, a.out,
-                     F.plan(), a.lines_per_batch, a.nbatch, a.bstride,
-                     a.lstride, a.estride, a.nin, a.nout, lpw, F.L(),
-                     a.colmajor ? 1 : 0, a.scale);
+template <int DIR>
+static void launch_lines(const LineFFTArgs& a, hipStream_t stream) {
+  LinesMap m{a.lines_per_batch, a.nin,     a.nin_hi,  a.nout,
+             a.nout_hi,         a.colmajor, (long)a.lines_per_batch * a.nbatch,
+             a.bstride,         a.lstride, a.estride, a.scale};
+  if (m.total == 0) return;
+  if (rt_fits(a.L)) {
+    const RtLaunch l = rt_launch(a.L, m.total, a.colmajor ? 16 : 4);
+    auto k = rt_lines_kernel<DIR>;
+    allow_lds((const void*)k, l.smem);
+    hipLaunchKernelGGL(k, dim3(cdiv(m.total, l.lpw)), dim3(l.nthr), l.smem,
+                       stream, a.in, a.out, l.plan, m, l.lpw);
+    TC_HIP(hipGetLastError());
+    return;
+  }
+  const FFTLength& F = fft_length(a.L);
+  const size_t smem = sizeof(float2) * (size_t)a.L;
+  const int nb = F.nb_for(1, 1024);
+  TC_REQUIRE(smem <= 160 * 1024, "fft_lines: line does not fit in LDS");
+  TC_REQUIRE(nb != 0, "fft_lines: FFT length too large");
+  auto k = nb <= 4 ? fft_lines_kernel<DIR, 4> : fft_lines_kernel<DIR, 8>;
+  allow_lds((const void*)k, smem);
+  hipLaunchKernelGGL(k, dim3((unsigned)m.total), dim3(1024), smem, stream, a.in,
+                     a.out, F.plan(), m);
   TC_HIP(hipGetLastError());
 }
 
+bool fft_ct_enabled() {
+  const char* e = std::getenv("TOMOCAM_HIP_CT_LINES");
+  return !(e && e[0] == '0');
+}
+
 void fft_lines(const LineFFTArgs& a, int dir, hipStream_t stream) {
-  TC_REQUIRE(a.nin <= a.L && a.nout <= a.L, "fft_lines: nin/nout exceed L");
-  {
-    const char* e = std::getenv("TOMOCAM_HIP_CT_LINES");
-    if (!(e && e[0] == '0') && fft_lines_ct(a, dir, stream)) return;
+  TC_REQUIRE(a.nin + a.nin_hi <= a.L && a.nout + a.nout_hi <= a.L,
+             "fft_lines: nin/nout exceed L");
+  if (fft_ct_enabled() && fft_lines_ct(a, dir, stream)) return;
+  if (dir < 0)
+    launch_lines<-1>(a, stream);
+  else
+    launch_lines<1>(a, stream);
+}
+
+// ---------------------------------------------------------------------------
+// real rows and rays on runtime plans (RealRowsArgs, RayArgs): a pair of rows
+// or rays of one slice per line
+// ---------------------------------------------------------------------------
+
+__global__ void __launch_bounds__(RT_MAX_THREADS)
+rt_r2c_rows_kernel(RealRowsArgs a, RtPlan P, int lpw) {
+  extern __shared__ float2 sm[];
+  const int tid = threadIdx.x, nthr = blockDim.x, L = P.L, H = L / 2 + 1;
+  const int npair = (a.nm + 1) / 2, lo = (a.nm + 1) / 2, hi = a.nm / 2;
+  const long g0 = (long)blockIdx.x * lpw, nlines = (long)a.nsl * npair;
+  for (int q = tid; q < lpw * L; q += nthr) {
+    const int l = q / L, i = q - l * L;
+    const long gl = g0 + l;
+    float2 w = make_float2(0.f, 0.f);
+    if (gl < nlines && (i < lo || i >= L - hi)) {
+      const long s = gl / npair;
+      const int ka = 2 * (int)(gl - s * npair);
+      const int k = i < lo ? i + hi : i - (L - hi);
+      const float* f = a.real_in + (s * a.nm + ka) * a.nm;
+      w.x = f[k] * a.corr[k] * a.corr[ka];
+      if (ka + 1 < a.nm) w.y = f[a.nm + k] * a.corr[k] * a.corr[ka + 1];
+    }
+    sm[l * P.ldl + rt_pad(i)] = w;
   }
-  const FFTLength& F = fft_length(a.L);
-  // lines per workgroup: enough for coalescing of column transforms, bounded
-  // by 64 KiB of LDS
-  int lpw = 1;
-  if (a.colmajor) {
-    lpw = (int)std::max<long>(1, std::min<long>(16, 65536 / (8L * a.L)));
+  __syncthreads();
+  const float2* z = rt_fft<-1>(sm, lpw, P, tid, nthr);
+  for (int q = tid; q < lpw * H; q += nthr) {
+    const int l = q / H, k = q - l * H;
+    const long gl = g0 + l;
+    if (gl >= nlines) break;
+    const long s = gl / npair;
+    const int ka = 2 * (int)(gl - s * npair);
+    const float2 zk = z[l * P.ldl + rt_pad(k)];
+    const float2 zm = cconj(z[l * P.ldl + rt_pad(k == 0 ? 0 : L - k)]);
+    const float2 sp = cadd(zk, zm), df = csub(zk, zm);
+    const int ra = ka < hi ? L + ka - hi : ka - hi;
+    const int rb = ka + 1 < hi ? L + ka + 1 - hi : ka + 1 - hi;
+    a.half[(s * L + ra) * a.pitch + k] = make_float2(0.5f * sp.x, 0.5f * sp.y);
+    if (ka + 1 < a.nm)
+      a.half[(s * L + rb) * a.pitch + k] =
+          make_float2(0.5f * df.y, -0.5f * df.x);
+  }
+}
+
+__global__ void __launch_bounds__(RT_MAX_THREADS)
+rt_c2r_rows_kernel(RealRowsArgs a, RtPlan P, int lpw) {
+  extern __shared__ float2 sm[];
+  const int tid = threadIdx.x, nthr = blockDim.x, L = P.L, H = L / 2 + 1;
+  const int npair = (a.nm + 1) / 2, hi = a.nm / 2;
+  const long g0 = (long)blockIdx.x * lpw, nlines = (long)a.nsl * npair;
+  for (int q = tid; q < lpw * H; q += nthr) {
+    const int l = q / H, k = q - l * H;
+    const long gl = g0 + l;
+    float2 x = make_float2(0.f, 0.f), y = x;
+    if (gl < nlines) {
+      const long s = gl / npair;
+      const int ka = 2 * (int)(gl - s * npair);
+      const int ra = ka < hi ? L + ka - hi : ka - hi;
+      const int rb = ka + 1 < hi ? L + ka + 1 - hi : ka + 1 - hi;
+      x = a.half[(s * L + ra) * a.pitch + k];
+      if (ka + 1 < a.nm) y = a.half[(s * L + rb) * a.pitch + k];
+      if (k == 0 || 2 * k == L) x.y = y.y = 0.f;  // real by symmetry
+    }
+    sm[l * P.ldl + rt_pad(k)] = make_float2(x.x - y.y, x.y + y.x);
+    if (k > 0 && L - k >= H)
+      sm[l * P.ldl + rt_pad(L - k)] = make_float2(x.x + y.y, y.x - x.y);
+  }
+  __syncthreads();
+  const float2* z = rt_fft<1>(sm, lpw, P, tid, nthr);
+  for (int q = tid; q < lpw * a.nm; q += nthr) {
+    const int l = q / a.nm, k = q - l * a.nm;
+    const long gl = g0 + l;
+    if (gl >= nlines) break;
+    const long s = gl / npair;
+    const int ka = 2 * (int)(gl - s * npair);
+    const float2 v = z[l * P.ldl + rt_pad(k < hi ? L + k - hi : k - hi)];
+    const float c = a.corr[k];
+    float* o = a.real_out + (s * a.nm + ka) * a.nm + k;
+    o[0] = v.x * c * (a.corr[ka] * a.scale);
+    if (ka + 1 < a.nm) o[a.nm] = v.y * c * (a.corr[ka + 1] * a.scale);
+  }
+}
+
+template <bool TO_HALF>
+__global__ void __launch_bounds__(RT_MAX_THREADS)
+rt_ray_kernel(RayArgs a, RtPlan P, int lpw) {
+  extern __shared__ float2 sm[];
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  const int L = P.L, N = a.N, c = N / 2;
+  const int npair = (a.P + 1) / 2;
+  const long g0 = (long)blockIdx.x * lpw, nlines = (long)a.nsl * npair;
+  for (int t = tid; t < lpw * L; t += nthr) {
+    const int l = t / L, z = t - l * L;
+    const long gl = g0 + l;
+    float2 v = make_float2(0.f, 0.f);
+    if (z < N && gl < nlines) {
+      const long s = gl / npair;
+      const int p = 2 * (int)(gl - s * npair);
+      const bool hasb = p + 1 < a.P;
+      if constexpr (TO_HALF) {
+        const float* r = a.real_in + (s * a.P + p) * N;
+        v.x = r[z] - ray_level(a, r);
+        if (hasb) v.y = r[N + z] - ray_level(a, r + N);
+      } else {
+        const float2* r = a.half_in + (s * a.P + p) * a.nh;
+        v = ray_pair_sample(r, hasb ? r + a.nh : nullptr, z - c, N);
+      }
+      v = cmul(v, a.chirp[z]);
+    }
+    sm[l * P.ldl + rt_pad(z)] = v;
+  }
+  __syncthreads();
+  float2* z = rt_fft<-1>(sm, lpw, P, tid, nthr);
+  for (int t = tid; t < lpw * L; t += nthr) {
+    const int l = t / L, k = t - l * L;
+    float2& v = z[l * P.ldl + rt_pad(k)];
+    v = cmul(v, a.bhat[k]);
+  }
+  __syncthreads();
+  z = rt_fft<1>(sm, lpw, P, tid, nthr, z != sm);
+  for (int t = tid; t < lpw * N; t += nthr) {
+    const int l = t / N, j = t - l * N;
+    const long gl = g0 + l;
+    if (gl >= nlines) break;
+    float2& y = z[l * P.ldl + rt_pad(j)];
+    const float2 v = cmul(y, a.chirp[j]);
+    if constexpr (TO_HALF) {
+      y = v;
+    } else {
+      const long s = gl / npair;
+      const int p = 2 * (int)(gl - s * npair);
+      float* o = a.real_out + (s * a.P + p) * N + j;
+      o[0] = v.x * a.scale;
+      if (p + 1 < a.P) o[N] = v.y * a.scale;
+    }
+  }
+  if constexpr (TO_HALF) {
+    __syncthreads();
+    for (int t = tid; t < lpw * a.nh; t += nthr) {
+      const int l = t / a.nh, m = t - l * a.nh;
+      if (g0 + l >= nlines) break;
+      const float2* y = z + l * P.ldl;
+      ray_store_pair(a, g0 + l, y[rt_pad(c + m < N ? c + m : 0)],
+                     y[rt_pad(c - m)], m);
+    }
+  }
+}
+
+// Rows and rays too long for two LDS buffers: packed into complex lines
+// z[line][L] in memory, transformed there, and taken apart.
+__global__ void long_rows_pack_kernel(RealRowsArgs a, float2* z, int r2c) {
+  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int npair = (a.nm + 1) / 2, hi = a.nm / 2, lo = (a.nm + 1) / 2;
+  if (idx >= (long)a.nsl * npair * a.L) return;
+  const long line = idx / a.L;
+  const int i = (int)(idx - line * a.L);
+  const long s = line / npair;
+  const int ka = 2 * (int)(line - s * npair);
+  const bool hasb = ka + 1 < a.nm;
+  float2 w = make_float2(0.f, 0.f);
+  if (r2c) {
+    if (i < lo || i >= a.L - hi) {
+      const int k = i < lo ? i + hi : i - (a.L - hi);
+      const float* f = a.real_in + (s * a.nm + ka) * a.nm;
+      w.x = f[k] * a.corr[k] * a.corr[ka];
+      if (hasb) w.y = f[a.nm + k] * a.corr[k] * a.corr[ka + 1];
+    }
   } else {
-    lpw = (int)std::max<long>(1, std::min<long>(4, 32768 / (8L * a.L)));
+    const bool low = i <= a.L / 2;
+    const int k = low ? i : a.L - i;
+    const int ra = ka < hi ? a.L + ka - hi : ka - hi;
+    const int rb = ka + 1 < hi ? a.L + ka + 1 - hi : ka + 1 - hi;
+    float2 x = a.half[(s * a.L + ra) * a.pitch + k];
+    float2 y = hasb ? a.half[(s * a.L + rb) * a.pitch + k]
+                    : make_float2(0.f, 0.f);
+    if (k == 0 || 2 * k == a.L) x.y = y.y = 0.f;
+    w = low ? make_float2(x.x - y.y, x.y + y.x)
+            : make_float2(x.x + y.y, y.x - x.y);
   }
-  int nthr = 256;
-  int nb = 0;
-  for (;;) {
-    nb = F.nb_for(lpw, nthr);
-    if (nb != 0 && nb <= 4) break;
-    if (nthr < 1024) {
-      nthr *= 2;
-      continue;
+  z[idx] = w;
+}
+
+__global__ void long_rows_unpack_kernel(RealRowsArgs a, const float2* z,
+                                        int r2c) {
+  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int npair = (a.nm + 1) / 2, hi = a.nm / 2;
+  const int width = r2c ? a.L / 2 + 1 : a.nm;
+  if (idx >= (long)a.nsl * npair * width) return;
+  const long line = idx / width;
+  const int k = (int)(idx - line * width);
+  const long s = line / npair;
+  const int ka = 2 * (int)(line - s * npair);
+  const bool hasb = ka + 1 < a.nm;
+  z += line * a.L;
+  if (r2c) {
+    const float2 zk = z[k], zm = cconj(z[k == 0 ? 0 : a.L - k]);
+    const float2 sp = cadd(zk, zm), df = csub(zk, zm);
+    const int ra = ka < hi ? a.L + ka - hi : ka - hi;
+    const int rb = ka + 1 < hi ? a.L + ka + 1 - hi : ka + 1 - hi;
+    a.half[(s * a.L + ra) * a.pitch + k] =
+        make_float2(0.5f * sp.x, 0.5f * sp.y);
+    if (hasb)
+      a.half[(s * a.L + rb) * a.pitch + k] =
+          make_float2(0.5f * df.y, -0.5f * df.x);
+  } else {
+    const float2 v = z[k < hi ? a.L + k - hi : k - hi];
+    const float c = a.corr[k];
+    float* o = a.real_out + (s * a.nm + ka) * a.nm + k;
+    o[0] = v.x * c * (a.corr[ka] * a.scale);
+    if (hasb) o[a.nm] = v.y * c * (a.corr[ka + 1] * a.scale);
+  }
+}
+
+__global__ void long_rays_pack_kernel(RayArgs a, float2* z, int to_half) {
+  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int npair = (a.P + 1) / 2, c = a.N / 2;
+  if (idx >= (long)a.nsl * npair * a.L) return;
+  const long line = idx / a.L;
+  const int i = (int)(idx - line * a.L);
+  const long s = line / npair;
+  const int p = 2 * (int)(line - s * npair);
+  const bool hasb = p + 1 < a.P;
+  float2 v = make_float2(0.f, 0.f);
+  if (i < a.N) {
+    if (to_half) {
+      const float* r = a.real_in + (s * a.P + p) * a.N;
+      v.x = r[i] - ray_level(a, r);
+      if (hasb) v.y = r[a.N + i] - ray_level(a, r + a.N);
+    } else {
+      const float2* r = a.half_in + (s * a.P + p) * a.nh;
+      v = ray_pair_sample(r, hasb ? r + a.nh : nullptr, i - c, a.N);
     }
-    if (lpw > 1) {
-      lpw /= 2;
-      continue;
+    v = cmul(v, a.chirp[i]);
+  }
+  z[idx] = v;
+}
+
+__global__ void long_rays_mul_kernel(float2* z, const float2* bhat, int L,
+                                     long n) {
+  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx < n) z[idx] = cmul(z[idx], bhat[idx % L]);
+}
+
+__global__ void long_rays_unpack_kernel(RayArgs a, const float2* z,
+                                        int to_half) {
+  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int npair = (a.P + 1) / 2, c = a.N / 2;
+  const int width = to_half ? a.nh : a.N;
+  if (idx >= (long)a.nsl * npair * width) return;
+  const long line = idx / width;
+  const int j = (int)(idx - line * width);
+  z += line * a.L;
+  if (to_half) {
+    const int jp = c + j < a.N ? c + j : 0, jn = c - j;
+    ray_store_pair(a, line, cmul(z[jp], a.chirp[jp]), cmul(z[jn], a.chirp[jn]),
+                   j);
+  } else {
+    const long s = line / npair;
+    const int p = 2 * (int)(line - s * npair);
+    const float2 v = cmul(z[j], a.chirp[j]);
+    float* o = a.real_out + (s * a.P + p) * a.N + j;
+    o[0] = v.x * a.scale;
+    if (p + 1 < a.P) o[a.N] = v.y * a.scale;
+  }
+}
+
+static void long_lines(float2* z, int L, long nlines, int dir,
+                       hipStream_t stream) {
+  LineFFTArgs l;
+  l.in = l.out = z;
+  l.L = l.nin = l.nout = L;
+  l.lines_per_batch = (int)nlines;
+  l.lstride = L;
+  fft_lines(l, dir, stream);
+}
+
+static void long_rows(RealRowsArgs a, bool r2c, hipStream_t stream) {
+  const int nsl = a.nsl, npair = (a.nm + 1) / 2;
+  DevBuf z(sizeof(float2) * (size_t)npair * a.L);
+  a.nsl = 1;  // a slice at a time: the lines take as much room as its half grid
+  for (int s = 0; s < nsl; ++s) {
+    hipLaunchKernelGGL(long_rows_pack_kernel,
+                       dim3(cdiv((size_t)npair * a.L, 256)), dim3(256), 0,
+                       stream, a, z.as<float2>(), r2c ? 1 : 0);
+    TC_HIP(hipGetLastError());
+    long_lines(z.as<float2>(), a.L, npair, r2c ? -1 : 1, stream);
+    const size_t n = (size_t)npair * (r2c ? a.L / 2 + 1 : a.nm);
+    hipLaunchKernelGGL(long_rows_unpack_kernel, dim3(cdiv(n, 256)), dim3(256),
+                       0, stream, a, z.as<float2>(), r2c ? 1 : 0);
+    TC_HIP(hipGetLastError());
+    if (r2c) a.real_in += (long)a.nm * a.nm;
+    else a.real_out += (long)a.nm * a.nm;
+    a.half += (long)a.L * a.pitch;
+  }
+}
+
+static void long_rays(RayArgs a, bool to_half, hipStream_t stream) {
+  const int nsl = a.nsl, npair = (a.P + 1) / 2;
+  const size_t nz = (size_t)npair * a.L;
+  DevBuf z(sizeof(float2) * nz);
+  a.nsl = 1;
+  for (int s = 0; s < nsl; ++s) {
+    hipLaunchKernelGGL(long_rays_pack_kernel, dim3(cdiv(nz, 256)), dim3(256), 0,
+                       stream, a, z.as<float2>(), to_half ? 1 : 0);
+    TC_HIP(hipGetLastError());
+    long_lines(z.as<float2>(), a.L, npair, -1, stream);
+    hipLaunchKernelGGL(long_rays_mul_kernel, dim3(cdiv(nz, 256)), dim3(256), 0,
+                       stream, z.as<float2>(), a.bhat, a.L, (long)nz);
+    TC_HIP(hipGetLastError());
+    long_lines(z.as<float2>(), a.L, npair, 1, stream);
+    const size_t n = (size_t)npair * (to_half ? a.nh : a.N);
+    hipLaunchKernelGGL(long_rays_unpack_kernel, dim3(cdiv(n, 256)), dim3(256),
+                       0, stream, a, z.as<float2>(), to_half ? 1 : 0);
+    TC_HIP(hipGetLastError());
+    if (to_half) {
+      a.real_in += (long)a.P * a.N;
+      a.half_out += (long)a.P * a.nh;
+    } else {
+      a.half_in += (long)a.P * a.nh;
+      a.real_out += (long)a.P * a.N;
     }
-    nb = F.nb_for(lpw, nthr);
-    TC_REQUIRE(nb != 0, "fft_lines: FFT length too large");
-    break;
   }
-  size_t smem = sizeof(float2) * (size_t)lpw * F.L();
-  TC_REQUIRE(smem <= 160 * 1024, "fft_lines: line does not fit in LDS");
-  long total = (long)a.lines_per_batch * a.nbatch;
-  unsigned nblk = cdiv(total, lpw);
-  if (total == 0) return;
-#define TC_LAUNCH(D, B)                                             \
-  if (dir == D && nb == B) {                                        \
-    launch_lines_nb<D, B>(a, F, lpw, nthr, smem, nblk, stream);     \
-    return;                                                         \
-  }
-  TC_LAUNCH(-1, 1) TC_LAUNCH(-1, 2) TC_LAUNCH(-1, 4) TC_LAUNCH(-1, 8)
-  TC_LAUNCH(1, 1) TC_LAUNCH(1, 2) TC_LAUNCH(1, 4) TC_LAUNCH(1, 8)
-#undef TC_LAUNCH
-  throw Error(TC_ERR_INTERNAL, "fft_lines: no kernel for configuration");
+}
+
+void fft_real_rows(const RealRowsArgs& a, bool r2c, hipStream_t stream) {
+  TC_REQUIRE(a.nm >= 1 && a.nm <= a.L && a.L % 2 == 0 &&
+                 a.pitch >= a.L / 2 + 1,
+             "fft_real_rows: bad shape");
+  if (fft_ct_enabled() && fft_real_rows_ct(a, r2c, stream)) return;
+  const long nlines = (long)a.nsl * ((a.nm + 1) / 2);
+  if (nlines == 0) return;
+  if (!rt_fits(a.L)) return long_rows(a, r2c, stream);
+  const RtLaunch l = rt_launch(a.L, nlines, 4);
+  auto k = r2c ? rt_r2c_rows_kernel : rt_c2r_rows_kernel;
+  allow_lds((const void*)k, l.smem);
+  hipLaunchKernelGGL(k, dim3(cdiv(nlines, l.lpw)), dim3(l.nthr), l.smem, stream,
+                     a, l.plan, l.lpw);
+  TC_HIP(hipGetLastError());
+}
+
+void fft_rays(const RayArgs& a, bool to_half, hipStream_t stream) {
+  const long nlines = (long)a.nsl * ((a.P + 1) / 2);
+  if (nlines <= 0) return;
+  if (fft_ct_enabled() && fft_rays_ct(a, to_half, stream)) return;
+  TC_REQUIRE(2 * a.N - 1 <= a.L, "ray DFT: length too short");
+  if (!rt_fits(a.L)) return long_rays(a, to_half, stream);
+  const RtLaunch l = rt_launch(a.L, nlines, 4);
+  auto k = to_half ? rt_ray_kernel<true> : rt_ray_kernel<false>;
+  allow_lds((const void*)k, l.smem);
+  hipLaunchKernelGGL(k, dim3(cdiv(nlines, l.lpw)), dim3(l.nthr), l.smem, stream,
+                     a, l.plan, l.lpw);
+  TC_HIP(hipGetLastError());
 }
 
 // Column transforms restricted to the columns [0, lo) and [cols - hi, cols)

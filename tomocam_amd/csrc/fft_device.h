@@ -242,12 +242,15 @@ class FFTLength {
   const FFTPlan& plan() const { return plan_; }
   int L() const { return plan_.L; }
   int min_radix() const;
+  // radices (largest first) of the two-buffer line transforms (fft.hip)
+  const std::vector<int>& radices() const { return radices_; }
   // Number of butterflies per thread (1, 2, 4 or 8) needed to run `nlines`
   // lines with `nthr` threads.
   int nb_for(int nlines, int nthr) const;
 
  private:
   FFTPlan plan_{};
+  std::vector<int> radices_;
   DevBuf tw_;
 };
 

@@ -1,0 +1,8 @@
+// Line transforms of the lengths of set 5 (fft_lines_ct.h).
+#include "fft_lines_ct.h"
+
+namespace tc {
+
+TC_FOR_LINE_LENGTHS_5(TC_LINE_OPS_DEF)
+
+}  // namespace tc

@@ -16,6 +16,8 @@ struct LineFFTArgs {
   long estride = 1;   // complex elements between elements of a line
   int nin = 0;        // leading input elements read (rest treated as zero)
   int nout = 0;       // leading output elements written
+  int nin_hi = 0;     // trailing input elements read as well
+  int nout_hi = 0;    // trailing output elements written as well
   bool colmajor = false;  // lines adjacent in memory (column transforms)
   float scale = 1.0f;
 };
@@ -26,17 +28,101 @@ struct LineFFTArgs {
 // runtime-plan kernel.
 void fft_lines(const LineFFTArgs& a, int dir, hipStream_t stream);
 
+// Rows of nm real modes <-> the non-redundant half (columns 0 .. L/2) of an
+// L x L Hermitian grid.  Mode index k stands for k - floor(nm/2); row k of
+// slice s is grid row (k - floor(nm/2)) mod L.
+//   r2c: half = forward row transforms of real_in, each value times
+//        corr[row] corr[column]; only the nm mode rows are written;
+//   c2r: real_out = scale corr corr times the inverse (exp(+i), unnormalised)
+//        transforms of the mode rows.
+struct RealRowsArgs {
+  const float* real_in = nullptr;  // [nsl][nm][nm]
+  float* real_out = nullptr;       // [nsl][nm][nm]
+  float2* half = nullptr;          // [nsl][L][pitch]
+  const float* corr = nullptr;     // [nm]
+  int L = 0, nm = 0, nsl = 0;
+  long pitch = 0;  // >= L/2 + 1
+  float scale = 1.0f;
+};
+void fft_real_rows(const RealRowsArgs& a, bool r2c, hipStream_t stream);
+
+// Centred DFTs V[j] = sum_z a[z] exp(sign 2 pi i (j - c)(z - c) / N),
+// c = floor(N/2), between nsl x P real rays of N samples and their half
+// spectra: nh = c + 1 values, V at j - c = 0 .. c.  The other half is its
+// conjugate.  For even N the last value stands for both j - c = -c (the DFT's
+// own sample) and +c, and is stored halved, so that the samples
+// -c .. c weighted alike are the exact DFT.
+//   to_half: half_out = scale (|j - c| / N if ramp) V of real_in;
+//   else:    real_out = scale V of half_in.
+struct RayArgs {
+  const float* real_in = nullptr;    // [nsl][P][N]
+  float* real_out = nullptr;         // [nsl][P][N]
+  const float2* half_in = nullptr;   // [nsl][P][nh]
+  float2* half_out = nullptr;        // [nsl][P][nh]
+  const float2* chirp = nullptr;     // [N]
+  const float2* bhat = nullptr;      // [L]
+  int N = 0, nh = 0, P = 0, nsl = 0, L = 0;
+  bool ramp = false;
+  float scale = 1.0f;
+};
+
+void fft_rays(const RayArgs& a, bool to_half, hipStream_t stream);
+
+// Sample t (centred, -c .. c) of ray a plus i times ray b (b may be null).
+__device__ __forceinline__ float2 ray_pair_sample(const float2* pa,
+                                                  const float2* pb, int t,
+                                                  int N) {
+  const int m = t < 0 ? -t : t;
+  float2 a = pa[m], b = pb ? pb[m] : make_float2(0.f, 0.f);
+  if (t < 0) {
+    a.y = -a.y;
+    b.y = -b.y;
+  }
+  if (2 * m == N) {  // the halves of +c and -c, added
+    a = make_float2(2.f * a.x, 0.f);
+    b = make_float2(2.f * b.x, 0.f);
+  }
+  return make_float2(a.x - b.y, a.y + b.x);
+}
+
+// With the ramp: a level near the ray's mean, taken off before the transform
+// (the DFT of a constant is N at j = c, where the ramp is 0, and 0 elsewhere).
+// The transform's rounding is relative to what is left, which for projections
+// of an object is a fraction of the whole, and the ramp would amplify it (FBP
+// of 16 x 333^2 against 64 bits: 2.6e-6 without, 1.9e-6 with).
+__device__ __forceinline__ float ray_level(const RayArgs& a, const float* ray) {
+  float v = 0.f;
+  if (a.ramp) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v += ray[(long)(2 * k + 1) * a.N / 16];
+  }
+  return 0.125f * v;
+}
+
+// Value m of ray pair `pair` from z = V_a + i V_b at +m (zp; for m = N/2 the
+// value at -m) and at -m (zn).
+__device__ __forceinline__ void ray_store_pair(const RayArgs& a, long pair,
+                                               float2 zp, float2 zn, int m) {
+  const int npair = (a.P + 1) / 2;
+  const long s = pair / npair;
+  const int p = 2 * (int)(pair - s * npair);
+  float f = 0.5f * a.scale;
+  if (a.ramp) f *= (float)m / (float)a.N;
+  if (2 * m == a.N) f *= 0.5f;
+  float2* o = a.half_out + (s * a.P + p) * a.nh + m;
+  o[0] = make_float2(f * (zp.x + zn.x), f * (zp.y - zn.y));
+  if (p + 1 < a.P) o[a.nh] = make_float2(f * (zp.y + zn.y), f * (zn.x - zp.x));
+}
+
 // The compile-time line plans: whether L has one, the smallest planned
-// length >= n (0: none), and the transform (false: no plan for a.L).
+// length >= n (0: none), and the transforms (false: no plan for the length).
 bool fft_lines_ct_has(int L);
 int fft_lines_ct_length(int n);
 bool fft_lines_ct(const LineFFTArgs& a, int dir, hipStream_t stream);
-// Chirp-z DFT of `nrays` rays of N samples on planned length L >= 2N - 1
-// (false: no plan for L): out[j] = chirp[j] IFFT_L(FFT_L(in chirp) bhat)[j]
-// times `scale` (and |j - N/2| / N if `ramp`).
-bool bluestein_ct(const void* in, bool in_real, void* out, bool out_real,
-                  const float2* chirp, const float2* bhat, int N, int L,
-                  long nrays, bool ramp, float scale, hipStream_t stream);
+bool fft_real_rows_ct(const RealRowsArgs& a, bool r2c, hipStream_t stream);
+bool fft_rays_ct(const RayArgs& a, bool to_half, hipStream_t stream);
+// False with TOMOCAM_HIP_CT_LINES=0: the runtime-plan kernels only.
+bool fft_ct_enabled();
 
 // In-place unnormalised 2D transform of `nbatch` complex [rows][cols] arrays.
 void fft2d(float2* data, int nbatch, int rows, int cols, long row_pitch,

@@ -15,6 +15,7 @@
 #include <memory>
 #include <vector>
 
+#include "fft_ops.h"
 #include "tc_common.h"
 
 namespace tc {
@@ -33,21 +34,29 @@ class PolarNufft {
   int nmodes() const { return nm_; }
   int nf() const { return nf_; }
 
+  // Samples of a ray that are stored: those at t = 0 .. floor(N/2).  Both
+  // transforms are of real images, so the samples at t and -t are conjugate.
+  // An even ray's last value is that of its sample t = -N/2, halved; its
+  // other half stands at t = +N/2, which leaves the real part of every sum
+  // as it is.
+  int nh() const { return N_ / 2 + 1; }
+
   // Type 1 (iflag +1): out[s][k2][k1] = scale * Re sum_j c[s][j]
-  // exp(+i (k1 x_j + k2 y_j)); c is [S][P][N] complex, out [S][nm][nm].
+  // exp(+i (k1 x_j + k2 y_j)); c is [S][P][nh] complex, out [S][nm][nm].
   void type1_real(const float2* c, float* out, int S, float scale,
                   hipStream_t stream);
 
   // Type 2 (iflag -1): c[s][j] = sum_k f[s][k2][k1] exp(-i (k1 x_j + k2 y_j))
-  // for real f [S][nm][nm]; c is [S][P][N] complex.
+  // for real f [S][nm][nm]; c is [S][P][nh] complex.
   void type2_real(const float* f, float2* c, int S, hipStream_t stream);
 
  private:
-  int P_, N_, nm_, nf_;
+  int P_, N_, nm_, nf_, pitch_;
   float beta_;
   DevBuf ax_, ay_;   // double[P]: cos/sin(theta) * nf / (N - 1)
   DevBuf corr_;      // float[nm]: (-1)^k h / psi_hat(k)
-  DevBuf fine_;      // float2 [batch][nf][nf]
+  DevBuf fine_;      // float2 [batch][nf][pitch]: columns 0 .. nf/2 of the
+                     // (Hermitian) grid
   int fine_batch_ = 0;
   float2* fine(int batch);
   // Spreading work list, built once per geometry: one item per (fine-grid
@@ -66,6 +75,8 @@ class PolarNufft {
   SpreadArgs spread_args() const;
   void make_segments(hipStream_t stream);
   void make_work(int chunk);
+  RealRowsArgs real_rows(int nsl) const;
+  void columns(int nsl, int dir, hipStream_t stream);
 };
 
 // Centred DFT along rays by Bluestein's algorithm:
@@ -75,14 +86,19 @@ class RayDft {
  public:
   RayDft(int N, int sign);
   int N() const { return N_; }
-  // in: [nrays][N] real (in_real) or complex; out: complex [nrays][N], or
-  // real part only (out_real).  ramp multiplies V[j] by |j - c| / N (the
-  // Ram-Lak filter of src/gpu/ramlak.cu:14-31); scale multiplies the output.
-  void apply(const void* in, bool in_real, void* out, bool out_real,
-             long nrays, bool ramp, float scale, hipStream_t stream);
+  // nsl x P real rays [N] to their half spectra [N/2 + 1] and back (the
+  // stored form of PolarNufft's samples); ramp multiplies V[j] by |j - c| / N
+  // (the Ram-Lak filter of src/gpu/ramlak.cu:14-31); scale multiplies the
+  // output.
+  void to_half(const float* in, float2* out, int nsl, int P, bool ramp,
+               float scale, hipStream_t stream);
+  void to_real(const float2* in, float* out, int nsl, int P, float scale,
+               hipStream_t stream);
 
  private:
+  void run(RayArgs a, bool to_half, hipStream_t stream);
   int N_, L_;
+  bool direct_;   // a planned length N: transformed as it is
   DevBuf chirp_;  // float2[N]: exp(sign i pi (z-c)^2 / N)
   DevBuf bhat_;   // float2[L]: FFT_L of the conjugate chirp, / L
 };

@@ -19,9 +19,22 @@ namespace tc {
 // kernel function and host-side correction factors
 // ---------------------------------------------------------------------------
 
-// exp(beta (sqrt(1 - z^2) - 1)) on |z| <= 1, else 0.  Hardware sqrt and
-// exp2 (about 1 ulp each): the kernel's own approximation error is ~1e-7.
+// exp(beta (sqrt(1 - z^2) - 1)) on |z| <= 1, else 0, with hardware sqrt, rcp
+// and exp2 (about 1 ulp each).
+//
+// Type 1 takes the exponent as -beta z^2 / (1 + sqrt(1 - z^2)): the difference
+// sqrt - 1 carries the root's rounding, times beta, into the weights near the
+// kernel's centre, a level error of up to 6e-7 of an image.  Type 2 keeps the
+// difference form (its weights are those of the earlier kernels, bit for bit),
+// because a residual P x - y amplifies any change of level in P x.
 __device__ __forceinline__ float es_kernel(float z, float beta) {
+  const float s = fmaf(-z, z, 1.0f);
+  const float r = __builtin_amdgcn_sqrtf(fmaxf(s, 0.f)) + 1.0f;
+  const float e = __builtin_amdgcn_exp2f(-1.44269504088896341f * beta *
+                                         (z * z) * __builtin_amdgcn_rcpf(r));
+  return s >= 0.f ? e : 0.f;
+}
+__device__ __forceinline__ float es_kernel_diff(float z, float beta) {
   const float s = 1.0f - z * z;
   const float e = __builtin_amdgcn_exp2f(
       beta * 1.44269504088896341f *
@@ -74,14 +87,15 @@ constexpr int SP_T = 32;
 constexpr int SP_LIST = 2048;  // most projection angles (11 bits of a segment)
 
 struct SpreadArgs {
-  const float2* c;  // [nsl][P][N]
-  float2* fine;     // [nsl][nf][nf]
+  const float2* c;  // [nsl][P][nh]: values at t = 0 .. nh - 1, t < 0 conjugate
+  float2* fine;     // [nsl][nf][pitch], columns 0 .. ncols - 1
   const double* ax;
   const double* ay;
   const int* seg_pj;    // segments of all tiles: p | jlo << 11 | shift << 27
   const int* seg_off;   // their first points' numbers within the tile
   const int* tile_seg;  // [ntiles + 1] first segment of each tile
-  int P, N, cidx, nf, nsl, ntx;
+  int P, N, cidx, nf, nsl, ntx;  // N samples per ray, t = j - cidx
+  int nh, ncols, pitch;
   double umax;
   float beta;
 };
@@ -124,10 +138,10 @@ __device__ __forceinline__ int block_scan_incl(int v, int* wsum) {
 }
 
 // Points per work item: a tile with more points is split into chunks whose
-// partial tiles a fix-up pass adds.  Small grids (fewer than 4096 tiles, a
+// partial tiles a fix-up pass adds.  Small grids (fewer than 2048 tiles, a
 // few workgroups per CU) take 512 so the central tiles, where every ray
 // passes, do not leave a tail; larger grids take 1024 (less fix-up).
-static int spread_chunk(int ntiles) { return ntiles < 4096 ? 512 : 1024; }
+static int spread_chunk(int ntiles) { return ntiles < 2048 ? 512 : 1024; }
 
 struct TileWindow {
   int X0, Y0, X1, Y1;
@@ -141,7 +155,7 @@ __device__ __forceinline__ TileWindow tile_window(const SpreadArgs& a,
   const int tx = tile - ty * a.ntx;
   w.X0 = tx * SP_T;
   w.Y0 = ty * SP_T;
-  w.X1 = min(w.X0 + SP_T, a.nf);
+  w.X1 = min(w.X0 + SP_T, a.ncols);
   w.Y1 = min(w.Y0 + SP_T, a.nf);
   const double hw = 0.5 * NUFFT_W;
   w.lox = w.X0 - hw;
@@ -300,7 +314,7 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
   const int s0 = blockIdx.y * SB;
   const int ns = min(SB, a.nsl - s0);
   const TileWindow w = tile_window(a, item.x);
-  const long sstride = (long)a.P * a.N;
+  const long sstride = (long)a.P * a.nh;
   const int seg1 = segs.y;
   f32x4 acc[4][Q];
 #pragma unroll
@@ -348,15 +362,16 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
       const int pj = sg_pj[lo];
       const int p = pj & 2047;
       const int j = ((pj >> 11) & 0xffff) + (f - sg_off[lo]);
+      const int t = j - a.cidx;
       const float2* cp =
-          a.c + (long)(s0 + half) * sstride + (long)p * a.N + j;
+          a.c + (long)(s0 + half) * sstride + (long)p * a.nh + abs(t);
       float2 cv[Q];
 #pragma unroll
       for (int q = 0; q < Q; ++q)
         cv[q] = 2 * q + half < ns ? cp[2 * q * sstride] : make_float2(0.f, 0.f);
       const double2 o = shift_origin(a, pj >> 27);
       float frac;
-      const int l0 = first_cell(half ? o.y : o.x, (double)(j - a.cidx),
+      const int l0 = first_cell(half ? o.y : o.x, (double)t,
                                 half ? a.ay[p] : a.ax[p], frac) -
                      (half ? w.Y0 : w.X0);  // -7 .. 31
       if (half)
@@ -372,7 +387,7 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
         pt_c[pt][(2 * half) * Q + q] = cv[q].x;
-        pt_c[pt][(2 * half + 1) * Q + q] = cv[q].y;
+        pt_c[pt][(2 * half + 1) * Q + q] = t < 0 ? -cv[q].y : cv[q].y;
       }
       // the segment of the next batch's first point
       if (tid == nb - 1) sg_first = seg + segment_of(fb0 + nb, SP_BATCH + 1);
@@ -451,7 +466,7 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
       if (dst) {
         dst[(s * SP_T + ly) * SP_T + lx] = val;
       } else if (in && s < ns) {
-        a.fine[((long)(s0 + s) * a.nf + w.Y0 + ly) * a.nf + w.X0 + lx] = val;
+        a.fine[((long)(s0 + s) * a.nf + w.Y0 + ly) * a.pitch + w.X0 + lx] = val;
       }
     }
   }
@@ -467,10 +482,13 @@ spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix,
   const int ns = min(sb, a.nsl - s0);
   const int ty = f.x / a.ntx, tx = f.x - (f.x / a.ntx) * a.ntx;
   const int X0 = tx * SP_T, Y0 = ty * SP_T;
-  const int X1 = min(X0 + SP_T, a.nf), Y1 = min(Y0 + SP_T, a.nf);
+  const int X1 = min(X0 + SP_T, a.ncols), Y1 = min(Y0 + SP_T, a.nf);
   // blockIdx.z picks a slice of the group, so a tile's slots are summed by sb
   // workgroups; each thread sums its four elements over the slots four slots
-  // at a time (16 loads in flight); the per-element order is slot order
+  // at a time (16 loads in flight); the per-element order is slot order.
+  // The sums are FP64: the centre's cells add a value of the same sign from
+  // every ray over many slots, and their rounding is a level error of the
+  // whole image (half the grid is stored, so nothing averages it).
   const int s = blockIdx.z;
   if (s >= ns) return;
   constexpr int PER = SP_T * SP_T / 256;
@@ -478,9 +496,9 @@ spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix,
   const float2* base = scratch + (long)f.y * slot_stride +
                        ((long)blockIdx.y * sb + s) * (SP_T * SP_T) +
                        threadIdx.x;
-  float2 sum[PER];
+  double2 sum[PER];
 #pragma unroll
-  for (int e = 0; e < PER; ++e) sum[e] = make_float2(0.f, 0.f);
+  for (int e = 0; e < PER; ++e) sum[e] = make_double2(0.0, 0.0);
   int k = 0;
   for (; k + 4 <= f.z; k += 4) {
     float2 q[4][PER];
@@ -510,9 +528,10 @@ spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix,
     const int cell = threadIdx.x + 256 * e;
     const int ly = cell / SP_T, lx = cell - ly * SP_T;
     if (Y0 + ly < Y1 && X0 + lx < X1) {
-      float2* o = a.fine + ((long)(s0 + s) * a.nf + Y0 + ly) * a.nf + X0 + lx;
+      float2* o =
+          a.fine + ((long)(s0 + s) * a.nf + Y0 + ly) * a.pitch + X0 + lx;
       const float2 cur = *o;
-      *o = make_float2(cur.x + sum[e].x, cur.y + sum[e].y);
+      *o = make_float2((float)(cur.x + sum[e].x), (float)(cur.y + sum[e].y));
     }
   }
 }
@@ -522,14 +541,19 @@ spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix,
 // ---------------------------------------------------------------------------
 
 struct InterpArgs {
-  const float2* fine;  // [nsl][nf][nf]
-  float2* c;           // [nsl][P][N]
+  const float2* fine;  // [nsl][nf][pitch], columns 0 .. nf/2
+  float2* c;           // [nsl][P][nh]
   const double* ax;
   const double* ay;
-  int P, N, cidx, nf, nsl;
+  int P, N, nh, nf, pitch, nsl;
   float beta;
 };
 
+// Samples t and -t of a ray are conjugate (the image is real), so each pair is
+// evaluated once, at whichever of the two lies in the stored half of the grid
+// (columns up to nf/2); a footprint column past either end of that half is
+// read at its mirror image, conjugated.
+//
 // Lane b of a point's group of eight reads footprint column b of every row
 // (its eight rows from one slice are eight loads), so a wave's gather for
 // one row covers eight points x 64 contiguous bytes instead of 64 scattered
@@ -547,19 +571,20 @@ __global__ void __launch_bounds__(256) interp_kernel(InterpArgs a) {
   const long pt = gid >> 3;
   const int b = (int)(gid & 7);
   // groups of eight are aligned to eight lanes: a group is all in or out
-  if (pt >= (long)a.P * a.N) return;
-  const int p = (int)(pt / a.N);
-  const int j = (int)(pt - (long)p * a.N);
-  const double hw = 0.5 * NUFFT_W;
-  const double t = (double)(j - a.cidx);
-  const double u = 0.5 * a.nf + t * a.ax[p];
-  const double v = 0.5 * a.nf + t * a.ay[p];
-  const int l0x = (int)ceil(u - hw);
-  const int l0y = (int)ceil(v - hw);
-  const float wxb = es_kernel((float)((l0x + b - u) * (2.0 / NUFFT_W)), a.beta);
-  const float wyb = es_kernel((float)((l0y + b - v) * (2.0 / NUFFT_W)), a.beta);
+  if (pt >= (long)a.P * a.nh) return;
+  const int p = (int)(pt / a.nh);
+  const int m = (int)(pt - (long)p * a.nh);
+  const double ax = a.ax[p];
+  const double t = ax > 0.0 ? -(double)m : (double)m;
+  float fx, fy;
+  const int l0x = first_cell(0.5 * a.nf, t, ax, fx);
+  const int l0y = first_cell(0.5 * a.nf, t, a.ay[p], fy);
+  const float wxb = es_kernel_diff((fx + (float)b) * (2.0f / NUFFT_W), a.beta);
+  const float wyb = es_kernel_diff((fy + (float)b) * (2.0f / NUFFT_W), a.beta);
   int qx = l0x + b;
   qx += qx < 0 ? a.nf : (qx >= a.nf ? -a.nf : 0);
+  const bool mirror = 2 * qx > a.nf;
+  if (mirror) qx = a.nf - qx;
   float wy[NUFFT_W];
   long roff[NUFFT_W];
 #pragma unroll
@@ -567,10 +592,16 @@ __global__ void __launch_bounds__(256) interp_kernel(InterpArgs a) {
     wy[r] = __shfl(wyb, r, 8);
     int qy = l0y + r;
     qy += qy < 0 ? a.nf : (qy >= a.nf ? -a.nf : 0);
-    roff[r] = (long)qy * a.nf + qx;
+    if (mirror && qy > 0) qy = a.nf - qy;
+    roff[r] = (long)qy * a.pitch + qx;
   }
-  const long plane = (long)a.nf * a.nf;
-  const long cplane = (long)a.P * a.N;
+  const float flip = mirror ? -wxb : wxb;
+  // conjugated where t < 0 was evaluated for t > 0; the sample at the ray's
+  // end of an even N is halved (RayArgs)
+  const float end = 2 * m == a.N ? 0.5f : 1.0f;
+  const float endi = t < 0.0 ? -end : end;
+  const long plane = (long)a.nf * a.pitch;
+  const long cplane = (long)a.P * a.nh;
   for (int s0 = 0; s0 < a.nsl; s0 += 8) {
     float2 part[8];
 #pragma unroll 2
@@ -587,7 +618,7 @@ __global__ void __launch_bounds__(256) interp_kernel(InterpArgs a) {
           acc.y = fmaf(val[r].y, wy[r], acc.y);
         }
       }
-      part[q] = make_float2(acc.x * wxb, acc.y * wxb);
+      part[q] = make_float2(acc.x * wxb, acc.y * flip);
     }
     // lanes with bit m set keep the upper half of their slice set
     float2 h4[4], h2[2];
@@ -612,64 +643,26 @@ __global__ void __launch_bounds__(256) interp_kernel(InterpArgs a) {
     // lane b now holds slice s0 + b (bits 4, 2, 1 of b chose the halves)
     if (s0 + b < a.nsl)
       a.c[(long)(s0 + b) * cplane + pt] =
-          make_float2(keep.x + got.x, keep.y + got.y);
+          make_float2(end * (keep.x + got.x), endi * (keep.y + got.y));
   }
-}
-
-// ---------------------------------------------------------------------------
-// deconvolution: fine-grid spectrum <-> modes k in [-floor(nm/2), ceil(nm/2))
-// ---------------------------------------------------------------------------
-
-__global__ void deconv_real_kernel(const float2* __restrict__ fine, float* out,
-                                   const float* __restrict__ corr, int nm,
-                                   int nf, int nsl, float scale) {
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long per = (long)nm * nm;
-  if (idx >= per * nsl) return;
-  const int s = (int)(idx / per);
-  const int rem = (int)(idx - (long)s * per);
-  const int k2i = rem / nm, k1i = rem - (rem / nm) * nm;
-  const int h = nm / 2;
-  int i1 = k1i - h, i2 = k2i - h;
-  i1 += i1 < 0 ? nf : 0;
-  i2 += i2 < 0 ? nf : 0;
-  const float2 v = fine[((long)s * nf + i2) * nf + i1];
-  out[idx] = v.x * corr[k1i] * corr[k2i] * scale;
-}
-
-__global__ void precorrect_kernel(const float* __restrict__ f, float2* fine,
-                                  const float* __restrict__ corr, int nm,
-                                  int nf, int nsl) {
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long per = (long)nf * nf;
-  if (idx >= per * nsl) return;
-  const int s = (int)(idx / per);
-  const long rem = idx - (long)s * per;
-  const int i2 = (int)(rem / nf), i1 = (int)(rem - (long)i2 * nf);
-  const int h = nm / 2, up = (nm + 1) / 2;
-  int k1 = i1 < up ? i1 : (i1 >= nf - h ? i1 - nf : nf);
-  int k2 = i2 < up ? i2 : (i2 >= nf - h ? i2 - nf : nf);
-  float2 v = make_float2(0.f, 0.f);
-  if (k1 != nf && k2 != nf) {
-    const int k1i = k1 + h, k2i = k2 + h;
-    v.x = f[((long)s * nm + k2i) * nm + k1i] * corr[k1i] * corr[k2i];
-  }
-  fine[idx] = v;
 }
 
 // ---------------------------------------------------------------------------
 // PolarNufft
 // ---------------------------------------------------------------------------
 
-// Fine-grid size for at least m points: the smallest length with a
-// compile-time line FFT plan when it exceeds the smallest even 2,3,5,7-smooth
-// length by at most 1/8 (the planned transforms run several times faster
-// than the runtime-plan kernel, and a larger grid only raises the
-// upsampling factor above 2), else that smooth length.
-static int fine_length(int m) {
-  const int smooth = fft_next_smooth(m, true);
-  const int c = fft_lines_ct_length(m);
-  return (c > 0 && c <= smooth + smooth / 8) ? c : smooth;
+// Fine-grid size for at least m points: of the lengths below the smallest that
+// holds m, when it exceeds the smallest even 2,3,5,7-smooth length by at most
+// 1/8, else that smooth length.  The grid's size sets the kernel's aliasing
+// error (about 1e-7 of the image's level), so it is a fixed rule and not
+// whatever length has a fast plan.
+static int grid_length(int m, bool even) {
+  static const int kGrids[] = {512,  768,  1024, 1458, 1536, 2048, 2304, 2916,
+                               3072, 4374, 4608, 5832, 6144, 8748, 11664};
+  const int smooth = fft_next_smooth(m, even);
+  for (int c : kGrids)
+    if (c >= m) return c <= smooth + smooth / 8 ? c : smooth;
+  return smooth;
 }
 
 PolarNufft::PolarNufft(const float* h_angles, int nproj, int npix, int nmodes)
@@ -678,7 +671,9 @@ PolarNufft::PolarNufft(const float* h_angles, int nproj, int npix, int nmodes)
   TC_REQUIRE(nproj >= 1 && npix >= 2 && nmodes >= 1, "NUFFT: bad geometry");
   TC_REQUIRE(nproj <= SP_LIST, "NUFFT: too many projection angles");
   TC_REQUIRE(npix < 65536, "NUFFT: too many samples per ray");
-  nf_ = fine_length(std::max(2 * nmodes, 2 * NUFFT_W));
+  nf_ = grid_length(std::max(2 * nmodes, 2 * NUFFT_W), true);
+  // half rows in whole 128-byte lines, so that tiles start on one
+  pitch_ = (nf_ / 2 + 1 + 15) / 16 * 16;
   beta_ = (float)(2.30 * NUFFT_W);
   std::vector<double> hx(P_), hy(P_);
   const double sc = (double)nf_ / (double)(npix - 1);
@@ -718,7 +713,7 @@ PolarNufft::PolarNufft(const float* h_angles, int nproj, int npix, int nmodes)
 
 float2* PolarNufft::fine(int batch) {
   if (batch > fine_batch_) {
-    fine_.alloc(sizeof(float2) * (size_t)batch * nf_ * nf_);
+    fine_.alloc(sizeof(float2) * (size_t)batch * nf_ * pitch_);
     fine_batch_ = batch;
   }
   return fine_.as<float2>();
@@ -732,11 +727,14 @@ SpreadArgs PolarNufft::spread_args() const {
   a.seg_off = seg_off_.as<int>();
   a.tile_seg = tile_seg_.as<int>();
   a.P = P_;
-  a.N = N_;
   a.cidx = N_ / 2;
+  a.N = 2 * a.cidx + 1;  // both ends of an even ray (halved values)
+  a.nh = nh();
   a.nf = nf_;
-  a.ntx = (int)cdiv(nf_, SP_T);
-  a.umax = std::max(a.cidx, N_ - 1 - a.cidx) * ((double)nf_ / (N_ - 1)) + 1.0;
+  a.ncols = nf_ / 2 + 1;
+  a.pitch = pitch_;
+  a.ntx = (int)cdiv(a.ncols, SP_T);
+  a.umax = a.cidx * ((double)nf_ / (N_ - 1)) + 1.0;
   a.beta = beta_;
   return a;
 }
@@ -745,9 +743,8 @@ SpreadArgs PolarNufft::spread_args() const {
 // read back once (the work list needs the points per tile), then written.
 void PolarNufft::make_segments(hipStream_t stream) {
   ArenaPause no_arena;  // the plan's lists, offsets filled synchronously
-  const int ntx = (int)cdiv(nf_, SP_T);
-  const int ntiles = ntx * ntx;
   SpreadArgs a = spread_args();
+  const int ntiles = a.ntx * (int)cdiv(nf_, SP_T);
   DevBuf dcounts(sizeof(int) * 2 * ntiles);
   hipLaunchKernelGGL(spread_segments_kernel<false>, dim3(ntiles), dim3(256), 0,
                      stream, a, dcounts.as<int>(), nullptr, nullptr);
@@ -850,8 +847,8 @@ static std::tuple<int, int, int, int, int> chunk_key(int P, int N, int nf,
 // point set-up for fewer slices), rounding up while that stays within
 // 1.25 GB.
 constexpr int SP_SB = 8;
-static int fine_batch(int nf, int S) {
-  const double per = 8.0 * nf * (double)nf, budget = 1.0e9;
+static int fine_batch(int nf, int pitch, int S) {
+  const double per = 8.0 * nf * (double)pitch, budget = 1.0e9;
   const int b0 = (int)std::max(1.0, std::floor(budget / per));
   int b = b0;
   const int up = (b0 + SP_SB - 1) / SP_SB * SP_SB;
@@ -865,14 +862,14 @@ static int fine_batch(int nf, int S) {
 void PolarNufft::type1_real(const float2* c, float* out, int S, float scale,
                             hipStream_t stream) {
   TC_REQUIRE(S >= 1, "NUFFT: need at least one slice");
-  const int B = fine_batch(nf_, S);
+  const int B = fine_batch(nf_, pitch_, S);
   float2* fg = fine(B);
   // slices a spreading workgroup takes: a point's weights and footprint serve
   // all of them, so as many as there are, up to 8 (64 accumulators a lane)
   auto group = [](int nb) { return nb <= 2 ? 2 : nb <= 4 ? 4 : SP_SB; };
   auto args = [&](int s0, int nb) {
     SpreadArgs a = spread_args();
-    a.c = c + (long)s0 * P_ * N_;
+    a.c = c + (long)s0 * P_ * nh();
     a.fine = fg;
     a.nsl = nb;
     return a;
@@ -971,13 +968,12 @@ void PolarNufft::type1_real(const float2* c, float* out, int S, float scale,
     const int nb = std::min(B, S - s0);
     const SpreadArgs a = args(s0, nb);
     spread(a, nb, scratch.as<float2>());
-    // only the columns of modes [-nm/2, (nm+1)/2) are read back
-    fft2d_pruned(fg, nb, nf_, (nm_ + 1) / 2, nm_ / 2, +1, true, stream);
-    const long tot = (long)nb * nm_ * nm_;
-    hipLaunchKernelGGL(deconv_real_kernel, dim3(cdiv(tot, 256)), dim3(256), 0,
-                       stream, fg, out + (long)s0 * nm_ * nm_, corr_.as<float>(),
-                       nm_, nf_, nb, scale);
-    TC_HIP(hipGetLastError());
+    // columns to the mode rows, then real rows
+    columns(nb, +1, stream);
+    RealRowsArgs r = real_rows(nb);
+    r.real_out = out + (long)s0 * nm_ * nm_;
+    r.scale = scale;
+    fft_real_rows(r, false, stream);
   }
   // the scratch slots are released on return: to the thread's arena
   // (reused in stream order) or by hipFree, which waits for the device
@@ -986,93 +982,78 @@ void PolarNufft::type1_real(const float2* c, float* out, int S, float scale,
 void PolarNufft::type2_real(const float* f, float2* c, int S,
                             hipStream_t stream) {
   TC_REQUIRE(S >= 1, "NUFFT: need at least one slice");
-  const int B = fine_batch(nf_, S);
+  const int B = fine_batch(nf_, pitch_, S);
   float2* fg = fine(B);
   for (int s0 = 0; s0 < S; s0 += B) {
     const int nb = std::min(B, S - s0);
-    const long tot = (long)nb * nf_ * nf_;
-    hipLaunchKernelGGL(precorrect_kernel, dim3(cdiv(tot, 256)), dim3(256), 0,
-                       stream, f + (long)s0 * nm_ * nm_, fg, corr_.as<float>(),
-                       nm_, nf_, nb);
-    TC_HIP(hipGetLastError());
-    // only the columns of modes [-nm/2, (nm+1)/2) are non-zero
-    fft2d_pruned(fg, nb, nf_, (nm_ + 1) / 2, nm_ / 2, -1, false, stream);
+    RealRowsArgs r = real_rows(nb);
+    r.real_in = f + (long)s0 * nm_ * nm_;
+    fft_real_rows(r, true, stream);
+    columns(nb, -1, stream);
     InterpArgs a;
     a.fine = fg;
-    a.c = c + (long)s0 * P_ * N_;
+    a.c = c + (long)s0 * P_ * nh();
     a.ax = ax_.as<double>();
     a.ay = ay_.as<double>();
     a.P = P_;
     a.N = N_;
-    a.cidx = N_ / 2;
+    a.nh = nh();
     a.nf = nf_;
+    a.pitch = pitch_;
     a.nsl = nb;
     a.beta = beta_;
-    hipLaunchKernelGGL(interp_kernel, dim3(cdiv(8L * P_ * N_, 256)),
+    hipLaunchKernelGGL(interp_kernel, dim3(cdiv(8L * P_ * a.nh, 256)),
                        dim3(256), 0, stream, a);
     TC_HIP(hipGetLastError());
   }
+}
+
+RealRowsArgs PolarNufft::real_rows(int nsl) const {
+  RealRowsArgs r;
+  r.half = fine_.as<float2>();
+  r.corr = corr_.as<float>();
+  r.L = nf_;
+  r.nm = nm_;
+  r.nsl = nsl;
+  r.pitch = pitch_;
+  return r;
+}
+
+// Column transforms of the half grid in place; of the rows only those of the
+// modes are non-zero on input (dir -1) or wanted on output (dir +1).
+void PolarNufft::columns(int nsl, int dir, hipStream_t stream) {
+  LineFFTArgs a;
+  a.in = a.out = fine_.as<float2>();
+  a.L = nf_;
+  a.nbatch = nsl;
+  a.lines_per_batch = nf_ / 2 + 1;
+  a.bstride = (long)nf_ * pitch_;
+  a.lstride = 1;
+  a.estride = pitch_;
+  a.colmajor = true;
+  const int lo = (nm_ + 1) / 2, hi = nm_ / 2;
+  a.nin = dir < 0 ? lo : nf_;
+  a.nin_hi = dir < 0 ? hi : 0;
+  a.nout = dir < 0 ? nf_ : lo;
+  a.nout_hi = dir < 0 ? 0 : hi;
+  fft_lines(a, dir, stream);
 }
 
 // ---------------------------------------------------------------------------
 // Bluestein ray DFT
 // ---------------------------------------------------------------------------
 
-template <int NB, bool IN_REAL, bool OUT_REAL, bool RAMP>
-__global__ void __launch_bounds__(1024)
-ray_dft_kernel(const void* __restrict__ in, void* __restrict__ out,
-               const float2* __restrict__ chirp, const float2* __restrict__ bhat,
-               FFTPlan P, int N, long nrays, int lpw, float scale) {
-  extern __shared__ float2 sm[];
-  const int tid = threadIdx.x, nthr = blockDim.x;
-  const int L = P.L;
-  const long r0 = (long)blockIdx.x * lpw;
-  for (int t = tid; t < lpw * L; t += nthr) {
-    const int l = t / L;
-    const int z = t - l * L;
-    float2 v = make_float2(0.f, 0.f);
-    if (z < N && r0 + l < nrays) {
-      const long o = (r0 + l) * N + z;
-      float2 a = IN_REAL ? make_float2(static_cast<const float*>(in)[o], 0.f)
-                         : static_cast<const float2*>(in)[o];
-      v = cmul(a, chirp[z]);
-    }
-    sm[t] = v;
-  }
-  __syncthreads();
-  fft_lds<-1, NB>(sm, lpw, L, P, tid, nthr);
-  for (int t = tid; t < lpw * L; t += nthr) {
-    const int k = t - (t / L) * L;
-    sm[t] = cmul(sm[t], bhat[k]);
-  }
-  __syncthreads();
-  fft_lds<1, NB>(sm, lpw, L, P, tid, nthr);
-  const int cidx = N / 2;
-  for (int t = tid; t < lpw * N; t += nthr) {
-    const int l = t / N;
-    const int j = t - l * N;
-    if (r0 + l >= nrays) continue;
-    float2 v = cmul(sm[l * L + j], chirp[j]);
-    float f = scale;
-    if (RAMP) f *= (float)abs(j - cidx) / (float)N;
-    const long o = (r0 + l) * N + j;
-    if (OUT_REAL)
-      static_cast<float*>(out)[o] = v.x * f;
-    else
-      static_cast<float2*>(out)[o] = cscale(v, f);
-  }
-}
-
 RayDft::RayDft(int N, int sign) : N_(N) {
   ArenaPause no_arena;  // cached plan, tables filled synchronously
   TC_REQUIRE(N >= 1, "ray DFT: N must be >= 1");
-  // the chirp-z length: a planned FFT length when within 1/8 of the
-  // smallest 2,3,5,7-smooth one (the planned kernel runs forward transform,
-  // multiply and inverse in registers)
-  {
-    const int smooth = fft_next_smooth(2 * N - 1, false);
+  direct_ = fft_lines_ct_has(N);
+  // The chirp-z length: a planned FFT length where there is one (the planned
+  // kernel runs forward transform, multiply and inverse in registers)
+  if (sign < 0) {
     const int c = fft_lines_ct_length(2 * N - 1);
-    L_ = (c > 0 && c <= smooth + smooth / 8) ? c : smooth;
+    L_ = c > 0 ? c : fft_next_smooth(2 * N - 1, false);
+  } else {
+    L_ = grid_length(2 * N - 1, false);
   }
   const int c = N / 2;
   const long twoN = 2L * N;
@@ -1107,38 +1088,37 @@ RayDft::RayDft(int N, int sign) : N_(N) {
   TC_HIP(hipDeviceSynchronize());
 }
 
-void RayDft::apply(const void* in, bool in_real, void* out, bool out_real,
-                   long nrays, bool ramp, float scale, hipStream_t stream) {
-  if (nrays <= 0) return;
-  {
-    const char* e = std::getenv("TOMOCAM_HIP_CT_LINES");
-    if (!(e && e[0] == '0') &&
-        bluestein_ct(in, in_real, out, out_real, chirp_.as<float2>(),
-                     bhat_.as<float2>(), N_, L_, nrays, ramp, scale, stream))
-      return;
-  }
-  const FFTLength& F = fft_length(L_);
-  LdsLaunch ll = plan_lds_launch(F, 4, 80 * 1024);
-  unsigned nblk = cdiv(nrays, ll.lpw);
-#define TC_RAY(IR, OR, RP)                                                   \
-  if (in_real == IR && out_real == OR && ramp == RP) {                       \
-    TC_DISPATCH_NB(ll.nb, {                                                  \
-      auto k = ray_dft_kernel<NB, IR, OR, RP>;                               \
-      allow_lds((const void*)k, ll.smem);                                    \
-      hipLaunchKernelGGL(k, dim3(nblk), dim3(ll.nthr), ll.smem, stream, in,  \
-                         out, chirp_.as<float2>(), bhat_.as<float2>(),       \
-                         F.plan(), N_, nrays, ll.lpw, scale);                \
-    });                                                                      \
-    TC_HIP(hipGetLastError());                                               \
-    return;                                                                  \
-  }
-  TC_RAY(true, false, false)
-  TC_RAY(true, false, true)
-  TC_RAY(false, true, false)
-  TC_RAY(false, false, false)
-  TC_RAY(true, true, false)
-#undef TC_RAY
-  throw Error(TC_ERR_INTERNAL, "ray DFT: unsupported combination");
+void RayDft::to_half(const float* in, float2* out, int nsl, int P, bool ramp,
+                     float scale, hipStream_t stream) {
+  RayArgs a;
+  a.real_in = in;
+  a.half_out = out;
+  a.nsl = nsl;
+  a.P = P;
+  a.ramp = ramp;
+  a.scale = scale;
+  run(a, true, stream);
+}
+
+void RayDft::to_real(const float2* in, float* out, int nsl, int P, float scale,
+                     hipStream_t stream) {
+  RayArgs a;
+  a.half_in = in;
+  a.real_out = out;
+  a.nsl = nsl;
+  a.P = P;
+  a.scale = scale;
+  run(a, false, stream);
+}
+
+void RayDft::run(RayArgs a, bool to_half, hipStream_t stream) {
+  a.chirp = chirp_.as<float2>();
+  a.bhat = bhat_.as<float2>();
+  a.N = N_;
+  a.nh = N_ / 2 + 1;
+  a.L = L_;
+  if (direct_ && fft_ct_enabled()) a.L = N_;
+  fft_rays(a, to_half, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1227,10 +1207,9 @@ void project(const float* img, float* sino, int S, int N, const float* h_angles,
   TC_REQUIRE(S >= 1 && N >= 2 && P >= 1, "project: bad shape");
   PolarNufft& nu = nufft_plan(h_angles, P, N, N);
   RayDft& rd = ray_dft_plan(N, +1);
-  DevBuf c(sizeof(float2) * (size_t)S * P * N);
+  DevBuf c(sizeof(float2) * (size_t)S * P * nu.nh());
   nu.type2_real(img, c.as<float2>(), S, stream);
-  rd.apply(c.as<float2>(), false, sino, true, (long)S * P, false,
-           1.0f / ((float)N * (float)N), stream);
+  rd.to_real(c.as<float2>(), sino, S, P, 1.0f / ((float)N * (float)N), stream);
 }
 
 void backproject(const float* sino, float* img, int S, int P, int N,
@@ -1238,24 +1217,25 @@ void backproject(const float* sino, float* img, int S, int P, int N,
   TC_REQUIRE(S >= 1 && N >= 2 && P >= 1, "backproject: bad shape");
   PolarNufft& nu = nufft_plan(h_angles, P, N, N);
   RayDft& rd = ray_dft_plan(N, -1);
-  DevBuf c(sizeof(float2) * (size_t)S * P * N);
-  rd.apply(sino, true, c.as<float2>(), false, (long)S * P, fbp, 1.0f, stream);
+  DevBuf c(sizeof(float2) * (size_t)S * P * nu.nh());
+  rd.to_half(sino, c.as<float2>(), S, P, fbp, 1.0f, stream);
   nu.type1_real(c.as<float2>(), img, S, 1.0f / ((float)N * (float)N), stream);
 }
 
-__global__ void fill_ones_kernel(float2* c, long n) {
+// unit samples, the end of an even ray halved (RayArgs)
+__global__ void fill_ones_kernel(float2* c, long n, int nh, int N) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) c[i] = make_float2(1.f, 0.f);
+  if (i < n) c[i] = make_float2(2 * (int)(i % nh) == N ? 0.5f : 1.f, 0.f);
 }
 
 void polar_psf(const float* h_angles, int P, int n, float* d_psf,
                hipStream_t stream) {
   TC_REQUIRE(P >= 1 && n >= 2, "PSF: bad geometry");
   PolarNufft& nu = nufft_plan(h_angles, P, n, 2 * n - 1);
-  DevBuf ones(sizeof(float2) * (size_t)P * n);
-  const long tot = (long)P * n;
+  const long tot = (long)P * nu.nh();
+  DevBuf ones(sizeof(float2) * (size_t)tot);
   hipLaunchKernelGGL(fill_ones_kernel, dim3(cdiv(tot, 256)), dim3(256), 0,
-                     stream, ones.as<float2>(), tot);
+                     stream, ones.as<float2>(), tot, nu.nh(), n);
   TC_HIP(hipGetLastError());
   nu.type1_real(ones.as<float2>(), d_psf, 1, 1.0f, stream);
   TC_HIP(hipStreamSynchronize(stream));
