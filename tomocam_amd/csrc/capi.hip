@@ -316,7 +316,7 @@ int tc_toeplitz_apply_mixed(tc_psf p, const float* d_x, float* d_out,
     tc::Psf& P = get_psf(p);
     TC_REQUIRE(d_x && d_out, "null argument");
     TC_REQUIRE(nslices >= 1, "Toeplitz: need at least one slice");
-    TC_REQUIRE(P.has_fused(), "mixed precision needs a compile-time FFT "
+    TC_REQUIRE(P.has_mixed(), "mixed precision needs a compile-time FFT "
                               "plan; FFT length " + std::to_string(P.M()) +
                               " has none");
     hipStream_t s = as_stream(stream);

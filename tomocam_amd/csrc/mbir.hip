@@ -921,7 +921,7 @@ Run2Stats run2_device(Psf& psf, const float* x0, const float* b, float* out,
   const hipStream_t stream = loop_stream.s;
   float *gsc = nullptr, *gsc_next = nullptr;
   if (opt.mixed) {
-    TC_REQUIRE(psf.has_fused(),
+    TC_REQUIRE(psf.has_mixed(),
                "mixed precision needs a compile-time FFT plan; FFT length " +
                    std::to_string(psf.M()) + " has none");
     bg16.alloc(half_pair_bytes(S, n, n));

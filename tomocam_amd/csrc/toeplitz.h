@@ -95,9 +95,10 @@ class Psf {
                          double* dot_partials, hipStream_t stream,
                          bool wt16 = true);
 
-  // True when this FFT length has the compile-time passes (fused commit and
-  // the mixed-precision forms).
+  // True when this FFT length has the compile-time passes (fused commit), and
+  // when it has the mixed-precision forms as well.
   bool has_fused() const;
+  bool has_mixed() const;
 
   // Autotuner: times one application of the compile-time passes for each
   // candidate slice-group size (half, once and twice the 144 MB rule's) on

@@ -24,6 +24,8 @@ int toeplitz_ct_lpw(int M);
 extern const int kToeplitzCtSizes[];
 extern const float kToeplitzCtCost[];
 extern const int kToeplitzCtCount;
+int toeplitz_plain_length(int m);
+bool toeplitz_ct_mixed(int M);
 
 // Compile-time plan sizes eligible for an n x n Toeplitz product: >= 2n - 1
 // and within 10 % of the smallest even 2,3,5,7-smooth length, ordered by
@@ -60,8 +62,11 @@ static std::pair<int, int> len_key(int n) {
 // FFT length for an n x n Toeplitz product: any even length >= 2n - 1 gives
 // the same result.  The autotuner's choice for this width if there is one;
 // else among the eligible compile-time plan sizes the one with the least
-// size x relative cost per point; with none, the smallest even smooth
-// length.
+// size x relative cost per point; with none, from 486 on the smallest FP32-only
+// plan within 1/8 of the smallest even smooth length, else that length.  (2 x
+// 849^2: 98 us on the runtime-plan kernels, 54 us with the plan; 2 x 3000^2:
+// 1279 us at 6000, 425 us at 6144.  Below 486 a line is a few hundred points
+// and the passes are bound by latency, with a plan or without.)
 int toeplitz_fft_length(int n) {
   {
     // (no device query while nothing is tuned: the rule works without one)
@@ -72,7 +77,10 @@ int toeplitz_fft_length(int n) {
     }
   }
   const std::vector<int> c = toeplitz_ct_candidates(n);
-  return c.empty() ? fft_next_smooth(2 * n - 1, true) : c[0];
+  if (!c.empty()) return c[0];
+  const int smooth = fft_next_smooth(2 * n - 1, true);
+  const int plain = smooth >= 486 ? toeplitz_plain_length(2 * n - 1) : 0;
+  return plain > 0 && plain <= smooth + smooth / 8 ? plain : smooth;
 }
 
 // ---------------------------------------------------------------------------
@@ -453,7 +461,7 @@ bool Psf::run_half(const void* g16, const float* gsc, float* out,
                    hipStream_t stream, bool wt16) {
   TC_REQUIRE(nslices >= 1, "Toeplitz: need at least one slice");
   TC_REQUIRE(g16 && gsc, "Toeplitz: null FP16 input or scales");
-  if (toeplitz_ct_lpw(M_) == 0) return false;
+  if (!has_mixed()) return false;
   const long nspec = (long)M_ * H_;
   // FP32 intermediates read the FP32 spectrum (an FP16 copy measured no
   // faster there, and its rounding accumulated in the MBIR's T sol
@@ -507,6 +515,7 @@ bool Psf::run_half(const void* g16, const float* gsc, float* out,
 }
 
 bool Psf::has_fused() const { return toeplitz_ct_lpw(M_) > 0; }
+bool Psf::has_mixed() const { return toeplitz_ct_mixed(M_); }
 
 void toeplitz_set_group(int H, int rp, int elem_bytes, int nslices,
                         int group);
@@ -518,7 +527,7 @@ __global__ void fill_float_kernel(float* p, long n, float v) {
 }
 
 int Psf::tune_groups(int nslices, bool half, hipStream_t stream) {
-  if (!has_fused() || nslices < 2) return 0;
+  if (!(half ? has_mixed() : has_fused()) || nslices < 2) return 0;
   const int eb = half ? 4 : 8;
   if (toeplitz_group_tuned(H_, rp_, eb, nslices)) return -1;
   const long plane = (long)n_ * n_;
