@@ -33,6 +33,7 @@ int tc_project_f64(const double* d_img, double* d_sino, int nslices, int npix,
                    const double* h_angles, int nproj, void* stream) {
   return tc::guarded([&] {
     TC_REQUIRE(d_img && d_sino && h_angles, "null argument");
+    tc::ArenaScope arena(as_stream(stream));
     tc::f64::project(d_img, d_sino, nslices, npix, h_angles, nproj,
                      as_stream(stream));
   });
@@ -43,6 +44,7 @@ int tc_backproject_f64(const double* d_sino, double* d_img, int nslices,
                        void* stream) {
   return tc::guarded([&] {
     TC_REQUIRE(d_sino && d_img && h_angles, "null argument");
+    tc::ArenaScope arena(as_stream(stream));
     tc::f64::backproject(d_sino, d_img, nslices, nproj, npix, h_angles,
                          fbp != 0, as_stream(stream));
   });
@@ -55,6 +57,7 @@ int tc_gradient_f64(const double* d_x, const double* d_sinoT, double* d_g,
     TC_REQUIRE(d_x && d_sinoT && d_g && h_angles, "null argument");
     TC_REQUIRE(nslices >= 1 && npix >= 2 && nproj >= 1,
                "FP64 gradient: bad shape");
+    tc::ArenaScope arena(as_stream(stream));
     tc::f64::gradient_nufft(d_x, d_sinoT, d_g, nslices, npix, h_angles, nproj,
                             as_stream(stream));
   });
@@ -174,6 +177,7 @@ int tc_mbir2_f64(const double* d_sino, const double* d_x0, double* d_recon,
   return tc::guarded([&] {
     TC_REQUIRE(d_sino && d_recon && h_angles, "null argument");
     TC_REQUIRE(sigma > 0.0, "mbir: sigma must be > 0");
+    tc::ArenaScope arena;
     tc::f64::Result r = tc::f64::mbir2(d_sino, d_x0, d_recon, nslices, nproj,
                                        nrays, h_angles, center, num_iters,
                                        sigma, 1.2, as_stream(stream));
@@ -188,6 +192,7 @@ int tc_mbir_f64(const double* d_sino, const double* d_x0, double* d_recon,
   return tc::guarded([&] {
     TC_REQUIRE(d_sino && d_x0 && d_recon && h_angles, "null argument");
     TC_REQUIRE(sigma > 0.0, "mbir: sigma must be > 0");
+    tc::ArenaScope arena;
     tc::f64::Result r = tc::f64::mbir_nufft(d_sino, d_x0, d_recon, nslices,
                                             nproj, nrays, h_angles, center,
                                             num_iters, sigma, 1.2,

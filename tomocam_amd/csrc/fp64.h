@@ -10,6 +10,9 @@
 // 2 (2n - 1) points).
 #pragma once
 
+#include <mutex>
+
+#include "spread_tiles.h"
 #include "tc_common.h"
 
 namespace tc {
@@ -36,7 +39,11 @@ class Nufft {
   int P_, N_, nm_, nf_;
   DevBuf cs_;    // double2 [P]: cos, sin of the angles
   DevBuf corr_;  // double [nm]: (-1)^k h / psi_hat(k)
-  DevBuf fine_;  // double2 [S][nf][nf]
+  DevBuf ax_, ay_;  // double [P]: grid steps per sample along x and y
+  // spreading lists, built on the first type 1
+  std::mutex mu_;
+  bool lists_ready_ = false;
+  TileLists lists_;
 };
 
 // projector (src/forward.cpp:33-52) and backprojector (src/backward.cpp:

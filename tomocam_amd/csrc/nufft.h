@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "fft_ops.h"
+#include "spread_tiles.h"
 #include "tc_common.h"
 
 namespace tc {
@@ -59,22 +60,12 @@ class PolarNufft {
                      // (Hermitian) grid
   int fine_batch_ = 0;
   float2* fine(int batch);
-  // Spreading work list, built once per geometry: one item per (fine-grid
-  // tile, chunk of at most chunk_ points) so that the tiles near the
-  // centre, which every ray crosses, are split over many workgroups.
+  // Spreading lists, built on the geometry's first type 1: one work item per
+  // (fine-grid tile, chunk of points) so that the tiles near the centre, which
+  // every ray crosses, are split over many workgroups.
   bool work_ready_ = false;
-  int nwork_ = 0, nslots_ = 0, nfix_ = 0, chunk_ = 0;
-  std::vector<int> counts_;      // polar points per fine-grid tile
-  std::vector<int> tile_first_;  // first segment of each tile
-  // ray segments of every tile (device lists, built once per geometry)
-  DevBuf seg_pj_, seg_off_, tile_seg_;
-  // two int4 per item: tile, first point, end point, scratch slot (-1: none);
-  // the tile's segment range
-  DevBuf work_;
-  DevBuf fix_;   // int4: tile, first slot, slot count, 0
+  TileLists lists_;
   SpreadArgs spread_args() const;
-  void make_segments(hipStream_t stream);
-  void make_work(int chunk);
   RealRowsArgs real_rows(int nsl) const;
   void columns(int nsl, int dir, hipStream_t stream);
 };

@@ -78,183 +78,17 @@ static void gauss_legendre(int n, std::vector<double>& x, std::vector<double>& w
 
 // ---------------------------------------------------------------------------
 // spreading (type 1): each workgroup owns a T x T tile of the fine grid and
-// adds every polar point whose kernel footprint meets it.  The ray segments
-// that meet a tile are enumerated analytically, once per geometry (no sorting
-// and no global atomics).
+// adds every polar point whose kernel footprint meets it, from the geometry's
+// segment lists (spread_tiles.h): no sorting and no global atomics.
 // ---------------------------------------------------------------------------
 
-constexpr int SP_T = 32;
-constexpr int SP_LIST = 2048;  // most projection angles (11 bits of a segment)
-
 struct SpreadArgs {
+  TileGeom g;       // columns 0 .. g.ncols - 1 of the grid
   const float2* c;  // [nsl][P][nh]: values at t = 0 .. nh - 1, t < 0 conjugate
-  float2* fine;     // [nsl][nf][pitch], columns 0 .. ncols - 1
-  const double* ax;
-  const double* ay;
-  const int* seg_pj;    // segments of all tiles: p | jlo << 11 | shift << 27
-  const int* seg_off;   // their first points' numbers within the tile
-  const int* tile_seg;  // [ntiles + 1] first segment of each tile
-  int P, N, cidx, nf, nsl, ntx;  // N samples per ray, t = j - cidx
-  int nh, ncols, pitch;
-  double umax;
+  float2* fine;     // [nsl][nf][pitch]
+  int nsl, nh, pitch;
   float beta;
 };
-
-// { t : lo < U0 + t a <= hi } intersected into [tlo, thi] (superset bounds)
-__device__ __forceinline__ void ray_interval(double a, double U0, double lo,
-                                             double hi, double& tlo,
-                                             double& thi) {
-  if (fabs(a) < 1e-12) {
-    if (!(U0 > lo - 1e-9 && U0 <= hi + 1e-9)) {
-      tlo = 1e30;
-      thi = -1e30;
-    }
-    return;
-  }
-  double t1 = (lo - U0) / a, t2 = (hi - U0) / a;
-  if (t1 > t2) {
-    double q = t1;
-    t1 = t2;
-    t2 = q;
-  }
-  tlo = fmax(tlo, t1);
-  thi = fmin(thi, t2);
-}
-
-// Inclusive prefix sum of one int per thread over a 256-thread block.
-__device__ __forceinline__ int block_scan_incl(int v, int* wsum) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int u = __shfl_up(v, d, 64);
-    if (lane >= d) v += u;
-  }
-  if (lane == 63) wsum[wid] = v;
-  __syncthreads();
-  int off = 0;
-  for (int w = 0; w < wid; ++w) off += wsum[w];
-  __syncthreads();
-  return v + off;
-}
-
-// Points per work item: a tile with more points is split into chunks whose
-// partial tiles a fix-up pass adds.  Small grids (fewer than 2048 tiles, a
-// few workgroups per CU) take 512 so the central tiles, where every ray
-// passes, do not leave a tail; larger grids take 1024 (less fix-up).
-static int spread_chunk(int ntiles) { return ntiles < 2048 ? 512 : 1024; }
-
-struct TileWindow {
-  int X0, Y0, X1, Y1;
-  double lox, hix, loy, hiy;
-};
-
-__device__ __forceinline__ TileWindow tile_window(const SpreadArgs& a,
-                                                  int tile) {
-  TileWindow w;
-  const int ty = tile / a.ntx;
-  const int tx = tile - ty * a.ntx;
-  w.X0 = tx * SP_T;
-  w.Y0 = ty * SP_T;
-  w.X1 = min(w.X0 + SP_T, a.ncols);
-  w.Y1 = min(w.Y0 + SP_T, a.nf);
-  const double hw = 0.5 * NUFFT_W;
-  w.lox = w.X0 - hw;
-  w.hix = w.X1 - 1 + hw;
-  w.loy = w.Y0 - hw;
-  w.hiy = w.Y1 - 1 + hw;
-  return w;
-}
-
-__device__ __forceinline__ bool shift_skipped(const SpreadArgs& a,
-                                              const TileWindow& w, double U0,
-                                              double V0) {
-  return U0 + a.umax <= w.lox || U0 - a.umax > w.hix ||
-         V0 + a.umax <= w.loy || V0 - a.umax > w.hiy;
-}
-
-// grid origin of periodic copy `shift` (0 .. 8, row-major over ky, kx)
-__device__ __forceinline__ double2 shift_origin(const SpreadArgs& a,
-                                                int shift) {
-  const int ky = shift / 3 - 1, kx = shift - (shift / 3) * 3 - 1;
-  return make_double2(0.5 * a.nf + kx * (double)a.nf,
-                      0.5 * a.nf + ky * (double)a.nf);
-}
-
-// first footprint cell and its distance from the point, along one axis (fma
-// so that every kernel rounds the coordinate alike)
-__device__ __forceinline__ int first_cell(double origin, double t, double step,
-                                          float& frac) {
-  const double u = fma(t, step, origin);
-  const double c = ceil(u - 0.5 * NUFFT_W);
-  frac = (float)(c - u);
-  return (int)c;
-}
-
-// Segments of one tile, counted (FILL false: counts[tile] = points,
-// counts[ntiles + tile] = segments) or written to the plan's lists.  Thread t
-// examines angles t, t + 256, ... of each periodic copy, in turn; a segment is
-// trimmed to the samples whose footprints really meet the tile.  The order
-// (copy, then a block-scanned order of the angles) is fixed, so every call of
-// the geometry adds a tile's points in the same order.
-template <bool FILL>
-__global__ void __launch_bounds__(256)
-spread_segments_kernel(SpreadArgs a, int* counts, int* seg_pj, int* seg_off) {
-  __shared__ int wsum[4];
-  __shared__ int carry[2];
-  const int tile = blockIdx.x, tid = threadIdx.x;
-  const TileWindow w = tile_window(a, tile);
-  const int s0 = FILL ? a.tile_seg[tile] : 0;
-  int nseg = 0, npts = 0;
-  for (int shift = 0; shift < 9; ++shift) {
-    const double2 o = shift_origin(a, shift);
-    if (shift_skipped(a, w, o.x, o.y)) continue;
-    for (int p0 = 0; p0 < a.P; p0 += 256) {
-      const int p = p0 + tid;
-      int jl = 1, jh = 0;
-      if (p < a.P) {
-        const double ax = a.ax[p], ay = a.ay[p];
-        double tlo = -1e30, thi = 1e30;
-        ray_interval(ax, o.x, w.lox, w.hix, tlo, thi);
-        ray_interval(ay, o.y, w.loy, w.hiy, tlo, thi);
-        if (tlo <= thi) {
-          tlo = fmax(tlo, -(double)a.N - 2.0);
-          thi = fmin(thi, (double)a.N + 2.0);
-          jl = max(0, (int)floor(tlo) + a.cidx - 1);
-          jh = min(a.N - 1, (int)ceil(thi) + a.cidx + 1);
-          auto meets = [&](int j) {
-            float f;
-            const double t = (double)(j - a.cidx);
-            const int lx = first_cell(o.x, t, ax, f);
-            const int ly = first_cell(o.y, t, ay, f);
-            return lx < w.X1 && lx + NUFFT_W > w.X0 && ly < w.Y1 &&
-                   ly + NUFFT_W > w.Y0;
-          };
-          while (jl <= jh && !meets(jl)) ++jl;
-          while (jl <= jh && !meets(jh)) --jh;
-        }
-      }
-      const int len = max(0, jh - jl + 1), has = len > 0;
-      const int iseg = block_scan_incl(has, wsum);
-      const int ipts = block_scan_incl(len, wsum);
-      if (FILL && has) {
-        seg_pj[s0 + nseg + iseg - 1] = p | (jl << 11) | (shift << 27);
-        seg_off[s0 + nseg + iseg - 1] = npts + ipts - len;
-      }
-      if (tid == 255) {
-        carry[0] = iseg;
-        carry[1] = ipts;
-      }
-      __syncthreads();
-      nseg += carry[0];
-      npts += carry[1];
-      __syncthreads();
-    }
-  }
-  if (!FILL && tid == 0) {
-    counts[tile] = npts;
-    counts[gridDim.x + tile] = nseg;
-  }
-}
 
 // One workgroup per (work item, group of SB slices): the points [f0, f1) of
 // its tile as a matrix product on the matrix cores.  The tile is 16 regions
@@ -276,20 +110,10 @@ spread_segments_kernel(SpreadArgs a, int* counts, int* seg_pj, int* seg_off) {
 // writing the grid.
 constexpr int SP_BATCH = 128;
 
-// Rows and columns of wave w's region g: each pair of 4-row bands has one
-// region of every wave, and so has each column half over two pairs.  A batch
-// is a few neighbouring rays, which may cross the tile along a few rows or
-// columns; with eight whole rows to a wave, such a batch left most waves idle.
-__device__ __forceinline__ int region_y(int w, int g) {
-  return 8 * g + 4 * (((w - g) & 3) >> 1);
-}
-__device__ __forceinline__ int region_x(int w, int g) {
-  return 16 * ((w - g) & 1);
-}
 using f32x4 = __attribute__((__vector_size__(4 * sizeof(float)))) float;
 
 template <int SB>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(64 * SP_WAVES)
 spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
   constexpr int Q = SB / 2;  // slice pairs
   // rows padded so that one thread a row writes 16 bytes without conflicts
@@ -300,8 +124,9 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
   // [Re, Im of even slices, Re, Im of odd slices][slice pair]
   __shared__ alignas(16) float pt_c[SP_BATCH][CS];
   __shared__ short2 pt_geo[SP_BATCH];  // (index | l0x << 8, l0y)
-  __shared__ int wlist[4][SP_BATCH + 12];
-  __shared__ int sg_off[SP_BATCH + 1], sg_pj[SP_BATCH];
+  __shared__ int wlist[SP_WAVES][SP_BATCH + 12];
+  __shared__ int sg_off[SP_BATCH + 1];
+  __shared__ int2 sg[SP_BATCH];
   __shared__ int sg_first;
   static_assert(SP_T == 32, "four 8-row bands per tile");
   const int tid = threadIdx.x;
@@ -313,12 +138,12 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
   const int4 segs = work[2 * wi + 1];  // the tile's segments [x, y)
   const int s0 = blockIdx.y * SB;
   const int ns = min(SB, a.nsl - s0);
-  const TileWindow w = tile_window(a, item.x);
-  const long sstride = (long)a.P * a.nh;
+  const TileWindow w = tile_window(a.g, item.x);
+  const long sstride = (long)a.g.P * a.nh;
   const int seg1 = segs.y;
-  f32x4 acc[4][Q];
+  f32x4 acc[SP_REGIONS][Q];
 #pragma unroll
-  for (int g = 0; g < 4; ++g)
+  for (int g = 0; g < SP_REGIONS; ++g)
 #pragma unroll
     for (int q = 0; q < Q; ++q) acc[g][q] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (tid < SP_BATCH) {
@@ -328,9 +153,9 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
   int seg = segs.x;
   if (item.y > 0) {
     // the segment that holds point f0 (offsets ascend from 0 at segs.x)
-    for (int i = seg + tid; i < seg1; i += 256) {
-      const int nxt = i + 1 < seg1 ? a.seg_off[i + 1] : 0x7fffffff;
-      if (a.seg_off[i] <= item.y && item.y < nxt) sg_first = i;
+    for (int i = seg + tid; i < seg1; i += 64 * SP_WAVES) {
+      const int nxt = i + 1 < seg1 ? a.g.seg_off[i + 1] : 0x7fffffff;
+      if (a.g.seg_off[i] <= item.y && item.y < nxt) sg_first = i;
     }
     __syncthreads();
     seg = sg_first;
@@ -343,8 +168,8 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
     // the batch's segments: every segment has a point, so at most nb of them
     if (tid <= SP_BATCH) {
       const int i = seg + tid;
-      sg_off[tid] = i < seg1 ? a.seg_off[i] : 0x7fffffff;
-      if (tid < SP_BATCH) sg_pj[tid] = i < seg1 ? a.seg_pj[i] : 0;
+      sg_off[tid] = i < seg1 ? a.g.seg_off[i] : 0x7fffffff;
+      if (tid < SP_BATCH) sg[tid] = i < seg1 ? a.g.seg[i] : make_int2(0, 0);
     }
     __syncthreads();
     auto segment_of = [&](int f, int n) {  // sg_off[lo] <= f < sg_off[lo + 1]
@@ -359,20 +184,18 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
     if (pt < nb) {
       const int f = fb0 + pt;
       const int lo = segment_of(f, SP_BATCH);
-      const int pj = sg_pj[lo];
-      const int p = pj & 2047;
-      const int j = ((pj >> 11) & 0xffff) + (f - sg_off[lo]);
-      const int t = j - a.cidx;
+      const int p = sg[lo].x, js = sg[lo].y;
+      const int t = (js & 0xffff) + (f - sg_off[lo]) - a.g.cidx;
       const float2* cp =
           a.c + (long)(s0 + half) * sstride + (long)p * a.nh + abs(t);
       float2 cv[Q];
 #pragma unroll
       for (int q = 0; q < Q; ++q)
         cv[q] = 2 * q + half < ns ? cp[2 * q * sstride] : make_float2(0.f, 0.f);
-      const double2 o = shift_origin(a, pj >> 27);
+      const double2 o = shift_origin(a.g, js >> 16);
       float frac;
-      const int l0 = first_cell(half ? o.y : o.x, (double)t,
-                                half ? a.ay[p] : a.ax[p], frac) -
+      const int l0 = first_cell<NUFFT_W>(half ? o.y : o.x, (double)t,
+                                         half ? a.g.ay[p] : a.g.ax[p], frac) -
                      (half ? w.Y0 : w.X0);  // -7 .. 31
       if (half)
         pt_geo[pt].y = (short)l0;
@@ -397,7 +220,7 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
     __syncthreads();
     seg = sg_first;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
+    for (int g = 0; g < SP_REGIONS; ++g) {
       const int ry = region_y(wave, g), rx = region_x(wave, g);
       // points whose footprints meet the region, in point order: index and
       // footprint origin in the region, plus 8
@@ -456,7 +279,7 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
                            : scratch + ((long)item.w * gridDim.y + blockIdx.y) *
                                            (SB * SP_T * SP_T);
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
+  for (int g = 0; g < SP_REGIONS; ++g) {
     const int ly = region_y(wave, g) + lk, lx = region_x(wave, g) + lm;
     const bool in = w.Y0 + ly < w.Y1 && w.X0 + lx < w.X1;
 #pragma unroll
@@ -466,7 +289,8 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
       if (dst) {
         dst[(s * SP_T + ly) * SP_T + lx] = val;
       } else if (in && s < ns) {
-        a.fine[((long)(s0 + s) * a.nf + w.Y0 + ly) * a.pitch + w.X0 + lx] = val;
+        a.fine[((long)(s0 + s) * a.g.nf + w.Y0 + ly) * a.pitch + w.X0 + lx] =
+            val;
       }
     }
   }
@@ -480,15 +304,14 @@ spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix,
   const int4 f = fix[blockIdx.x];
   const int s0 = blockIdx.y * sb;
   const int ns = min(sb, a.nsl - s0);
-  const int ty = f.x / a.ntx, tx = f.x - (f.x / a.ntx) * a.ntx;
-  const int X0 = tx * SP_T, Y0 = ty * SP_T;
-  const int X1 = min(X0 + SP_T, a.ncols), Y1 = min(Y0 + SP_T, a.nf);
-  // blockIdx.z picks a slice of the group, so a tile's slots are summed by sb
-  // workgroups; each thread sums its four elements over the slots four slots
-  // at a time (16 loads in flight); the per-element order is slot order.
-  // The sums are FP64: the centre's cells add a value of the same sign from
-  // every ray over many slots, and their rounding is a level error of the
-  // whole image (half the grid is stored, so nothing averages it).
+  const TileWindow w = tile_window(a.g, f.x);
+  // blockIdx.z picks a slice of the group; each thread sums four cells over the
+  // slots, four slots at a time (16 loads in flight); the order per cell is slot
+  // order.  (One cell a thread and sixteen slots at a time, four times the
+  // workgroups: 22 instead of 11 us at 8 x 512^2, where most tiles have few
+  // slots.)  The sums are FP64: the centre's cells add a value of the same sign
+  // from every ray over many slots, and their rounding is a level error of the
+  // whole image.
   const int s = blockIdx.z;
   if (s >= ns) return;
   constexpr int PER = SP_T * SP_T / 256;
@@ -527,9 +350,9 @@ spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix,
   for (int e = 0; e < PER; ++e) {
     const int cell = threadIdx.x + 256 * e;
     const int ly = cell / SP_T, lx = cell - ly * SP_T;
-    if (Y0 + ly < Y1 && X0 + lx < X1) {
-      float2* o =
-          a.fine + ((long)(s0 + s) * a.nf + Y0 + ly) * a.pitch + X0 + lx;
+    if (w.Y0 + ly < w.Y1 && w.X0 + lx < w.X1) {
+      float2* o = a.fine + ((long)(s0 + s) * a.g.nf + w.Y0 + ly) * a.pitch +
+                  w.X0 + lx;
       const float2 cur = *o;
       *o = make_float2((float)(cur.x + sum[e].x), (float)(cur.y + sum[e].y));
     }
@@ -577,8 +400,8 @@ __global__ void __launch_bounds__(256) interp_kernel(InterpArgs a) {
   const double ax = a.ax[p];
   const double t = ax > 0.0 ? -(double)m : (double)m;
   float fx, fy;
-  const int l0x = first_cell(0.5 * a.nf, t, ax, fx);
-  const int l0y = first_cell(0.5 * a.nf, t, a.ay[p], fy);
+  const int l0x = first_cell<NUFFT_W>(0.5 * a.nf, t, ax, fx);
+  const int l0y = first_cell<NUFFT_W>(0.5 * a.nf, t, a.ay[p], fy);
   const float wxb = es_kernel_diff((fx + (float)b) * (2.0f / NUFFT_W), a.beta);
   const float wyb = es_kernel_diff((fy + (float)b) * (2.0f / NUFFT_W), a.beta);
   int qx = l0x + b;
@@ -669,7 +492,7 @@ PolarNufft::PolarNufft(const float* h_angles, int nproj, int npix, int nmodes)
     : P_(nproj), N_(npix), nm_(nmodes) {
   ArenaPause no_arena;  // cached plan, tables filled synchronously
   TC_REQUIRE(nproj >= 1 && npix >= 2 && nmodes >= 1, "NUFFT: bad geometry");
-  TC_REQUIRE(nproj <= SP_LIST, "NUFFT: too many projection angles");
+  TC_REQUIRE(nproj <= 2048, "NUFFT: too many projection angles");
   TC_REQUIRE(npix < 65536, "NUFFT: too many samples per ray");
   nf_ = grid_length(std::max(2 * nmodes, 2 * NUFFT_W), true);
   // half rows in whole 128-byte lines, so that tiles start on one
@@ -721,111 +544,20 @@ float2* PolarNufft::fine(int batch) {
 
 SpreadArgs PolarNufft::spread_args() const {
   SpreadArgs a{};
-  a.ax = ax_.as<double>();
-  a.ay = ay_.as<double>();
-  a.seg_pj = seg_pj_.as<int>();
-  a.seg_off = seg_off_.as<int>();
-  a.tile_seg = tile_seg_.as<int>();
-  a.P = P_;
-  a.cidx = N_ / 2;
-  a.N = 2 * a.cidx + 1;  // both ends of an even ray (halved values)
+  a.g.ax = ax_.as<double>();
+  a.g.ay = ay_.as<double>();
+  a.g.P = P_;
+  a.g.cidx = N_ / 2;
+  a.g.N = 2 * a.g.cidx + 1;  // both ends of an even ray (halved values)
+  a.g.nf = nf_;
+  a.g.ncols = nf_ / 2 + 1;
+  a.g.ntx = (int)cdiv(a.g.ncols, SP_T);
+  a.g.umax = a.g.cidx * ((double)nf_ / (N_ - 1)) + 1.0;
+  lists_.fill(a.g);
   a.nh = nh();
-  a.nf = nf_;
-  a.ncols = nf_ / 2 + 1;
   a.pitch = pitch_;
-  a.ntx = (int)cdiv(a.ncols, SP_T);
-  a.umax = a.cidx * ((double)nf_ / (N_ - 1)) + 1.0;
   a.beta = beta_;
   return a;
-}
-
-// The ray segments of every tile of this geometry: counted on the device,
-// read back once (the work list needs the points per tile), then written.
-void PolarNufft::make_segments(hipStream_t stream) {
-  ArenaPause no_arena;  // the plan's lists, offsets filled synchronously
-  SpreadArgs a = spread_args();
-  const int ntiles = a.ntx * (int)cdiv(nf_, SP_T);
-  DevBuf dcounts(sizeof(int) * 2 * ntiles);
-  hipLaunchKernelGGL(spread_segments_kernel<false>, dim3(ntiles), dim3(256), 0,
-                     stream, a, dcounts.as<int>(), nullptr, nullptr);
-  TC_HIP(hipGetLastError());
-  std::vector<int> h(2 * (size_t)ntiles);
-  TC_HIP(hipMemcpyAsync(h.data(), dcounts.as<void>(), sizeof(int) * h.size(),
-                        hipMemcpyDeviceToHost, stream));
-  TC_HIP(hipStreamSynchronize(stream));
-  counts_.assign(h.begin(), h.begin() + ntiles);
-  std::vector<int>& first = tile_first_;
-  first.assign(ntiles + 1, 0);
-  for (int t = 0; t < ntiles; ++t) first[t + 1] = first[t] + h[ntiles + t];
-  tile_seg_.alloc(sizeof(int) * first.size());
-  TC_HIP(hipMemcpy(tile_seg_.as<void>(), first.data(),
-                   sizeof(int) * first.size(), hipMemcpyHostToDevice));
-  const size_t nseg = std::max(1, first[ntiles]);
-  seg_pj_.alloc(sizeof(int) * nseg);
-  seg_off_.alloc(sizeof(int) * nseg);
-  a = spread_args();
-  hipLaunchKernelGGL(spread_segments_kernel<true>, dim3(ntiles), dim3(256), 0,
-                     stream, a, nullptr, seg_pj_.as<int>(), seg_off_.as<int>());
-  TC_HIP(hipGetLastError());
-}
-
-// The work and fix-up lists for `chunk` points per item, uploaded to the
-// plan's buffers (synchronous copies: the caller has no kernel reading the
-// previous lists in flight).
-void PolarNufft::make_work(int chunk) {
-  ArenaPause no_arena;  // the plan's work lists, filled synchronously
-  const int ntiles = (int)counts_.size();
-  std::vector<int4> work, fix;
-  int slot = 0;
-  for (int t = 0; t < ntiles; ++t) {
-    const int c = counts_[t];
-    const int nch = std::max(1, (c + chunk - 1) / chunk);
-    work.push_back(make_int4(t, 0, std::min(c, chunk), -1));
-    if (nch > 1) {
-      fix.push_back(make_int4(t, slot, nch - 1, 0));
-      for (int k = 1; k < nch; ++k)
-        work.push_back(make_int4(t, k * chunk, std::min(c, (k + 1) * chunk),
-                                 slot++));
-    }
-  }
-  // Heaviest items first: a workgroup's time grows with its points, and
-  // workgroups start in block order, so the long ones must not be last
-  // (16 x 2908^2 at 1501 angles: 28.6 -> 19.9 ms per backprojection).
-  // Block b reads item xcd_remap(b) (each XCD takes a contiguous range of
-  // the list), so rank b of the sorted order goes to index xcd_remap(b).
-  // Each item writes its own tile or slot, and the fix-up adds slots in
-  // slot order, so the result does not depend on the order.
-  {
-    std::vector<int4> byw(work);
-    std::stable_sort(byw.begin(), byw.end(), [](const int4& x, const int4& y) {
-      return x.z - x.y > y.z - y.y;
-    });
-    const int n = (int)byw.size();
-    const int q = n >> 3, rmd = n & 7;
-    for (int b = 0; b < n; ++b) {
-      const int x = b & 7, t = b >> 3;
-      work[x * q + (x < rmd ? x : rmd) + t] = byw[b];
-    }
-  }
-  // each item with its tile's range of segments
-  std::vector<int4> items;
-  items.reserve(2 * work.size());
-  for (const int4& x : work) {
-    items.push_back(x);
-    items.push_back(make_int4(tile_first_[x.x], tile_first_[x.x + 1], 0, 0));
-  }
-  nwork_ = (int)work.size();
-  nslots_ = slot;
-  nfix_ = (int)fix.size();
-  chunk_ = chunk;
-  work_.alloc(sizeof(int4) * items.size());
-  TC_HIP(hipMemcpy(work_.as<void>(), items.data(), sizeof(int4) * items.size(),
-                   hipMemcpyHostToDevice));
-  if (nfix_) {
-    fix_.alloc(sizeof(int4) * nfix_);
-    TC_HIP(hipMemcpy(fix_.as<void>(), fix.data(), sizeof(int4) * nfix_,
-                     hipMemcpyHostToDevice));
-  }
 }
 
 // Spreading chunks picked by the autotuner, keyed by (device, angles, ray
@@ -880,28 +612,30 @@ void PolarNufft::type1_real(const float2* c, float* out, int S, float scale,
     const unsigned ng = cdiv(nb, sb);
     auto k = sb == 2 ? spread_kernel<2> : sb == 4 ? spread_kernel<4>
                                                   : spread_kernel<SP_SB>;
-    hipLaunchKernelGGL(k, dim3((unsigned)nwork_, ng), dim3(256), 0, stream, a,
-                       work_.as<int4>(), scratch);
+    hipLaunchKernelGGL(k, dim3((unsigned)lists_.nwork(), ng),
+                       dim3(64 * SP_WAVES), 0, stream, a,
+                       lists_.work(), scratch);
     TC_HIP(hipGetLastError());
-    if (nfix_) {
-      hipLaunchKernelGGL(spread_fixup_kernel, dim3((unsigned)nfix_, ng, sb),
-                         dim3(256), 0, stream, a, fix_.as<int4>(), scratch, sb);
+    if (lists_.nfix()) {
+      hipLaunchKernelGGL(spread_fixup_kernel,
+                         dim3((unsigned)lists_.nfix(), ng, sb), dim3(256), 0,
+                         stream, a, lists_.fix(), scratch, sb);
       TC_HIP(hipGetLastError());
     }
   };
   auto scratch_bytes = [&](int nb) {
     const int sb = group(nb);
-    return sizeof(float2) * (size_t)std::max(nslots_, 1) * cdiv(nb, sb) * sb *
+    return sizeof(float2) * (size_t)std::max(lists_.nslots(), 1) * cdiv(nb, sb) * sb *
            SP_T * SP_T;
   };
   if (!work_ready_) {
-    make_segments(stream);
-    const int ntiles = (int)counts_.size();
+    lists_.make_segments(spread_args().g, NUFFT_W, stream);
     // Points per work item: TOMOCAM_HIP_SPREAD_CHUNK (>= 64), else the
     // autotuner's choice for this geometry, else (tuning allowed) the
-    // fastest of the rule's choice, 512, 1024 and 2048 on this call's first
+    // fastest of the rule's choice and two others near it on this call's first
     // batch: best of two timed runs after a warm-up, the rule's choice kept
-    // unless another is >= 5 % faster.  The chunk sets the order in which a
+    // unless another is >= 5 % and >= 20 us faster (events and launches of
+    // small grids scatter by some microseconds).  The chunk sets the order in which a
     // tile's points are summed, so the wide margin keeps near-ties (2048 is
     // within 0.7-1.3 % of 1024 on large grids) on the rule's choice and the
     // results the same from process to process.  Each work item writes its
@@ -916,18 +650,22 @@ void PolarNufft::type1_real(const float2* c, float* out, int S, float scale,
       if (it != g_chunk_tuned.end()) chunk = it->second;
     }
     if (!chunk && autotune_enabled()) {
-      constexpr float kMargin = 0.05f;
+      constexpr float kMargin = 0.05f, kMarginMs = 0.02f;
       const int nb = std::min(B, S);
-      std::vector<int> cands{spread_chunk(ntiles)};
-      for (int k : {512, 1024, 2048})
-        if (k != cands[0]) cands.push_back(k);
+      const int rule = lists_.rule_chunk();
+      std::vector<int> cands{rule};
+      if (rule < 512)
+        cands.insert(cands.end(), {384 - rule, 512});  // 128 and 256, 512
+      else
+        for (int k : {512, 1024, 2048})
+          if (k != rule) cands.push_back(k);
       hipEvent_t e0, e1;
       TC_HIP(hipEventCreate(&e0));
       TC_HIP(hipEventCreate(&e1));
       float best_ms = 0.f;
       try {
         for (int k : cands) {
-          make_work(k);
+          lists_.make_work(k);
           DevBuf scr(scratch_bytes(nb));
           float ms = 0.f;
           for (int rep = 0; rep < 3; ++rep) {
@@ -944,7 +682,8 @@ void PolarNufft::type1_real(const float2* c, float* out, int S, float scale,
                          "[tomocam] spread tune %d angles x %d, grid %d, %d "
                          "slices: chunk %d: %.3f ms\n", P_, N_, nf_, nb, k,
                          (double)ms);
-          if (chunk == 0 || ms < (1.0f - kMargin) * best_ms) {
+          if (chunk == 0 ||
+              ms < std::min((1.0f - kMargin) * best_ms, best_ms - kMarginMs)) {
             chunk = k;
             best_ms = ms;
           }
@@ -959,8 +698,8 @@ void PolarNufft::type1_real(const float2* c, float* out, int S, float scale,
       std::lock_guard<std::mutex> lk(g_chunk_mu);
       g_chunk_tuned[key] = chunk;
     }
-    if (!chunk) chunk = spread_chunk(ntiles);
-    if (chunk != chunk_) make_work(chunk);
+    if (!chunk) chunk = lists_.rule_chunk();
+    if (chunk != lists_.chunk()) lists_.make_work(chunk);
     work_ready_ = true;
   }
   DevBuf scratch(scratch_bytes(B));
