@@ -5,6 +5,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <tuple>
 
 #include "fft_ops.h"
 #include "fft_rt.h"
@@ -126,6 +127,43 @@ const FFTLength& fft_length(int L) {
   if (it == cache.end())
     it = cache.emplace(key, std::make_unique<FFTLength>(L)).first;
   return *it->second;
+}
+
+const float2* fft_stage_twiddles(const std::vector<int>& a,
+                                 const std::vector<int>& b) {
+  using Key = std::tuple<int, std::vector<int>, std::vector<int>>;
+  static std::mutex mu;
+  static std::map<Key, std::unique_ptr<DevBuf>> cache;
+  int dev = 0;
+  TC_HIP(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lk(mu);
+  Key key(dev, a, b);
+  auto it = cache.find(key);
+  if (it == cache.end()) {
+    ArenaPause no_arena;  // process-lifetime table, filled synchronously
+    std::vector<float2> h;
+    for (const std::vector<int>* rs : {&a, &b}) {
+      long L = 1, Ns = 1;
+      for (int r : *rs) L *= r;
+      for (size_t s = 0; s < rs->size(); ++s) {
+        const int R = (*rs)[s];
+        const long step = L / (Ns * R);
+        if (s > 0)
+          for (int r = 1; r < R; ++r)
+            for (long k = 0; k < Ns; ++k) {
+              const double x = -2.0 * M_PI * (double)(k * r * step) / (double)L;
+              h.push_back(make_float2((float)std::cos(x), (float)std::sin(x)));
+            }
+        Ns *= R;
+      }
+    }
+    if (h.empty()) h.push_back(make_float2(1.f, 0.f));
+    auto buf = std::make_unique<DevBuf>(sizeof(float2) * h.size());
+    TC_HIP(hipMemcpy(buf->as<void>(), h.data(), sizeof(float2) * h.size(),
+                     hipMemcpyHostToDevice));
+    it = cache.emplace(std::move(key), std::move(buf)).first;
+  }
+  return it->second->as<float2>();
 }
 
 // bytes of LDS of lpw lines in two buffers

@@ -4,7 +4,8 @@
 // thread); T = L / E threads cooperate on one line.  In stage s (radix R,
 // Ns = R_1 ... R_{s-1}) thread t owns butterflies j = t + i T, i < E / R:
 //   inputs   x[j + r L/R]                           (r < R)
-//   twiddle  w_L^(r (j mod Ns) L/(Ns R))
+//   twiddle  w_L^(r (j mod Ns) L/(Ns R)), from the stage's table [r - 1][k]
+//            of (R - 1) Ns values (k = j mod Ns)
 //   outputs  y[(j - j mod Ns) R + (j mod Ns) + r Ns]
 // Each radix-R DFT (R up to 27, composite radices by Cooley-Tukey in
 // registers) runs entirely in registers; consecutive stages exchange data
@@ -15,6 +16,8 @@
 // stage-1 input set equal to the forward's last-stage output set, so a
 // forward-multiply-inverse sequence never leaves registers in between.
 #pragma once
+
+#include <atomic>
 
 #include "fft_device.h"
 
@@ -195,22 +198,39 @@ struct RadixList {
   }
 };
 
+// Where stage s's twiddles start in the plan's table, and its length.
+template <int... Rs>
+constexpr int stage_tw_offset(int s) {
+  int o = 0;
+  for (int i = 1; i < s; ++i)
+    o += (RadixList<Rs...>::at(i) - 1) * RadixList<Rs...>::ns(i);
+  return o;
+}
+
 // One stage's arithmetic on registers v[E] holding inputs v[i R + r] =
-// x[j + r L/R], j = t + i T; twiddle then DFT.
+// x[j + r L/R], j = t + i T; twiddle then DFT.  tw: the stage's table; for a
+// fixed r consecutive threads read consecutive values, at constant distances
+// from one offset.  (Read as w_L^m from one table of length L, a wave's loads
+// were 8 r step bytes apart, up to a cache line a lane: the twiddles then took
+// as much of the address unit's time as the arithmetic did of the vector
+// unit's.  With 32-bit offsets: Toeplitz column
+// pass of 8 x 1454^2 163 -> 141 us, 8 x 2188 lines of 4374 654 -> 593 us.)
 // ZIN (first stage only): inputs r >= R/2 of every butterfly are zero.
 template <int L, int T, int E, int R, int Ns, int DIR, bool ZIN = false>
 __device__ __forceinline__ void stage_compute(float2* v, int t,
                                               const float2* __restrict__ tw) {
   static_assert(!ZIN || Ns == 1, "zero inputs only in the first stage");
   constexpr int NB = E / R;
-  constexpr int step = L / (Ns * R);
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
     if (Ns > 1) {
-      const int k = (t + i * T) % Ns;
+      const unsigned k = (unsigned)((t + i * T) % Ns);
 #pragma unroll
       for (int r = 1; r < R; ++r) {
-        const float2 w = tw[k * r * step];
+        // scalar base and 32-bit offset
+        const float2 w = *reinterpret_cast<const float2*>(
+            reinterpret_cast<const char*>(tw + (r - 1) * Ns) +
+            k * (unsigned)sizeof(float2));
         v[i * R + r] = DIR < 0 ? cmul(v[i * R + r], w) : cmulc(v[i * R + r], w);
       }
     }
@@ -350,7 +370,9 @@ struct StagesDispatch {
         if (active) stage_read<L, T, E, R, Nsp, Rp>(v, line, t);
         __syncthreads();
       }
-      if (active) stage_compute<L, T, E, R, Ns, DIR, ZIN && s == 0>(v, t, tw);
+      if (active)
+        stage_compute<L, T, E, R, Ns, DIR, ZIN && s == 0>(
+            v, t, tw + stage_tw_offset<Rs...>(s));
       StagesDispatch<L, T, E, DIR, ZIN, s + 1, Rs...>::run(v, line, t, active,
                                                            tw);
     }
@@ -360,7 +382,8 @@ struct StagesDispatch {
 // Full transform on registers.  Before: v[i R1 + r] = x[t + i T + r L/R1].
 // After: v[i RS + r] = X[t + i T + r L/RS].  ZIN: the input is zero from
 // index L/2 on (a zero-padded line), so v[i R1 + r] for r >= R1/2 are zero
-// and are not read; needs an even R1 whose first factor is 2.
+// and are not read; needs an even R1 whose first factor is 2.  tw: the stage
+// tables of Rs, one after the other (plan_twiddles).
 template <int L, int E, int DIR, bool ZIN, int... Rs>
 __device__ __forceinline__ void transform(float2* v, float2* line, int t,
                                           bool active,
@@ -368,6 +391,31 @@ __device__ __forceinline__ void transform(float2* v, float2* line, int t,
   static_assert(plan_valid<L, E, Rs...>(), "invalid FFT plan");
   StagesDispatch<L, L / E, E, DIR, ZIN, 0, Rs...>::run(v, line, t, active,
                                                        tw);
+}
+
+// The stage tables of the radices Fwd, then those of Inv, in one buffer on the
+// current device (cached); the second ones start at tw_count<Fwd>.
+template <class Rad>
+struct TwCount;
+template <int... Rs>
+struct TwCount<Radices<Rs...>> {
+  static constexpr int value = stage_tw_offset<Rs...>((int)sizeof...(Rs));
+  static std::vector<int> radices() { return {Rs...}; }
+};
+template <class Rad>
+constexpr int tw_count = TwCount<Rad>::value;
+template <class Fwd, class Inv>
+const float2* plan_twiddles() {
+  constexpr int kDev = 64;
+  static std::atomic<const float2*> seen[kDev];
+  int dev = 0;
+  TC_HIP(hipGetDevice(&dev));
+  if (dev < kDev)
+    if (const float2* p = seen[dev].load(std::memory_order_acquire)) return p;
+  const float2* p =
+      fft_stage_twiddles(TwCount<Fwd>::radices(), TwCount<Inv>::radices());
+  if (dev < kDev) seen[dev].store(p, std::memory_order_release);
+  return p;
 }
 
 // index of register element (i, r) for a stage of radix R

@@ -257,4 +257,9 @@ class FFTLength {
 // Cache of FFTLength objects per (device, L); entries live until exit.
 const FFTLength& fft_length(int L);
 
+// Stage twiddles of the radices a, then of the radices b, of a compile-time
+// plan (fft_ct.h), cached per device; entries live until exit.
+const float2* fft_stage_twiddles(const std::vector<int>& a,
+                                 const std::vector<int>& b);
+
 }  // namespace tc

@@ -60,6 +60,7 @@ struct LinePlan {
   static constexpr int RS = RadixOps<Fwd>::last;
   static_assert(RadixOps<Inv>::first == RS && RadixOps<Inv>::last == R1,
                 "Inv must be Fwd reversed");
+  static const float2* twiddles() { return ct::plan_twiddles<Fwd, Inv>(); }
   template <int DIR>
   __device__ __forceinline__ static void run(float2* v, float2* line, int t,
                                              bool active,
@@ -69,7 +70,8 @@ struct LinePlan {
   __device__ __forceinline__ static void run_inv(float2* v, float2* line,
                                                  int t, bool active,
                                                  const float2* __restrict__ tw) {
-    RadixOps<Inv>::template run<L_, E_, 1>(v, line, t, active, tw);
+    RadixOps<Inv>::template run<L_, E_, 1>(v, line, t, active,
+                                           tw + ct::tw_count<Fwd>);
   }
 };
 
@@ -130,7 +132,7 @@ void launch_ct_lines(const LineFFTArgs& a, hipStream_t stream) {
   allow_lds((const void*)k, smem);
   const unsigned nblk = (unsigned)cdiv(nlines, P::LPW);
   hipLaunchKernelGGL(k, dim3(nblk), dim3(P::NT), smem, stream, a.in, a.out,
-                     fft_length(P::L).plan().tw, a.lines_per_batch, nlines,
+                     P::twiddles(), a.lines_per_batch, nlines,
                      a.bstride, a.lstride, a.estride, a.nin, a.nin_hi, a.nout,
                      a.nout_hi, a.scale);
   TC_HIP(hipGetLastError());
@@ -293,7 +295,7 @@ void run_real_rows(const RealRowsArgs& a, bool r2c, hipStream_t stream) {
   if (nlines == 0) return;
   const size_t smem = sizeof(float2) * (size_t)P::LPW * P::LS;
   const unsigned nblk = (unsigned)cdiv(nlines, P::LPW);
-  const float2* tw = fft_length(P::L).plan().tw;
+  const float2* tw = P::twiddles();
   auto k = r2c ? ct_r2c_rows_kernel<P> : ct_c2r_rows_kernel<P>;
   allow_lds((const void*)k, smem);
   hipLaunchKernelGGL(k, dim3(nblk), dim3(P::NT), smem, stream, a, tw);
@@ -477,7 +479,7 @@ void run_rays(const RayArgs& a, bool to_half, hipStream_t stream) {
   if (nlines == 0) return;
   const size_t smem = sizeof(float2) * (size_t)P::LPW * P::LS;
   const unsigned nblk = (unsigned)cdiv(nlines, P::LPW);
-  const float2* tw = fft_length(P::L).plan().tw;
+  const float2* tw = P::twiddles();
   auto k = a.N == a.L ? (to_half ? ct_ray_direct_kernel<P, true>
                                  : ct_ray_direct_kernel<P, false>)
                       : (to_half ? ct_ray_kernel<P, true>
@@ -495,6 +497,7 @@ struct LineOps {
   void (*lines)(const LineFFTArgs&, int dir, hipStream_t);
   void (*real_rows)(const RealRowsArgs&, bool r2c, hipStream_t);
   void (*rays)(const RayArgs&, bool to_half, hipStream_t);
+  const float2* (*twiddles)();
 };
 
 // Plans, ascending: length, elements per thread, lines per workgroup and
@@ -572,6 +575,6 @@ using L11664 = LinePlan<11664, 36, 1, Radices<36, 18, 18>, Radices<18, 18, 36>>;
 
 #define TC_LINE_OPS_DEF(LL)                                             \
   LineOps kLineOps##LL = {LL, run_lines<L##LL>, run_real_rows<L##LL>, \
-                                run_rays<L##LL>};
+                                run_rays<L##LL>, L##LL::twiddles};
 
 }  // namespace tc

@@ -21,6 +21,12 @@ int fft_lines_ct_length(int n) {
   return 0;
 }
 
+void fft_prepare(int L) {
+  const LineOps* o = fft_ct_enabled() ? find_ops(L) : nullptr;
+  if (o) o->twiddles();
+  else fft_length(L);
+}
+
 bool fft_lines_ct(const LineFFTArgs& a, int dir, hipStream_t stream) {
   const LineOps* o = find_ops(a.L);
   if (!o) return false;

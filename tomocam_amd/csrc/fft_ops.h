@@ -118,6 +118,9 @@ __device__ __forceinline__ void ray_store_pair(const RayArgs& a, long pair,
 // length >= n (0: none), and the transforms (false: no plan for the length).
 bool fft_lines_ct_has(int L);
 int fft_lines_ct_length(int n);
+// Lays out the twiddle tables of length L, so that no later call does (a first
+// transform may run under stream capture).
+void fft_prepare(int L);
 bool fft_lines_ct(const LineFFTArgs& a, int dir, hipStream_t stream);
 bool fft_real_rows_ct(const RealRowsArgs& a, bool r2c, hipStream_t stream);
 bool fft_rays_ct(const RayArgs& a, bool to_half, hipStream_t stream);

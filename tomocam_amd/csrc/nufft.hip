@@ -529,6 +529,7 @@ PolarNufft::PolarNufft(const float* h_angles, int nproj, int npix, int nmodes)
     if (k & 1) c = -c;
     corr[ki] = (float)c;
   }
+  fft_prepare(nf_);
   corr_.alloc(sizeof(float) * nm_);
   TC_HIP(hipMemcpy(corr_.as<void>(), corr.data(), sizeof(float) * nm_,
                    hipMemcpyHostToDevice));
@@ -786,6 +787,7 @@ RayDft::RayDft(int N, int sign) : N_(N) {
   ArenaPause no_arena;  // cached plan, tables filled synchronously
   TC_REQUIRE(N >= 1, "ray DFT: N must be >= 1");
   direct_ = fft_lines_ct_has(N);
+  if (direct_) fft_prepare(N);
   // The chirp-z length: a planned FFT length where there is one (the planned
   // kernel runs forward transform, multiply and inverse in registers)
   if (sign < 0) {

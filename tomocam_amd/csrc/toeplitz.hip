@@ -25,6 +25,7 @@ extern const int kToeplitzCtSizes[];
 extern const float kToeplitzCtCost[];
 extern const int kToeplitzCtCount;
 int toeplitz_plain_length(int m);
+bool toeplitz_ct_prepare(int M);
 bool toeplitz_ct_mixed(int M);
 
 // Compile-time plan sizes eligible for an n x n Toeplitz product: >= 2n - 1
@@ -127,6 +128,10 @@ Psf::Psf(const float* d_psf, int n, hipStream_t stream) : n_(n) {
 void Psf::build_spectrum(int M, hipStream_t stream) {
   M_ = M;
   H_ = M_ / 2 + 1;
+  {
+    ArenaPause no_arena;  // process-lifetime tables
+    if (!toeplitz_ct_prepare(M_)) fft_length(M_);
+  }
   // everything sized by the FFT length starts over
   spec16_.release();
   spec16_exp_ = 0;

@@ -74,6 +74,8 @@ struct TPlan {
   static constexpr bool ZA = ZA_;
   using Fwd = Fwd_;
   using Inv = Inv_;
+  static constexpr int TWI = ct::tw_count<Fwd_>;  // the inverse's twiddles
+  static const float2* twiddles() { return ct::plan_twiddles<Fwd_, Inv_>(); }
   // LDS elements per line (padded exchanges) and line strides of the row
   // passes (LS) and the column pass (LSC)
   static constexpr int LE = LineElems<L_, Fwd_>::value > LineElems<L_, Inv_>::value
@@ -105,8 +107,24 @@ __device__ __forceinline__ int col_scale_index(int s, int k1, int row, int H) {
 // pass reads whole columns.  (A row-group-major layout, which makes the row
 // passes stream contiguously, measured slower overall: the column pass loses
 // more than the row passes gain.)
-__device__ __forceinline__ long wt_at(int s, int k1, int row, int H, int rp) {
-  return ((long)s * H + k1) * rp + row;
+//
+// Every access of the passes is a slice's base (the same for the whole
+// workgroup, in scalar registers) plus a 32-bit byte offset: as 64-bit
+// addresses per lane the offsets took a fifth of the passes' vector
+// instructions.
+__device__ __forceinline__ unsigned wt_at(int k1, int row, int rp) {
+  return (unsigned)k1 * (unsigned)rp + (unsigned)row;
+}
+// element i of a uniform base
+template <typename T>
+__device__ __forceinline__ T& at32(T* base, unsigned i) {
+  return *reinterpret_cast<T*>(reinterpret_cast<char*>(base) +
+                               i * (unsigned)sizeof(T));
+}
+template <typename T>
+__device__ __forceinline__ const T& at32(const T* base, unsigned i) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) +
+                                     i * (unsigned)sizeof(T));
 }
 
 // Line-search commit fused into passes A and C (CM = 0: none; 1: y = sol;
@@ -166,10 +184,16 @@ ct_rows_fwd(const void* __restrict__ xv, void* __restrict__ wtv,
   // wait out each load's latency in turn.
   float2 v[E];
   float2 y[CM != 0 ? E : 1];
-  const long oa = (long)s * n * n + (long)ra * n;
+  const long plane = (long)s * n * n;
+  const unsigned oa = (unsigned)ra * (unsigned)n;
+  const float* xp = reinterpret_cast<const float*>(xv) + plane;
+  const float* solp = CM != 0 ? cp.sol + plane : nullptr;
+  const float* xpp = CM == 2 ? cp.xp + plane : nullptr;
+  float* dstp = CM != 0 ? cp.dst + plane : nullptr;
   // FP16 input: the row-pair layout, rows ra and ra + 1 in one word
   const unsigned* xw = reinterpret_cast<const unsigned*>(xv) +
-                       ((long)s * ((n + 1) / 2) + ra / 2) * n;
+                       (long)s * ((n + 1) / 2) * n;
+  const unsigned ow = (unsigned)(ra / 2) * (unsigned)n;
   static_assert(R1 % 2 == 0, "plans need an even first radix");
 #pragma unroll
   for (int i = 0; i < E / R1; ++i)
@@ -183,21 +207,21 @@ ct_rows_fwd(const void* __restrict__ xv, void* __restrict__ wtv,
           // the raw word (second half 0 past the last row), unpacked only
           // once every load is issued: an unpack next to its load makes
           // each load wait out its latency in turn
-          if (hasa) re = __uint_as_float(xw[c]);
+          if (hasa) re = __uint_as_float(at32(xw, ow + c));
         } else {
-          if (hasa) re = reinterpret_cast<const float*>(xv)[oa + c];
-          if (hasb) im = reinterpret_cast<const float*>(xv)[oa + n + c];
+          if (hasa) re = at32(xp, oa + c);
+          if (hasb) im = at32(xp, oa + n + c);
         }
         if constexpr (CM != 0) {
           float ya = 0.f, yb = 0.f;
           if (hasa) {
-            ya = cp.sol[oa + c];
-            if constexpr (CM == 2) ya = fmaf(cp.beta, ya - cp.xp[oa + c], ya);
+            ya = at32(solp, oa + c);
+            if constexpr (CM == 2) ya = fmaf(cp.beta, ya - at32(xpp, oa + c), ya);
           }
           if (hasb) {
-            yb = cp.sol[oa + n + c];
+            yb = at32(solp, oa + n + c);
             if constexpr (CM == 2)
-              yb = fmaf(cp.beta, yb - cp.xp[oa + n + c], yb);
+              yb = fmaf(cp.beta, yb - at32(xpp, oa + n + c), yb);
           }
           y[e] = make_float2(ya, yb);
         }
@@ -218,8 +242,8 @@ ct_rows_fwd(const void* __restrict__ xv, void* __restrict__ wtv,
         const int c = t + i * T + r * (L / R1);
         const int e = i * R1 + r;
         if (c < n) {
-          if (hasa) cp.dst[oa + c] = fmaf(-se, v[e].x, y[e].x);
-          if (hasb) cp.dst[oa + n + c] = fmaf(-se, v[e].y, y[e].y);
+          if (hasa) at32(dstp, oa + c) = fmaf(-se, v[e].x, y[e].x);
+          if (hasb) at32(dstp, oa + n + c) = fmaf(-se, v[e].y, y[e].y);
         }
       }
   }
@@ -232,6 +256,7 @@ ct_rows_fwd(const void* __restrict__ xv, void* __restrict__ wtv,
   __syncthreads();
   constexpr bool W16 = (HM & HM_WT16) != 0;
   const float hw = W16 ? 0.5f * ha.wsc : 0.5f;
+  const long ws = (long)s * H * rp;  // (H rp and rows rr are even)
   for (int q = threadIdx.x; q < LPW * H; q += P::NT) {
     const int k = q / LPW;
     const int l = q - k * LPW;
@@ -242,13 +267,13 @@ ct_rows_fwd(const void* __restrict__ xv, void* __restrict__ wtv,
       const float2 sp = cadd(zk, zm), df = csub(zk, zm);
       if constexpr (W16) {
         // |value| <= n * 2^16 * wsc <= 2^15: no overflow
-        *reinterpret_cast<uint2*>(reinterpret_cast<unsigned*>(wtv) +
-                                  wt_at(s, k, rr, H, rp)) =
+        at32(reinterpret_cast<uint2*>(reinterpret_cast<unsigned*>(wtv) + ws),
+             wt_at(k, rr, rp) / 2) =
             make_uint2(pack_half2(hw * sp.x, hw * sp.y),
                        pack_half2(hw * df.y, -hw * df.x));
       } else {
-        *reinterpret_cast<float4*>(reinterpret_cast<float2*>(wtv) +
-                                   wt_at(s, k, rr, H, rp)) =
+        at32(reinterpret_cast<float4*>(reinterpret_cast<float2*>(wtv) + ws),
+             wt_at(k, rr, rp) / 2) =
             make_float4(hw * sp.x, hw * sp.y, hw * df.y, -hw * df.x);
       }
     }
@@ -285,6 +310,7 @@ ct_cols(void* __restrict__ wtv, const void* __restrict__ specv,
   // are inactive
   const bool active = line < LPW && k1 < H;
   const int kc = active ? k1 : 0;
+  const long ws = (long)s * H * rp;
   // the slice's FP16 input scale (for the dot), fetched up front
   const float gsc_s = (HM & HM_IN16) ? ha.gsc[s] : 1.0f;
   float2 v[E];
@@ -295,12 +321,13 @@ ct_cols(void* __restrict__ wtv, const void* __restrict__ specv,
       const int idx = t + i * T + r * (L / R1);
       float2 w = make_float2(0.f, 0.f);
       if (r < R1 / 2 && active && idx < n) {
-        const long o = wt_at(s, kc, idx, H, rp);
+        const unsigned o = wt_at(kc, idx, rp);
         // FP16: the raw word, unpacked once every load is issued
         if constexpr ((HM & HM_WT16) != 0)
-          w.x = __uint_as_float(reinterpret_cast<const unsigned*>(wtv)[o]);
+          w.x = __uint_as_float(
+              at32(reinterpret_cast<const unsigned*>(wtv) + ws, o));
         else
-          w = reinterpret_cast<const float2*>(wtv)[o];
+          w = at32(reinterpret_cast<const float2*>(wtv) + ws, o);
       }
       v[i * R1 + r] = w;
     }
@@ -316,21 +343,21 @@ ct_cols(void* __restrict__ wtv, const void* __restrict__ specv,
   float hs[S16 ? 1 : E];
   __half2 hs2[S16 ? (E + 1) / 2 : 1];
   {
-    const long so = (long)kc * L;
+    const unsigned so = (unsigned)kc * (unsigned)L;
 #pragma unroll
     for (int i = 0; i < E / RS; ++i)
 #pragma unroll
       for (int r = 0; r < RS; ++r) {
         const int e = i * RS + r;
-        const long o = so + t + i * T + r * (L / RS);
+        const unsigned o = so + t + i * T + r * (L / RS);
         if constexpr (S16) {
-          const __half h = reinterpret_cast<const __half*>(specv)[o];
+          const __half h = at32(reinterpret_cast<const __half*>(specv), o);
           if (e & 1)
             hs2[e / 2].y = h;
           else
             hs2[e / 2].x = h;
         } else {
-          hs[e] = reinterpret_cast<const float*>(specv)[o];
+          hs[e] = at32(reinterpret_cast<const float*>(specv), o);
         }
       }
   }
@@ -357,7 +384,7 @@ ct_cols(void* __restrict__ wtv, const void* __restrict__ specv,
     acc = (double)(wgt * facc);
   }
   // the inverse's first stage needs no exchange (same element set)
-  I::run(v, ln, t, active, tw);
+  I::run(v, ln, t, active, tw + P::TWI);
   if constexpr ((HM & HM_WT16) != 0) {
     // Power-of-two scale per 32 consecutive threads (a half wave): their
     // largest kept value maps below 2^14.  A shuffle reduction within the
@@ -391,7 +418,7 @@ ct_cols(void* __restrict__ wtv, const void* __restrict__ specv,
         for (int r = 0; r < R1 / 2; ++r) {
           const int idx = t + i * T + r * (L / R1);
           if (idx < n)
-            reinterpret_cast<unsigned*>(wtv)[wt_at(s, kc, idx, H, rp)] =
+            at32(reinterpret_cast<unsigned*>(wtv) + ws, wt_at(kc, idx, rp)) =
                 pack_half2(kap * v[i * R1 + r].x, kap * v[i * R1 + r].y);
         }
     }
@@ -406,7 +433,7 @@ ct_cols(void* __restrict__ wtv, const void* __restrict__ specv,
       for (int r = 0; r < R1 / 2; ++r) {
         const int idx = t + i * T + r * (L / R1);
         if (idx < n)
-          reinterpret_cast<float2*>(wtv)[wt_at(s, kc, idx, H, rp)] =
+          at32(reinterpret_cast<float2*>(wtv) + ws, wt_at(kc, idx, rp)) =
               v[i * R1 + r];
       }
   }
@@ -445,6 +472,7 @@ ct_rows_inv(const void* __restrict__ wtv, const float* bvec, float* out,
   // the transform instead of delaying the epilogue
   const float gsc_s = (HM & HM_IN16) ? ha.gsc[s] : 1.0f;
   // every Wt load of the thread in flight at once, then the LDS writes
+  const long ws = (long)s * H * rp;
   constexpr int HC = L / 2 + 1;
   constexpr int NQ = (LPW * HC + P::NT - 1) / P::NT;
   float4 w4[NQ];
@@ -463,18 +491,18 @@ ct_rows_inv(const void* __restrict__ wtv, const float* bvec, float* out,
       u16[j] = make_uint2(0u, 0u);
     }
     if (q < LPW * H && rr < rp) {
-      const long o = wt_at(s, k, rr, H, rp);
+      const unsigned o = wt_at(k, rr, rp) / 2;
       if constexpr (W16) {
-        u16[j] = *reinterpret_cast<const uint2*>(
-            reinterpret_cast<const unsigned*>(wtv) + o);
+        u16[j] = at32(reinterpret_cast<const uint2*>(
+                          reinterpret_cast<const unsigned*>(wtv) + ws), o);
         // rows rr and rr + 1 may lie in different scale groups (odd T)
         const int i0 = col_scale_index<P>(s, k, rr, H);
         const int i1 = col_scale_index<P>(s, k, rr + 1, H);
         cs[j] = ha.cinv[i0];
         cs1[j] = i1 == i0 ? cs[j] : ha.cinv[i1];
       } else {
-        w4[j] = *reinterpret_cast<const float4*>(
-            reinterpret_cast<const float2*>(wtv) + o);
+        w4[j] = at32(reinterpret_cast<const float4*>(
+                         reinterpret_cast<const float2*>(wtv) + ws), o);
       }
     }
   }
@@ -515,9 +543,11 @@ ct_rows_inv(const void* __restrict__ wtv, const float* bvec, float* out,
 #pragma unroll
     for (int r = 0; r < R1; ++r) v[i * R1 + r] = ln[t + i * T + r * (L / R1)];
   __syncthreads();
-  I::run(v, ln, t, true, tw);
+  I::run(v, ln, t, true, tw + P::TWI);
   const int ra = r0 + 2 * line;
-  const long oa = (long)s * n * n + (long)ra * n;
+  const long plane = (long)s * n * n;
+  const unsigned oa = (unsigned)ra * (unsigned)n;
+  float* outp = out + plane;
   const bool hasa = ra < n, hasb = ra + 1 < n;
   // FP16 input: the transform is in units of gsc times the true values;
   // an FP16 spectrum with FP32 intermediates leaves its 2^e scale here
@@ -538,18 +568,19 @@ ct_rows_inv(const void* __restrict__ wtv, const float* bvec, float* out,
   for (int h = 0; h < NB; ++h) {
     float2 e0[MODE != 0 ? EB : 1], e1[MODE == 3 ? EB : 1];
     if constexpr (MODE != 0) {
-      const float* src0 = MODE == 1 ? bvec : cp.Tsol;
+      const float* src0 = (MODE == 1 ? bvec : cp.Tsol) + plane;
+      const float* src1 = MODE == 3 ? cp.Tx + plane : nullptr;
 #pragma unroll
       for (int j = 0; j < EB; ++j) {
         const int e = h * EB + j, i = e / RS, r = e - i * RS;
         const int c = t + i * T + r * (L / RS);
         float2 p0 = make_float2(0.f, 0.f), p1 = p0;
         if (r < RS / 2 && c < n) {
-          if (hasa) p0.x = src0[oa + c];
-          if (hasb) p0.y = src0[oa + n + c];
+          if (hasa) p0.x = at32(src0, oa + c);
+          if (hasb) p0.y = at32(src0, oa + n + c);
           if constexpr (MODE == 3) {
-            if (hasa) p1.x = cp.Tx[oa + c];
-            if (hasb) p1.y = cp.Tx[oa + n + c];
+            if (hasa) p1.x = at32(src1, oa + c);
+            if (hasb) p1.y = at32(src1, oa + n + c);
           }
         }
         e0[j] = p0;
@@ -580,8 +611,8 @@ ct_rows_inv(const void* __restrict__ wtv, const float* bvec, float* out,
           o.x = fmaf(-se, q.x, ty.x);
           o.y = fmaf(-se, q.y, ty.y);
         }
-        if (hasa) out[oa + c] = o.x;
-        if (hasb) out[oa + n + c] = o.y;
+        if (hasa) at32(outp, oa + c) = o.x;
+        if (hasb) at32(outp, oa + n + c) = o.y;
       }
     }
   }
@@ -594,7 +625,7 @@ static void run_ct(const void* x, const float* b, float* out, void* wt,
                    double img_b, double spec_b, const Psf::StepCommit* sc,
                    const ToeplitzHalf* half, const ToeplitzStreams* ts,
                    int group_cap) {
-  const float2* tw = fft_length(P::L).plan().tw;
+  const float2* tw = P::twiddles();
   // kernel-timer classes: the FP16-storage passes are timed apart
   constexpr bool H16 = HM != 0;  // any FP16 storage: timed apart
   constexpr bool W16 = (HM & HM_WT16) != 0;
@@ -706,6 +737,7 @@ static void run_ct(const void* x, const float* b, float* out, void* wt,
 // (Psf::apply's arguments).
 struct ToeplitzPlainOps {
   int M, lpwc;
+  const float2* (*twiddles)();
   void (*run)(const float* x, const float* b, float* out, float2* wt,
               const float* spec, int n, int H, int rp, int nslices, int mode,
               double* partials, hipStream_t stream, double img_b,
@@ -786,6 +818,7 @@ using PlainPlan8192 = TPlan<8192, 32, 1, Radices<32, 16, 16>,
 
 #define TC_TOEPLITZ_PLAIN_DEF(LL)                                  \
   ToeplitzPlainOps kToeplitzPlain##LL = {LL, PlainPlan##LL::LPWC,  \
+                                         PlainPlan##LL::twiddles,       \
                                          run_plain<PlainPlan##LL>};
 
 }  // namespace tc

@@ -172,6 +172,26 @@ int toeplitz_ct_lpw(int M) {
   }
 }
 
+// Lays out the twiddle tables of M's plan; false: no compile-time plan.
+bool toeplitz_ct_prepare(int M) {
+  switch (M) {
+    case 750: Plan750::twiddles(); return true;
+    case 1458: Plan1458::twiddles(); return true;
+    case 2250: Plan2250::twiddles(); return true;
+    case 2916: Plan2916::twiddles(); return true;
+    case 4500: Plan4500::twiddles(); return true;
+    case 4608: Plan4608::twiddles(); return true;
+    case 2304: Plan2304::twiddles(); return true;
+    case 768: Plan768::twiddles(); return true;
+    case 5832: Plan5832::twiddles(); return true;
+    default: {
+      const ToeplitzPlainOps* o = find_plain(M);
+      if (o) o->twiddles();
+      return o != nullptr;
+    }
+  }
+}
+
 // whether M has the mixed-precision forms
 bool toeplitz_ct_mixed(int M) {
   for (int i = 0; i < kToeplitzCtCount; ++i)
