@@ -193,18 +193,20 @@ RtLaunch rt_launch(int L, long nlines, int want) {
   return l;
 }
 
-// Line l of batch b starts at b*bstride + l*lstride, element i at + i*estride
+// Line l of batch b starts at b*bstride + (l/lgroup)*lstride + l%lgroup,
+// element i at + i*estride
 // (complex elements).  Of a line, the elements [0, nin) and [L - nin_hi, L)
 // are read (the others are zero) and [0, nout) and [L - nout_hi, L) written.
 struct LinesMap {
-  int lines_per_batch, nin, nin_hi, nout, nout_hi, colmajor;
+  int lines_per_batch, nin, nin_hi, nout, nout_hi, colmajor, lgroup;
   long total, bstride, lstride, estride;
   float scale;
 };
 
 __device__ __forceinline__ long line_base(const LinesMap& m, long gl) {
   const long b = gl / m.lines_per_batch;
-  return b * m.bstride + (gl - b * m.lines_per_batch) * m.lstride;
+  const int l = (int)(gl - b * m.lines_per_batch);
+  return b * m.bstride + (l / m.lgroup) * m.lstride + l % m.lgroup;
 }
 
 template <int DIR>
@@ -259,7 +261,8 @@ fft_lines_kernel(const float2* __restrict__ in, float2* __restrict__ out,
 template <int DIR>
 static void launch_lines(const LineFFTArgs& a, hipStream_t stream) {
   LinesMap m{a.lines_per_batch, a.nin,     a.nin_hi,  a.nout,
-             a.nout_hi,         a.colmajor, (long)a.lines_per_batch * a.nbatch,
+             a.nout_hi,         a.colmajor, a.lgroup,
+             (long)a.lines_per_batch * a.nbatch,
              a.bstride,         a.lstride, a.estride, a.scale};
   if (m.total == 0) return;
   if (rt_fits(a.L)) {
@@ -325,10 +328,11 @@ rt_r2c_rows_kernel(RealRowsArgs a, RtPlan P, int lpw) {
   }
   __syncthreads();
   const float2* z = rt_fft<-1>(sm, lpw, P, tid, nthr);
-  for (int q = tid; q < lpw * H; q += nthr) {
-    const int l = q / H, k = q - l * H;
+  for (int q = tid; q < lpw * ((H + HG_B - 1) / HG_B * HG_B); q += nthr) {
+    const int kb = q / (HG_B * lpw), l = q / HG_B - kb * lpw;
+    const int k = kb * HG_B + q % HG_B;
     const long gl = g0 + l;
-    if (gl >= nlines) break;
+    if (k >= H || gl >= nlines) continue;
     const long s = gl / npair;
     const int ka = 2 * (int)(gl - s * npair);
     const float2 zk = z[l * P.ldl + rt_pad(k)];
@@ -336,10 +340,10 @@ rt_r2c_rows_kernel(RealRowsArgs a, RtPlan P, int lpw) {
     const float2 sp = cadd(zk, zm), df = csub(zk, zm);
     const int ra = ka < hi ? L + ka - hi : ka - hi;
     const int rb = ka + 1 < hi ? L + ka + 1 - hi : ka + 1 - hi;
-    a.half[(s * L + ra) * a.pitch + k] = make_float2(0.5f * sp.x, 0.5f * sp.y);
+    float2* half = a.half + s * half_grid_size(L);
+    half[half_at(L, ra, k)] = make_float2(0.5f * sp.x, 0.5f * sp.y);
     if (ka + 1 < a.nm)
-      a.half[(s * L + rb) * a.pitch + k] =
-          make_float2(0.5f * df.y, -0.5f * df.x);
+      half[half_at(L, rb, k)] = make_float2(0.5f * df.y, -0.5f * df.x);
   }
 }
 
@@ -349,8 +353,10 @@ rt_c2r_rows_kernel(RealRowsArgs a, RtPlan P, int lpw) {
   const int tid = threadIdx.x, nthr = blockDim.x, L = P.L, H = L / 2 + 1;
   const int npair = (a.nm + 1) / 2, hi = a.nm / 2;
   const long g0 = (long)blockIdx.x * lpw, nlines = (long)a.nsl * npair;
-  for (int q = tid; q < lpw * H; q += nthr) {
-    const int l = q / H, k = q - l * H;
+  for (int q = tid; q < lpw * ((H + HG_B - 1) / HG_B * HG_B); q += nthr) {
+    const int kb = q / (HG_B * lpw), l = q / HG_B - kb * lpw;
+    const int k = kb * HG_B + q % HG_B;
+    if (k >= H) continue;
     const long gl = g0 + l;
     float2 x = make_float2(0.f, 0.f), y = x;
     if (gl < nlines) {
@@ -358,8 +364,9 @@ rt_c2r_rows_kernel(RealRowsArgs a, RtPlan P, int lpw) {
       const int ka = 2 * (int)(gl - s * npair);
       const int ra = ka < hi ? L + ka - hi : ka - hi;
       const int rb = ka + 1 < hi ? L + ka + 1 - hi : ka + 1 - hi;
-      x = a.half[(s * L + ra) * a.pitch + k];
-      if (ka + 1 < a.nm) y = a.half[(s * L + rb) * a.pitch + k];
+      const float2* half = a.half + s * half_grid_size(L);
+      x = half[half_at(L, ra, k)];
+      if (ka + 1 < a.nm) y = half[half_at(L, rb, k)];
       if (k == 0 || 2 * k == L) x.y = y.y = 0.f;  // real by symmetry
     }
     sm[l * P.ldl + rt_pad(k)] = make_float2(x.x - y.y, x.y + y.x);
@@ -471,9 +478,9 @@ __global__ void long_rows_pack_kernel(RealRowsArgs a, float2* z, int r2c) {
     const int k = low ? i : a.L - i;
     const int ra = ka < hi ? a.L + ka - hi : ka - hi;
     const int rb = ka + 1 < hi ? a.L + ka + 1 - hi : ka + 1 - hi;
-    float2 x = a.half[(s * a.L + ra) * a.pitch + k];
-    float2 y = hasb ? a.half[(s * a.L + rb) * a.pitch + k]
-                    : make_float2(0.f, 0.f);
+    const float2* half = a.half + s * half_grid_size(a.L);
+    float2 x = half[half_at(a.L, ra, k)];
+    float2 y = hasb ? half[half_at(a.L, rb, k)] : make_float2(0.f, 0.f);
     if (k == 0 || 2 * k == a.L) x.y = y.y = 0.f;
     w = low ? make_float2(x.x - y.y, x.y + y.x)
             : make_float2(x.x + y.y, y.x - x.y);
@@ -498,11 +505,10 @@ __global__ void long_rows_unpack_kernel(RealRowsArgs a, const float2* z,
     const float2 sp = cadd(zk, zm), df = csub(zk, zm);
     const int ra = ka < hi ? a.L + ka - hi : ka - hi;
     const int rb = ka + 1 < hi ? a.L + ka + 1 - hi : ka + 1 - hi;
-    a.half[(s * a.L + ra) * a.pitch + k] =
-        make_float2(0.5f * sp.x, 0.5f * sp.y);
+    float2* half = a.half + s * half_grid_size(a.L);
+    half[half_at(a.L, ra, k)] = make_float2(0.5f * sp.x, 0.5f * sp.y);
     if (hasb)
-      a.half[(s * a.L + rb) * a.pitch + k] =
-          make_float2(0.5f * df.y, -0.5f * df.x);
+      half[half_at(a.L, rb, k)] = make_float2(0.5f * df.y, -0.5f * df.x);
   } else {
     const float2 v = z[k < hi ? a.L + k - hi : k - hi];
     const float c = a.corr[k];
@@ -591,7 +597,7 @@ static void long_rows(RealRowsArgs a, bool r2c, hipStream_t stream) {
     TC_HIP(hipGetLastError());
     if (r2c) a.real_in += (long)a.nm * a.nm;
     else a.real_out += (long)a.nm * a.nm;
-    a.half += (long)a.L * a.pitch;
+    a.half += half_grid_size(a.L);
   }
 }
 
@@ -624,8 +630,7 @@ static void long_rays(RayArgs a, bool to_half, hipStream_t stream) {
 }
 
 void fft_real_rows(const RealRowsArgs& a, bool r2c, hipStream_t stream) {
-  TC_REQUIRE(a.nm >= 1 && a.nm <= a.L && a.L % 2 == 0 &&
-                 a.pitch >= a.L / 2 + 1,
+  TC_REQUIRE(a.nm >= 1 && a.nm <= a.L && a.L % 2 == 0,
              "fft_real_rows: bad shape");
   if (fft_ct_enabled() && fft_real_rows_ct(a, r2c, stream)) return;
   const long nlines = (long)a.nsl * ((a.nm + 1) / 2);

@@ -75,8 +75,8 @@ struct LinePlan {
   }
 };
 
-// Line l of batch b starts at b * bstride + l * lstride; element i at
-// + i * estride.  Of a line, the elements [0, nin) and [L - nin_hi, L) are
+// Line l of batch b starts at b * bstride + (l / lgroup) * lstride +
+// l % lgroup; element i at + i * estride.  Of a line, the elements [0, nin) and [L - nin_hi, L) are
 // read (the others are zero) and [0, nout) and [L - nout_hi, L) written.
 // COL: the workgroup's lines are adjacent columns, so consecutive threads
 // take consecutive lines (coalesced loads of a row); otherwise consecutive
@@ -85,7 +85,7 @@ template <class P, int DIR, bool COL>
 __global__ void __launch_bounds__(P::NT)
 ct_lines_kernel(const float2* in, float2* out, const float2* __restrict__ tw,
                 int lines_per_batch, long nlines, long bstride, long lstride,
-                long estride, int nin, int nin_hi, int nout, int nout_hi,
+                int lgroup, long estride, int nin, int nin_hi, int nout, int nout_hi,
                 float scale) {
   extern __shared__ float2 sm[];
   constexpr int L = P::L, E = P::E, T = P::T, LPW = P::LPW;
@@ -95,8 +95,8 @@ ct_lines_kernel(const float2* in, float2* out, const float2* __restrict__ tw,
   const long gl = (long)xcd_remap(blockIdx.x, gridDim.x) * LPW + line;
   const bool active = gl < nlines;
   const long b = active ? gl / lines_per_batch : 0;
-  const long base = active ? b * bstride + (gl - b * lines_per_batch) * lstride
-                           : 0;
+  const int lb = active ? (int)(gl - b * lines_per_batch) : 0;
+  const long base = b * bstride + (lb / lgroup) * lstride + lb % lgroup;
   float2 v[E];
 #pragma unroll
   for (int i = 0; i < E / R1; ++i)
@@ -133,7 +133,7 @@ void launch_ct_lines(const LineFFTArgs& a, hipStream_t stream) {
   const unsigned nblk = (unsigned)cdiv(nlines, P::LPW);
   hipLaunchKernelGGL(k, dim3(nblk), dim3(P::NT), smem, stream, a.in, a.out,
                      P::twiddles(), a.lines_per_batch, nlines,
-                     a.bstride, a.lstride, a.estride, a.nin, a.nin_hi, a.nout,
+                     a.bstride, a.lstride, a.lgroup, a.estride, a.nin, a.nin_hi, a.nout,
                      a.nout_hi, a.scale);
   TC_HIP(hipGetLastError());
 }
@@ -199,21 +199,36 @@ ct_r2c_rows_kernel(RealRowsArgs a, const float2* __restrict__ tw) {
       for (int r = 0; r < RS; ++r) ln[t + i * T + r * (L / RS)] = v[i * RS + r];
   }
   __syncthreads();
-  for (int q = threadIdx.x; q < LPW * H; q += P::NT) {
-    const int l = q / H, k = q - (q / H) * H;
+  // two columns of both rows a thread: 16-byte stores, consecutive threads
+  // along a block's columns, then along the workgroup's row pairs
+  constexpr int HC = HG_B / 2, NC = (H + HG_B - 1) / HG_B * HC;
+  for (int q = threadIdx.x; q < LPW * NC; q += P::NT) {
+    const int l = q / HC % LPW;
+    const int k = (q / (HC * LPW) * HC + q % HC) * 2;
     const long gl = g0 + l;
-    if (gl >= nlines) break;
+    if (k >= H || gl >= nlines) continue;
     const long s = gl / npair;
     const int ka = 2 * (int)(gl - s * npair);
-    const float2 zk = sm[l * P::LS + k];
-    const float2 zm = cconj(sm[l * P::LS + (k == 0 ? 0 : L - k)]);
-    const float2 sp = cadd(zk, zm), df = csub(zk, zm);
     const int ra = ka < hi ? L + ka - hi : ka - hi;
     const int rb = ka + 1 < hi ? L + ka + 1 - hi : ka + 1 - hi;
-    a.half[(s * L + ra) * a.pitch + k] = make_float2(0.5f * sp.x, 0.5f * sp.y);
-    if (ka + 1 < a.nm)
-      a.half[(s * L + rb) * a.pitch + k] =
-          make_float2(0.5f * df.y, -0.5f * df.x);
+    float4 fa, fb;  // column H, if any, is in the block's padding
+    {
+      const float2 zk = sm[l * P::LS + k];
+      const float2 zm = cconj(sm[l * P::LS + (k == 0 ? 0 : L - k)]);
+      const float2 sp = cadd(zk, zm), df = csub(zk, zm);
+      fa.x = 0.5f * sp.x, fa.y = 0.5f * sp.y;
+      fb.x = 0.5f * df.y, fb.y = -0.5f * df.x;
+    }
+    {
+      const float2 zk = sm[l * P::LS + k + 1];
+      const float2 zm = cconj(sm[l * P::LS + L - k - 1]);
+      const float2 sp = cadd(zk, zm), df = csub(zk, zm);
+      fa.z = 0.5f * sp.x, fa.w = 0.5f * sp.y;
+      fb.z = 0.5f * df.y, fb.w = -0.5f * df.x;
+    }
+    float2* half = a.half + s * half_grid_size(L);
+    *reinterpret_cast<float4*>(half + half_at(L, ra, k)) = fa;
+    if (ka + 1 < a.nm) *reinterpret_cast<float4*>(half + half_at(L, rb, k)) = fb;
   }
 }
 
@@ -227,30 +242,43 @@ ct_c2r_rows_kernel(RealRowsArgs a, const float2* __restrict__ tw) {
   const long g0 = (long)xcd_remap(blockIdx.x, gridDim.x) * LPW;
   const long nlines = (long)a.nsl * npair;
   const int lo = (a.nm + 1) / 2, hi = a.nm / 2;
-  // every load of the thread in flight at once, then the LDS writes
-  constexpr int NQ = (LPW * H + P::NT - 1) / P::NT;
-  float2 wa[NQ], wb[NQ];
+  // two columns of both rows a thread, consecutive threads along a block's
+  // columns, then along the workgroup's row pairs; every load of the thread in
+  // flight at once, then the LDS writes
+  constexpr int HC = HG_B / 2, NC = (H + HG_B - 1) / HG_B * HC;
+  constexpr int NQ = (LPW * NC + P::NT - 1) / P::NT;
+  float4 wa[NQ], wb[NQ];
 #pragma unroll
   for (int j = 0; j < NQ; ++j) {
     const int q = (int)threadIdx.x + j * P::NT;
-    const int l = q / H, k = q - (q / H) * H;
+    const int l = q / HC % LPW;
+    const int k = (q / (HC * LPW) * HC + q % HC) * 2;
     const long gl = g0 + l;
-    wa[j] = wb[j] = make_float2(0.f, 0.f);
-    if (q < LPW * H && gl < nlines) {
+    wa[j] = wb[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (k < H && gl < nlines) {
       const long s = gl / npair;
       const int ka = 2 * (int)(gl - s * npair);
       const int ra = ka < hi ? L + ka - hi : ka - hi;
       const int rb = ka + 1 < hi ? L + ka + 1 - hi : ka + 1 - hi;
-      wa[j] = a.half[(s * L + ra) * a.pitch + k];
-      if (ka + 1 < a.nm) wb[j] = a.half[(s * L + rb) * a.pitch + k];
+      const float2* half = a.half + s * half_grid_size(L);
+      wa[j] = *reinterpret_cast<const float4*>(half + half_at(L, ra, k));
+      if (ka + 1 < a.nm)
+        wb[j] = *reinterpret_cast<const float4*>(half + half_at(L, rb, k));
     }
   }
 #pragma unroll
   for (int j = 0; j < NQ; ++j) {
     const int q = (int)threadIdx.x + j * P::NT;
-    if (q < LPW * H) {
-      const int l = q / H, k = q - (q / H) * H;
-      float2 x = wa[j], y = wb[j];
+    const int l = q / HC % LPW;
+    const int k0 = (q / (HC * LPW) * HC + q % HC) * 2;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int k = k0 + e;
+      if (k >= H) break;
+      float2 x = e ? make_float2(wa[j].z, wa[j].w)
+                   : make_float2(wa[j].x, wa[j].y);
+      float2 y = e ? make_float2(wb[j].z, wb[j].w)
+                   : make_float2(wb[j].x, wb[j].y);
       if (k == 0 || 2 * k == L) x.y = y.y = 0.f;  // real by symmetry
       sm[l * P::LS + k] = make_float2(x.x - y.y, x.y + y.x);
       if (k > 0 && L - k >= H)
@@ -556,7 +584,7 @@ using L3072 = LinePlan<3072, 24, 2, Radices<24, 8, 4, 4>, Radices<4, 4, 8, 24>>;
 using L3456 = LinePlan<3456, 24, 2, Radices<24, 24, 6>, Radices<6, 24, 24>>;
 using L3888 = LinePlan<3888, 36, 2, Radices<18, 18, 12>, Radices<12, 18, 18>>;
 using L4096 = LinePlan<4096, 16, 1, Radices<16, 16, 16>, Radices<16, 16, 16>>;
-using L4374 = LinePlan<4374, 18, 1, Radices<18, 9, 9, 3>, Radices<3, 9, 9, 18>>;
+using L4374 = LinePlan<4374, 18, 2, Radices<18, 9, 9, 3>, Radices<3, 9, 9, 18>>;
 using L4608 = LinePlan<4608, 24, 1, Radices<24, 24, 8>, Radices<8, 24, 24>>;
 using L5184 = LinePlan<5184, 36, 1, Radices<36, 12, 12>, Radices<12, 12, 36>>;
 using L5832 = LinePlan<5832, 18, 1, Radices<18, 18, 18>, Radices<18, 18, 18>>;

@@ -12,7 +12,8 @@ struct LineFFTArgs {
   int lines_per_batch = 0;
   int nbatch = 1;
   long bstride = 0;   // complex elements between batches
-  long lstride = 0;   // complex elements between lines of a batch
+  long lstride = 0;   // complex elements between groups of lines
+  int lgroup = 1;     // adjacent lines (element distance 1) in a group
   long estride = 1;   // complex elements between elements of a line
   int nin = 0;        // leading input elements read (rest treated as zero)
   int nout = 0;       // leading output elements written
@@ -28,8 +29,26 @@ struct LineFFTArgs {
 // runtime-plan kernel.
 void fft_lines(const LineFFTArgs& a, int dir, hipStream_t stream);
 
-// Rows of nm real modes <-> the non-redundant half (columns 0 .. L/2) of an
-// L x L Hermitian grid.  Mode index k stands for k - floor(nm/2); row k of
+// Storage of the non-redundant half (columns 0 .. L/2) of an L x L Hermitian
+// grid: blocks of HG_B columns, each block row by row.  A column's elements
+// are HG_B apart and two adjacent rows share 2 HG_B adjacent elements, so
+// neither the column pass (8 useful bytes in each line it touches, row by row)
+// nor the row pass (the same, column by column) pays for the other; the
+// spreading's regions of 4 x 16 cells are whole cache lines.  Against whole
+// rows (columns / interpolation / rows to image, us): 593 / - / 145 -> 270 / -
+// / 154 at 8 x 2048^2 on 4374^2, 95 / 117 / - -> 55 / 91 / - at 8 x 1024^2 and
+// 720 angles on 2048^2.  Blocks of 2: columns 45, but interpolation 1.5 times as
+// long; of 8: columns 85.
+constexpr int HG_B = 4;
+__host__ __device__ __forceinline__ long half_grid_size(int L) {
+  return (long)L * ((L / 2 + HG_B) / HG_B * HG_B);
+}
+// element of a slice; below 2^31 for every L whose lines fit in LDS
+__device__ __forceinline__ unsigned half_at(int L, int row, int col) {
+  return (unsigned)(((col / HG_B) * L + row) * HG_B + col % HG_B);
+}
+
+// Rows of nm real modes <-> the half of an L x L Hermitian grid.  Mode index k stands for k - floor(nm/2); row k of
 // slice s is grid row (k - floor(nm/2)) mod L.
 //   r2c: half = forward row transforms of real_in, each value times
 //        corr[row] corr[column]; only the nm mode rows are written;
@@ -38,10 +57,9 @@ void fft_lines(const LineFFTArgs& a, int dir, hipStream_t stream);
 struct RealRowsArgs {
   const float* real_in = nullptr;  // [nsl][nm][nm]
   float* real_out = nullptr;       // [nsl][nm][nm]
-  float2* half = nullptr;          // [nsl][L][pitch]
+  float2* half = nullptr;          // [nsl][half_grid_size(L)]
   const float* corr = nullptr;     // [nm]
   int L = 0, nm = 0, nsl = 0;
-  long pitch = 0;  // >= L/2 + 1
   float scale = 1.0f;
 };
 void fft_real_rows(const RealRowsArgs& a, bool r2c, hipStream_t stream);

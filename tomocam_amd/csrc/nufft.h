@@ -52,11 +52,11 @@ class PolarNufft {
   void type2_real(const float* f, float2* c, int S, hipStream_t stream);
 
  private:
-  int P_, N_, nm_, nf_, pitch_;
+  int P_, N_, nm_, nf_;
   float beta_;
   DevBuf ax_, ay_;   // double[P]: cos/sin(theta) * nf / (N - 1)
   DevBuf corr_;      // float[nm]: (-1)^k h / psi_hat(k)
-  DevBuf fine_;      // float2 [batch][nf][pitch]: columns 0 .. nf/2 of the
+  DevBuf fine_;      // float2 [batch][half_grid_size(nf)]: columns 0 .. nf/2 of the
                      // (Hermitian) grid
   int fine_batch_ = 0;
   float2* fine(int batch);

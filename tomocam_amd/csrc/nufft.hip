@@ -85,8 +85,8 @@ static void gauss_legendre(int n, std::vector<double>& x, std::vector<double>& w
 struct SpreadArgs {
   TileGeom g;       // columns 0 .. g.ncols - 1 of the grid
   const float2* c;  // [nsl][P][nh]: values at t = 0 .. nh - 1, t < 0 conjugate
-  float2* fine;     // [nsl][nf][pitch]
-  int nsl, nh, pitch;
+  float2* fine;     // [nsl][half_grid_size(g.nf)]
+  int nsl, nh;
   float beta;
 };
 
@@ -106,8 +106,8 @@ struct SpreadArgs {
 // The former kernel added points to LDS cells (read, add, write of 8 bytes per
 // cell, slice and point), about 615 SIMD cycles a point for four slices; here
 // a point costs 16.6 % of 16 regions x 32 cycles for two slices.
-// 8 x 2048^2 at 1501 angles (4374^2 grid): 2.81 -> 0.72 ms, now bound by
-// writing the grid.
+// 8 x 2048^2 at 1501 angles (4374^2 grid, 613 MB of half grids): 0.34 ms, of
+// which writing takes 0.13 at the rate of a large copy.
 constexpr int SP_BATCH = 128;
 
 using f32x4 = __attribute__((__vector_size__(4 * sizeof(float)))) float;
@@ -289,8 +289,8 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
       if (dst) {
         dst[(s * SP_T + ly) * SP_T + lx] = val;
       } else if (in && s < ns) {
-        a.fine[((long)(s0 + s) * a.g.nf + w.Y0 + ly) * a.pitch + w.X0 + lx] =
-            val;
+        a.fine[(s0 + s) * half_grid_size(a.g.nf) +
+               half_at(a.g.nf, w.Y0 + ly, w.X0 + lx)] = val;
       }
     }
   }
@@ -351,8 +351,8 @@ spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix,
     const int cell = threadIdx.x + 256 * e;
     const int ly = cell / SP_T, lx = cell - ly * SP_T;
     if (w.Y0 + ly < w.Y1 && w.X0 + lx < w.X1) {
-      float2* o = a.fine + ((long)(s0 + s) * a.g.nf + w.Y0 + ly) * a.pitch +
-                  w.X0 + lx;
+      float2* o = a.fine + (s0 + s) * half_grid_size(a.g.nf) +
+                  half_at(a.g.nf, w.Y0 + ly, w.X0 + lx);
       const float2 cur = *o;
       *o = make_float2((float)(cur.x + sum[e].x), (float)(cur.y + sum[e].y));
     }
@@ -364,11 +364,11 @@ spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix,
 // ---------------------------------------------------------------------------
 
 struct InterpArgs {
-  const float2* fine;  // [nsl][nf][pitch], columns 0 .. nf/2
+  const float2* fine;  // [nsl][half_grid_size(nf)]
   float2* c;           // [nsl][P][nh]
   const double* ax;
   const double* ay;
-  int P, N, nh, nf, pitch, nsl;
+  int P, N, nh, nf, nsl;
   float beta;
 };
 
@@ -377,20 +377,47 @@ struct InterpArgs {
 // (columns up to nf/2); a footprint column past either end of that half is
 // read at its mirror image, conjugated.
 //
-// Lane b of a point's group of eight reads footprint column b of every row
-// (its eight rows from one slice are eight loads), so a wave's gather for
-// one row covers eight points x 64 contiguous bytes instead of 64 scattered
-// cells.  The lane weights its column sum by wx[b]; the eight columns are
-// then summed across the group for eight slices at once by a transposing
-// butterfly (exchange halves with lanes b^4, b^2, b^1: 14 shuffles per
-// eight slices), after which lane b holds slice b of the chunk and writes
-// it.  The summation order is fixed, so results are deterministic.
+// Eight lanes take a point.  The grid stores HG_B = 4 columns a block, four
+// rows of a block in 128 bytes, and a footprint's 8 columns lie in three
+// blocks: lane (r, c) = (b >> 1, b & 1) reads columns 2 c, 2 c + 1 of every
+// block in rows r and r + 4, six 16-byte loads a slice, each covering 128
+// adjacent bytes a point (weights past the footprint are zero).  The loads
+// are bound by the cache lines they touch, about 10 a point and slice; one
+// column a lane, row by row, touched about 22 (8 x 1024^2 at 720 angles:
+// 117 -> 91 us; 8 x 512^2 at 360: 41 -> 27 us).  Where the three blocks reach past the stored half (near columns 0
+// and nf/2) the wave takes that form: lane b reads footprint column b of
+// every row, or its mirror image.
+//
+// The eight lanes' sums are then added across the group for eight slices at
+// once by a transposing butterfly (exchange halves with lanes b^4, b^2, b^1:
+// 14 shuffles per eight slices), after which lane b holds slice b of the chunk
+// and writes it.  The summation order is fixed by the geometry, so results are
+// deterministic.
 __device__ __forceinline__ float2 shfl_xor2(float2 v, int m) {
   return make_float2(__shfl_xor(v.x, m, 8), __shfl_xor(v.y, m, 8));
 }
 
+// Sum over the group's lanes of a lane's part(q) for slices q = 0 .. 7: lane b
+// gets slice b's.  Each exchange halves the slices a lane stands for; they are
+// taken in the order that lets every exchange happen as soon as it can, so
+// that few partial sums are held.
+template <int M, class F>
+__device__ __forceinline__ float2 group_sum(const F& part, int b, int q) {
+  if constexpr (M == 0) {
+    return part(q);
+  } else {
+    const float2 lo = group_sum<M == 4 ? 0 : 2 * M>(part, b, q);
+    const float2 hi = group_sum<M == 4 ? 0 : 2 * M>(part, b, q + M);
+    const bool up = (b & M) != 0;
+    const float2 keep = up ? hi : lo, got = shfl_xor2(up ? lo : hi, M);
+    return make_float2(keep.x + got.x, keep.y + got.y);
+  }
+}
+
 __global__ void __launch_bounds__(256) interp_kernel(InterpArgs a) {
-  const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  // each XCD takes adjacent rays, whose footprints overlap in its L2
+  const long gid =
+      (long)xcd_remap(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   const long pt = gid >> 3;
   const int b = (int)(gid & 7);
   // groups of eight are aligned to eight lanes: a group is all in or out
@@ -404,69 +431,113 @@ __global__ void __launch_bounds__(256) interp_kernel(InterpArgs a) {
   const int l0y = first_cell<NUFFT_W>(0.5 * a.nf, t, a.ay[p], fy);
   const float wxb = es_kernel_diff((fx + (float)b) * (2.0f / NUFFT_W), a.beta);
   const float wyb = es_kernel_diff((fy + (float)b) * (2.0f / NUFFT_W), a.beta);
+  // conjugated where t < 0 was evaluated for t > 0; the sample at the ray's
+  // end of an even N is halved (RayArgs)
+  const float end = 2 * m == a.N ? 0.5f : 1.0f;
+  const float endi = t < 0.0 ? -end : end;
+  const long plane = half_grid_size(a.nf);
+  const long cplane = (long)a.P * a.nh;
+  const int x0 = l0x & ~(HG_B - 1);
+  if (!__any(l0x < 0 || x0 + 3 * HG_B > a.nf / 2 + 1)) {
+    const int r0 = b >> 1, c0 = 2 * (b & 1);
+    float wx[3][2], wy[2];
+    unsigned off[2];
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int f = x0 + HG_B * j + c0 + e - l0x;  // footprint column
+        const float w = __shfl(wxb, f & 7, 8);
+        wx[j][e] = f >= 0 && f < NUFFT_W ? w : 0.f;
+      }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      wy[h] = __shfl(wyb, r0 + 4 * h, 8);
+      int qy = l0y + r0 + 4 * h;
+      qy += qy < 0 ? a.nf : (qy >= a.nf ? -a.nf : 0);
+      off[h] = half_at(a.nf, qy, x0) + c0;
+    }
+    for (int s0 = 0; s0 < a.nsl; s0 += 8) {
+      auto part = [&](int q) {
+        const float2* g = a.fine + (long)(s0 + q) * plane;
+        float4 val[2][3];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int j = 0; j < 3; ++j)
+            val[h][j] = *reinterpret_cast<const float4*>(
+                g + (long)j * HG_B * a.nf + off[h]);
+        float2 sum[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          sum[h] = make_float2(0.f, 0.f);
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            sum[h].x = fmaf(val[h][j].x, wx[j][0], sum[h].x);
+            sum[h].y = fmaf(val[h][j].y, wx[j][0], sum[h].y);
+            sum[h].x = fmaf(val[h][j].z, wx[j][1], sum[h].x);
+            sum[h].y = fmaf(val[h][j].w, wx[j][1], sum[h].y);
+          }
+        }
+        return make_float2(fmaf(wy[1], sum[1].x, wy[0] * sum[0].x),
+                           fmaf(wy[1], sum[1].y, wy[0] * sum[0].y));
+      };
+      // whole chunks without a branch a slice, so that loads of several slices
+      // are in flight
+      const float2 v =
+          s0 + 8 <= a.nsl
+              ? group_sum<1>(part, b, 0)
+              : group_sum<1>(
+                    [&](int q) {
+                      return s0 + q < a.nsl ? part(q) : make_float2(0.f, 0.f);
+                    },
+                    b, 0);
+      if (s0 + b < a.nsl)
+        a.c[(long)(s0 + b) * cplane + pt] = make_float2(end * v.x, endi * v.y);
+    }
+    return;
+  }
   int qx = l0x + b;
   qx += qx < 0 ? a.nf : (qx >= a.nf ? -a.nf : 0);
   const bool mirror = 2 * qx > a.nf;
   if (mirror) qx = a.nf - qx;
   float wy[NUFFT_W];
-  long roff[NUFFT_W];
+  unsigned roff[NUFFT_W];
 #pragma unroll
   for (int r = 0; r < NUFFT_W; ++r) {
     wy[r] = __shfl(wyb, r, 8);
     int qy = l0y + r;
     qy += qy < 0 ? a.nf : (qy >= a.nf ? -a.nf : 0);
     if (mirror && qy > 0) qy = a.nf - qy;
-    roff[r] = (long)qy * a.pitch + qx;
+    roff[r] = half_at(a.nf, qy, qx);
   }
   const float flip = mirror ? -wxb : wxb;
-  // conjugated where t < 0 was evaluated for t > 0; the sample at the ray's
-  // end of an even N is halved (RayArgs)
-  const float end = 2 * m == a.N ? 0.5f : 1.0f;
-  const float endi = t < 0.0 ? -end : end;
-  const long plane = (long)a.nf * a.pitch;
-  const long cplane = (long)a.P * a.nh;
-  for (int s0 = 0; s0 < a.nsl; s0 += 8) {
-    float2 part[8];
-#pragma unroll 2
-    for (int q = 0; q < 8; ++q) {
-      float2 acc = make_float2(0.f, 0.f);
-      if (s0 + q < a.nsl) {
-        const float2* g = a.fine + (long)(s0 + q) * plane;
-        float2 val[NUFFT_W];
+  // a slice at a time: few waves come here, and must not cost the others
+  // registers
+#pragma unroll 1
+  for (int s = 0; s < a.nsl; ++s) {
+    const float2* g = a.fine + (long)s * plane;
+    float2 val[NUFFT_W];
 #pragma unroll
-        for (int r = 0; r < NUFFT_W; ++r) val[r] = g[roff[r]];
+    for (int r = 0; r < NUFFT_W; ++r) val[r] = g[roff[r]];
+    float2 acc = make_float2(0.f, 0.f);
 #pragma unroll
-        for (int r = 0; r < NUFFT_W; ++r) {
-          acc.x = fmaf(val[r].x, wy[r], acc.x);
-          acc.y = fmaf(val[r].y, wy[r], acc.y);
-        }
+    for (int r = 0; r < NUFFT_W; ++r) {
+      acc.x = fmaf(val[r].x, wy[r], acc.x);
+      acc.y = fmaf(val[r].y, wy[r], acc.y);
+    }
+    {
+      // no contraction: every lane holds the same sum, whichever stores it
+#pragma clang fp contract(off)
+      acc = make_float2(acc.x * wxb, acc.y * flip);
+#pragma unroll
+      for (int k = 4; k > 0; k >>= 1) {
+        const float2 got = shfl_xor2(acc, k);
+        acc = make_float2(acc.x + got.x, acc.y + got.y);
       }
-      part[q] = make_float2(acc.x * wxb, acc.y * flip);
     }
-    // lanes with bit m set keep the upper half of their slice set
-    float2 h4[4], h2[2];
-    const bool u4 = (b & 4) != 0, u2 = (b & 2) != 0, u1 = (b & 1) != 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float2 keep = u4 ? part[4 + k] : part[k];
-      const float2 give = u4 ? part[k] : part[4 + k];
-      const float2 got = shfl_xor2(give, 4);
-      h4[k] = make_float2(keep.x + got.x, keep.y + got.y);
-    }
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const float2 keep = u2 ? h4[2 + k] : h4[k];
-      const float2 give = u2 ? h4[k] : h4[2 + k];
-      const float2 got = shfl_xor2(give, 2);
-      h2[k] = make_float2(keep.x + got.x, keep.y + got.y);
-    }
-    const float2 keep = u1 ? h2[1] : h2[0];
-    const float2 give = u1 ? h2[0] : h2[1];
-    const float2 got = shfl_xor2(give, 1);
-    // lane b now holds slice s0 + b (bits 4, 2, 1 of b chose the halves)
-    if (s0 + b < a.nsl)
-      a.c[(long)(s0 + b) * cplane + pt] =
-          make_float2(end * (keep.x + got.x), endi * (keep.y + got.y));
+    if (b == (s & 7))
+      a.c[(long)s * cplane + pt] = make_float2(end * acc.x, endi * acc.y);
   }
 }
 
@@ -495,8 +566,6 @@ PolarNufft::PolarNufft(const float* h_angles, int nproj, int npix, int nmodes)
   TC_REQUIRE(nproj <= 2048, "NUFFT: too many projection angles");
   TC_REQUIRE(npix < 65536, "NUFFT: too many samples per ray");
   nf_ = grid_length(std::max(2 * nmodes, 2 * NUFFT_W), true);
-  // half rows in whole 128-byte lines, so that tiles start on one
-  pitch_ = (nf_ / 2 + 1 + 15) / 16 * 16;
   beta_ = (float)(2.30 * NUFFT_W);
   std::vector<double> hx(P_), hy(P_);
   const double sc = (double)nf_ / (double)(npix - 1);
@@ -537,7 +606,7 @@ PolarNufft::PolarNufft(const float* h_angles, int nproj, int npix, int nmodes)
 
 float2* PolarNufft::fine(int batch) {
   if (batch > fine_batch_) {
-    fine_.alloc(sizeof(float2) * (size_t)batch * nf_ * pitch_);
+    fine_.alloc(sizeof(float2) * (size_t)batch * half_grid_size(nf_));
     fine_batch_ = batch;
   }
   return fine_.as<float2>();
@@ -556,7 +625,6 @@ SpreadArgs PolarNufft::spread_args() const {
   a.g.umax = a.g.cidx * ((double)nf_ / (N_ - 1)) + 1.0;
   lists_.fill(a.g);
   a.nh = nh();
-  a.pitch = pitch_;
   a.beta = beta_;
   return a;
 }
@@ -580,8 +648,8 @@ static std::tuple<int, int, int, int, int> chunk_key(int P, int N, int nf,
 // point set-up for fewer slices), rounding up while that stays within
 // 1.25 GB.
 constexpr int SP_SB = 8;
-static int fine_batch(int nf, int pitch, int S) {
-  const double per = 8.0 * nf * (double)pitch, budget = 1.0e9;
+static int fine_batch(int nf, int S) {
+  const double per = 8.0 * (double)half_grid_size(nf), budget = 1.0e9;
   const int b0 = (int)std::max(1.0, std::floor(budget / per));
   int b = b0;
   const int up = (b0 + SP_SB - 1) / SP_SB * SP_SB;
@@ -595,7 +663,7 @@ static int fine_batch(int nf, int pitch, int S) {
 void PolarNufft::type1_real(const float2* c, float* out, int S, float scale,
                             hipStream_t stream) {
   TC_REQUIRE(S >= 1, "NUFFT: need at least one slice");
-  const int B = fine_batch(nf_, pitch_, S);
+  const int B = fine_batch(nf_, S);
   float2* fg = fine(B);
   // slices a spreading workgroup takes: a point's weights and footprint serve
   // all of them, so as many as there are, up to 8 (64 accumulators a lane)
@@ -722,7 +790,7 @@ void PolarNufft::type1_real(const float2* c, float* out, int S, float scale,
 void PolarNufft::type2_real(const float* f, float2* c, int S,
                             hipStream_t stream) {
   TC_REQUIRE(S >= 1, "NUFFT: need at least one slice");
-  const int B = fine_batch(nf_, pitch_, S);
+  const int B = fine_batch(nf_, S);
   float2* fg = fine(B);
   for (int s0 = 0; s0 < S; s0 += B) {
     const int nb = std::min(B, S - s0);
@@ -739,7 +807,6 @@ void PolarNufft::type2_real(const float* f, float2* c, int S,
     a.N = N_;
     a.nh = nh();
     a.nf = nf_;
-    a.pitch = pitch_;
     a.nsl = nb;
     a.beta = beta_;
     hipLaunchKernelGGL(interp_kernel, dim3(cdiv(8L * P_ * a.nh, 256)),
@@ -755,7 +822,6 @@ RealRowsArgs PolarNufft::real_rows(int nsl) const {
   r.L = nf_;
   r.nm = nm_;
   r.nsl = nsl;
-  r.pitch = pitch_;
   return r;
 }
 
@@ -767,9 +833,10 @@ void PolarNufft::columns(int nsl, int dir, hipStream_t stream) {
   a.L = nf_;
   a.nbatch = nsl;
   a.lines_per_batch = nf_ / 2 + 1;
-  a.bstride = (long)nf_ * pitch_;
-  a.lstride = 1;
-  a.estride = pitch_;
+  a.bstride = half_grid_size(nf_);
+  a.lgroup = HG_B;
+  a.lstride = (long)nf_ * HG_B;
+  a.estride = HG_B;
   a.colmajor = true;
   const int lo = (nm_ + 1) / 2, hi = nm_ / 2;
   a.nin = dir < 0 ? lo : nf_;
