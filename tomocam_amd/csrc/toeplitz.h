@@ -4,7 +4,7 @@
 // placed circularly on an M x M grid (M = smallest even 2,3,5,7-smooth size
 // >= 2n-1), whose spectrum is real and even.  One application is three
 // passes over HBM:
-//   A  pair-packed real row FFTs of the n non-zero rows -> Wt[s][k1][row]
+//   A  pair-packed real row FFTs of the n non-zero rows -> Wt
 //      (k1 < H = M/2+1, stored k1-major so pass B reads whole columns);
 //   B  per k1: zero-padded column FFT, multiply by the real spectrum, inverse
 //      column FFT, keep the n output rows; also sum |X|^2 * spectrum (the

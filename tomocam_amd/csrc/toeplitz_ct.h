@@ -103,17 +103,24 @@ __device__ __forceinline__ int col_scale_index(int s, int k1, int row, int H) {
   return (s * ((H + LPWC - 1) / LPWC) + kg) * P::SG + (tid >> 5);
 }
 
-// Wt element (slice s, column k1, row): layout [s][k1][rp], so the column
-// pass reads whole columns.  (A row-group-major layout, which makes the row
-// passes stream contiguously, measured slower overall: the column pass loses
-// more than the row passes gain.)
+// Wt element (column k1, row) of a slice: blocks of WT_B columns, each block
+// by row pairs, a pair's columns side by side, its two rows adjacent.  A row
+// pass moves 16 bytes a pair and column, so two columns make 32 adjacent ones;
+// the column pass reads half of every 32.  Against whole columns (WT_B = 1):
+// passes of 8 x 1454^2 fwd / cols / inv 68 / 146 / 74 -> 62 / 147 / 71 us, two
+// slices of 2908^2 202 / 363 / 234 -> 165 / 370 / 191 us; 4: the column pass
+// loses what the row passes gain (154 us, 8 x 1454^2).  The last block holds
+// what columns are left, so the workspace has no padding.
 //
 // Every access of the passes is a slice's base (the same for the whole
 // workgroup, in scalar registers) plus a 32-bit byte offset: as 64-bit
 // addresses per lane the offsets took a fifth of the passes' vector
 // instructions.
-__device__ __forceinline__ unsigned wt_at(int k1, int row, int rp) {
-  return (unsigned)k1 * (unsigned)rp + (unsigned)row;
+constexpr unsigned WT_B = 2;
+__device__ __forceinline__ unsigned wt_at(int k1, int row, int H, int rp) {
+  const unsigned k0 = (unsigned)k1 / WT_B * WT_B, r = row;
+  const unsigned w = min(WT_B, (unsigned)H - k0);
+  return k0 * (unsigned)rp + ((r / 2) * w + ((unsigned)k1 - k0)) * 2 + r % 2;
 }
 // element i of a uniform base
 template <typename T>
@@ -141,7 +148,7 @@ struct CommitPtrs {
 };
 
 // ---------------------------------------------------------------------------
-// pass A: pair-packed forward row FFTs -> Wt[s][k1][row]
+// pass A: pair-packed forward row FFTs -> Wt
 //   (+ dst = y - s x when committing a step: x is the gradient there)
 // ---------------------------------------------------------------------------
 
@@ -268,12 +275,12 @@ ct_rows_fwd(const void* __restrict__ xv, void* __restrict__ wtv,
       if constexpr (W16) {
         // |value| <= n * 2^16 * wsc <= 2^15: no overflow
         at32(reinterpret_cast<uint2*>(reinterpret_cast<unsigned*>(wtv) + ws),
-             wt_at(k, rr, rp) / 2) =
+             wt_at(k, rr, H, rp) / 2) =
             make_uint2(pack_half2(hw * sp.x, hw * sp.y),
                        pack_half2(hw * df.y, -hw * df.x));
       } else {
         at32(reinterpret_cast<float4*>(reinterpret_cast<float2*>(wtv) + ws),
-             wt_at(k, rr, rp) / 2) =
+             wt_at(k, rr, H, rp) / 2) =
             make_float4(hw * sp.x, hw * sp.y, hw * df.y, -hw * df.x);
       }
     }
@@ -321,7 +328,7 @@ ct_cols(void* __restrict__ wtv, const void* __restrict__ specv,
       const int idx = t + i * T + r * (L / R1);
       float2 w = make_float2(0.f, 0.f);
       if (r < R1 / 2 && active && idx < n) {
-        const unsigned o = wt_at(kc, idx, rp);
+        const unsigned o = wt_at(kc, idx, H, rp);
         // FP16: the raw word, unpacked once every load is issued
         if constexpr ((HM & HM_WT16) != 0)
           w.x = __uint_as_float(
@@ -418,7 +425,7 @@ ct_cols(void* __restrict__ wtv, const void* __restrict__ specv,
         for (int r = 0; r < R1 / 2; ++r) {
           const int idx = t + i * T + r * (L / R1);
           if (idx < n)
-            at32(reinterpret_cast<unsigned*>(wtv) + ws, wt_at(kc, idx, rp)) =
+            at32(reinterpret_cast<unsigned*>(wtv) + ws, wt_at(kc, idx, H, rp)) =
                 pack_half2(kap * v[i * R1 + r].x, kap * v[i * R1 + r].y);
         }
     }
@@ -433,7 +440,7 @@ ct_cols(void* __restrict__ wtv, const void* __restrict__ specv,
       for (int r = 0; r < R1 / 2; ++r) {
         const int idx = t + i * T + r * (L / R1);
         if (idx < n)
-          at32(reinterpret_cast<float2*>(wtv) + ws, wt_at(kc, idx, rp)) =
+          at32(reinterpret_cast<float2*>(wtv) + ws, wt_at(kc, idx, H, rp)) =
               v[i * R1 + r];
       }
   }
@@ -491,7 +498,7 @@ ct_rows_inv(const void* __restrict__ wtv, const float* bvec, float* out,
       u16[j] = make_uint2(0u, 0u);
     }
     if (q < LPW * H && rr < rp) {
-      const unsigned o = wt_at(k, rr, rp) / 2;
+      const unsigned o = wt_at(k, rr, H, rp) / 2;
       if constexpr (W16) {
         u16[j] = at32(reinterpret_cast<const uint2*>(
                           reinterpret_cast<const unsigned*>(wtv) + ws), o);
