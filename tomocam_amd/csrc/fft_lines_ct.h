@@ -154,7 +154,7 @@ void run_lines(const LineFFTArgs& a, int dir, hipStream_t stream) {
 // slice make one complex line, so a row costs half a complex transform and
 // the half spectrum half the memory; the corrections of the NUFFT modes are
 // applied on the way.  8 x 1024^2 on a 2048^2 grid: correction and padding
-// (95 us) and complex row transforms (90 us) -> 41 us.
+// (95 us) and complex row transforms (90 us) -> 35 us.
 // ---------------------------------------------------------------------------
 
 template <class P>
