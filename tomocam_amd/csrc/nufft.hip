@@ -322,40 +322,33 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
 
 // Adds the scratch slots of multi-chunk tiles into the fine grid, in slot
 // order (deterministic).  sb: slices per group of the spreading launch.
-__global__ void __launch_bounds__(256)
-spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix,
-                    const float2* __restrict__ scratch, int sb) {
-  const int4 f = fix[blockIdx.x];
-  const int s0 = blockIdx.y * sb;
-  const int ns = min(sb, a.nsl - s0);
+// blockIdx.z picks a slice of the group.  A thread sums four cells over the
+// slots, four slots at a time (16 loads in flight); of the first nheavy tiles,
+// whose slots would be a long chain, one cell and sixteen slots at a time, four
+// workgroups a tile.  (All tiles that way: 22 instead of 11 us at 8 x 512^2,
+// where most tiles have few slots; none: 36 instead of 17 us at 8 x 2048^2, whose
+// centre has 211 slots.)  The order per cell is slot order.  The sums are FP64: the centre's cells add a value of the same sign
+// from every ray over many slots, and their rounding is a level error of the
+// whole image.
+template <int PER, int U>
+__device__ __forceinline__ void spread_fixup(const SpreadArgs& a, int4 f, int s,
+                                             const float2* base,
+                                             long slot_stride, int first) {
   const TileWindow w = tile_window(a.g, f.x);
-  // blockIdx.z picks a slice of the group; each thread sums four cells over the
-  // slots, four slots at a time (16 loads in flight); the order per cell is slot
-  // order.  (One cell a thread and sixteen slots at a time, four times the
-  // workgroups: 22 instead of 11 us at 8 x 512^2, where most tiles have few
-  // slots.)  The sums are FP64: the centre's cells add a value of the same sign
-  // from every ray over many slots, and their rounding is a level error of the
-  // whole image.
-  const int s = blockIdx.z;
-  if (s >= ns) return;
-  constexpr int PER = SP_T * SP_T / 256;
-  const long slot_stride = (long)gridDim.y * sb * (SP_T * SP_T);
-  const float2* base = scratch + (long)f.y * slot_stride +
-                       ((long)blockIdx.y * sb + s) * (SP_T * SP_T) +
-                       threadIdx.x;
+  base += first;
   double2 sum[PER];
 #pragma unroll
   for (int e = 0; e < PER; ++e) sum[e] = make_double2(0.0, 0.0);
   int k = 0;
-  for (; k + 4 <= f.z; k += 4) {
-    float2 q[4][PER];
+  for (; k + U <= f.z; k += U) {
+    float2 q[U][PER];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int e = 0; e < PER; ++e)
         q[u][e] = base[(long)(k + u) * slot_stride + 256 * e];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int e = 0; e < PER; ++e) {
         sum[e].x += q[u][e].x;
@@ -372,15 +365,34 @@ spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix,
   }
 #pragma unroll
   for (int e = 0; e < PER; ++e) {
-    const int cell = threadIdx.x + 256 * e;
+    const int cell = first + 256 * e;
     const int ly = cell / SP_T, lx = cell - ly * SP_T;
     if (w.Y0 + ly < w.Y1 && w.X0 + lx < w.X1) {
-      float2* o = a.fine + (s0 + s) * half_grid_size(a.g.nf) +
+      float2* o = a.fine + s * half_grid_size(a.g.nf) +
                   half_at(a.g.nf, w.Y0 + ly, w.X0 + lx);
       const float2 cur = *o;
       *o = make_float2((float)(cur.x + sum[e].x), (float)(cur.y + sum[e].y));
     }
   }
+}
+
+__global__ void __launch_bounds__(256)
+spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix, int nheavy,
+                    const float2* __restrict__ scratch, int sb) {
+  static_assert(SP_T * SP_T == 4 * 256, "four cells a thread");
+  const int s = blockIdx.y * sb + blockIdx.z;
+  if (s >= a.nsl) return;
+  const int b = blockIdx.x;
+  const bool heavy = b < 4 * nheavy;
+  const int4 f = fix[heavy ? b / 4 : b - 3 * nheavy];
+  const long slot_stride = (long)gridDim.y * sb * (SP_T * SP_T);
+  const float2* base =
+      scratch + (long)f.y * slot_stride + (long)s * (SP_T * SP_T);
+  if (heavy)
+    spread_fixup<1, 16>(a, f, s, base, slot_stride,
+                        256 * (b & 3) + (int)threadIdx.x);
+  else
+    spread_fixup<4, 4>(a, f, s, base, slot_stride, threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -711,8 +723,10 @@ void PolarNufft::type1_real(const float2* c, float* out, int S, float scale,
     TC_HIP(hipGetLastError());
     if (lists_.nfix()) {
       hipLaunchKernelGGL(spread_fixup_kernel,
-                         dim3((unsigned)lists_.nfix(), ng, sb), dim3(256), 0,
-                         stream, a, lists_.fix(), scratch, sb);
+                         dim3((unsigned)(lists_.nfix() + 3 * lists_.nheavy()),
+                              ng, sb),
+                         dim3(256), 0, stream, a, lists_.fix(),
+                         lists_.nheavy(), scratch, sb);
       TC_HIP(hipGetLastError());
     }
   };

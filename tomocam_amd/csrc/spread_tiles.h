@@ -11,6 +11,14 @@
 namespace tc {
 
 constexpr int SP_T = 32;  // tile edge (grid points)
+// The cells within SP_CENTRE of the grid's centre get points from every ray, and
+// the same values again and again (the sample t = 0 of each ray is one point).
+// Added one after the other, hundreds in a work item, their rounding is not
+// random: a level error of the whole image or PSF (T x of 1454^2 at 720 angles
+// against 64 bits: 6.3e-7 with items of 1024 points there, 3.8e-6 with 4096).
+// The tiles that hold such cells are cut into items of SP_CENTRE_CHUNK points,
+// whose sums the fix-up adds in FP64: 6.4e-8.
+constexpr int SP_CENTRE = 8, SP_CENTRE_CHUNK = 128;
 
 struct TileGeom {
   const double* ax;  // [P] grid steps per sample along x and y
@@ -71,15 +79,18 @@ __device__ __forceinline__ int region_x(int w, int g) {
   return 16 * ((w - g) & 1);
 }
 
+constexpr int SP_FIX_HEAVY = 16;
+
 // The lists of one geometry (device) and the work cut from them.
 class TileLists {
  public:
   // Points per tile and every tile's segments, for kernel width W (8 or 16);
   // reads the counts back (one synchronisation).  g: ax .. umax filled in.
   void make_segments(const TileGeom& g, int W, hipStream_t stream);
-  // The work and fix-up lists for `chunk` points per item.  Synchronous
-  // copies: the caller has no kernel reading the previous lists in flight.
-  void make_work(int chunk);
+  // The work and fix-up lists for `chunk` points per item (the tiles about the
+  // centre: at most SP_CENTRE_CHUNK).  Synchronous copies: the caller has no
+  // kernel reading the previous lists in flight.
+  void make_work(int chunk_max);
   void fill(TileGeom& g) const;  // the list pointers
 
   // Points per item by rule: a workgroup takes its points 128 at a time, in
@@ -94,12 +105,15 @@ class TileLists {
   int nwork() const { return nwork_; }
   int nslots() const { return nslots_; }  // scratch tiles of further chunks
   int nfix() const { return nfix_; }
+  // the fix-up list starts with the tiles of more than SP_FIX_HEAVY slots
+  int nheavy() const { return nheavy_; }
   const int4* work() const { return work_.as<int4>(); }
   const int4* fix() const { return fix_.as<int4>(); }
 
  private:
-  int nwork_ = 0, nslots_ = 0, nfix_ = 0, chunk_ = 0;
+  int nwork_ = 0, nslots_ = 0, nfix_ = 0, nheavy_ = 0, chunk_ = 0;
   std::vector<int> counts_;      // polar points per tile
+  std::vector<char> centre_;     // whether it holds cells about the centre
   std::vector<int> tile_first_;  // first segment of each tile
   DevBuf seg_, seg_off_, tile_seg_;
   // two int4 per item: tile, first point, end point, scratch slot (-1: none);

@@ -144,6 +144,14 @@ void TileLists::make_segments(const TileGeom& geom, int W, hipStream_t stream) {
                         hipMemcpyDeviceToHost, stream));
   TC_HIP(hipStreamSynchronize(stream));
   counts_.assign(h.begin(), h.begin() + ntiles);
+  centre_.resize(ntiles);
+  for (int t = 0; t < ntiles; ++t) {
+    auto near = [&](int i) {  // tile i along an axis
+      return i * SP_T <= g.nf / 2 + SP_CENTRE &&
+             (i + 1) * SP_T > g.nf / 2 - SP_CENTRE;
+    };
+    centre_[t] = near(t / g.ntx) && near(t % g.ntx);
+  }
   tile_first_.assign(ntiles + 1, 0);
   for (int t = 0; t < ntiles; ++t)
     tile_first_[t + 1] = tile_first_[t] + h[ntiles + t];
@@ -162,13 +170,15 @@ void TileLists::make_segments(const TileGeom& geom, int W, hipStream_t stream) {
 // The work and fix-up lists for `chunk` points per item, uploaded to the
 // plan's buffers (synchronous copies: the caller has no kernel reading the
 // previous lists in flight).
-void TileLists::make_work(int chunk) {
+void TileLists::make_work(int chunk_max) {
   ArenaPause no_arena;  // the plan's work lists, filled synchronously
   const int ntiles = (int)counts_.size();
   std::vector<int4> work, fix;
   int slot = 0;
   for (int t = 0; t < ntiles; ++t) {
     const int c = counts_[t];
+    const int chunk =
+        centre_[t] ? std::min(chunk_max, SP_CENTRE_CHUNK) : chunk_max;
     const int nch = std::max(1, (c + chunk - 1) / chunk);
     work.push_back(make_int4(t, 0, std::min(c, chunk), -1));
     if (nch > 1) {
@@ -197,6 +207,10 @@ void TileLists::make_work(int chunk) {
       work[x * q + (x < rmd ? x : rmd) + t] = byw[b];
     }
   }
+  // a fix-up's time grows with the slots of its tile
+  std::stable_sort(fix.begin(), fix.end(), [](const int4& x, const int4& y) {
+    return x.z > y.z;
+  });
   // each item with its tile's range of segments
   std::vector<int4> items;
   items.reserve(2 * work.size());
@@ -207,7 +221,9 @@ void TileLists::make_work(int chunk) {
   nwork_ = (int)work.size();
   nslots_ = slot;
   nfix_ = (int)fix.size();
-  chunk_ = chunk;
+  nheavy_ = 0;
+  while (nheavy_ < nfix_ && fix[nheavy_].z > SP_FIX_HEAVY) ++nheavy_;
+  chunk_ = chunk_max;
   work_.alloc(sizeof(int4) * items.size());
   TC_HIP(hipMemcpy(work_.as<void>(), items.data(), sizeof(int4) * items.size(),
                    hipMemcpyHostToDevice));
