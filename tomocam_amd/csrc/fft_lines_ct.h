@@ -529,9 +529,9 @@ struct LineOps {
 };
 
 // Plans, ascending: length, elements per thread, lines per workgroup and
-// radices (each divides the elements per thread).  The lengths are at most
-// 1/8 apart from 192 on, so that a grid or chirp length rounded up to one
-// costs little; radices of 8 to 36 keep the LDS exchanges at one to three.
+// radices (each divides the elements per thread).  From 192 on the lengths are
+// at most 1/8 apart, but for 216 to 256, 324 to 384 and 648 to 768 (18.5 %), so
+// that a chirp length rounded up to one costs little; radices of 8 to 36 keep the LDS exchanges at one to three.
 #define TC_FOR_LINE_LENGTHS_1(X) \
   X(64) X(96) X(128) X(144) X(192) X(216) X(256) X(288) X(324) X(384) X(432)
 #define TC_FOR_LINE_LENGTHS_2(X) \

@@ -96,7 +96,7 @@ class Psf {
                          bool wt16 = true);
 
   // True when this FFT length has the compile-time passes (fused commit), and
-  // when it has the mixed-precision forms as well.
+  // when this width is served in mixed precision as well.
   bool has_fused() const;
   bool has_mixed() const;
 

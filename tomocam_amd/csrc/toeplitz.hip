@@ -24,9 +24,8 @@ int toeplitz_ct_lpw(int M);
 extern const int kToeplitzCtSizes[];
 extern const float kToeplitzCtCost[];
 extern const int kToeplitzCtCount;
-int toeplitz_plain_length(int m);
+int toeplitz_plan_length(int m, int most);
 bool toeplitz_ct_prepare(int M);
-bool toeplitz_ct_mixed(int M);
 
 // Compile-time plan sizes eligible for an n x n Toeplitz product: >= 2n - 1
 // and within 10 % of the smallest even 2,3,5,7-smooth length, ordered by
@@ -63,11 +62,15 @@ static std::pair<int, int> len_key(int n) {
 // FFT length for an n x n Toeplitz product: any even length >= 2n - 1 gives
 // the same result.  The autotuner's choice for this width if there is one;
 // else among the eligible compile-time plan sizes the one with the least
-// size x relative cost per point; with none, from 486 on the smallest FP32-only
-// plan within 1/8 of the smallest even smooth length, else that length.  (2 x
-// 849^2: 98 us on the runtime-plan kernels, 54 us with the plan; 2 x 3000^2:
-// 1279 us at 6000, 425 us at 6144.  Below 486 a line is a few hundred points
-// and the passes are bound by latency, with a plan or without.)
+// size x relative cost per point (they come first because they alone have the
+// mixed-precision forms, and an operator serves both); with none, from 486 on
+// the cheapest plan of any kind within 1/7 of the smallest even smooth length,
+// which every width from 243 to 4096 has (there without the mixed forms, see
+// has_mixed), else that length.  Runtime-plan kernels against the plan: 2 x 849^2
+// 98 and 54 us; 4 x 330^2, 672 and 768 points, 35 and 27 us; 2 x 1310^2, 2646 and 2916, 280
+// and 72 us; 2 x 2620^2, 5250 and 5832, 1003 and 293 us; 2 x 3000^2, 6000 and
+// 6144, 1279 and 425 us.  Shorter lengths have no plans: trial ones took 13.5
+// instead of 18.8 us at 1 x 128^2 and 21.1 instead of 23.9 at 1 x 181^2.
 int toeplitz_fft_length(int n) {
   {
     // (no device query while nothing is tuned: the rule works without one)
@@ -80,8 +83,10 @@ int toeplitz_fft_length(int n) {
   const std::vector<int> c = toeplitz_ct_candidates(n);
   if (!c.empty()) return c[0];
   const int smooth = fft_next_smooth(2 * n - 1, true);
-  const int plain = smooth >= 486 ? toeplitz_plain_length(2 * n - 1) : 0;
-  return plain > 0 && plain <= smooth + smooth / 8 ? plain : smooth;
+  const int plan = smooth < 486
+                       ? 0
+                       : toeplitz_plan_length(2 * n - 1, smooth + smooth / 7);
+  return plan > 0 ? plan : smooth;
 }
 
 // ---------------------------------------------------------------------------
@@ -520,7 +525,11 @@ bool Psf::run_half(const void* g16, const float* gsc, float* out,
 }
 
 bool Psf::has_fused() const { return toeplitz_ct_lpw(M_) > 0; }
-bool Psf::has_mixed() const { return toeplitz_ct_mixed(M_); }
+bool Psf::has_mixed() const {
+  // the mixed forms serve the widths whose smooth length is within 10 %
+  const std::vector<int> c = toeplitz_ct_candidates(n_);
+  return std::find(c.begin(), c.end(), M_) != c.end();
+}
 
 void toeplitz_set_group(int H, int rp, int elem_bytes, int nslices,
                         int group);

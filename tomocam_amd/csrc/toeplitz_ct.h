@@ -762,8 +762,9 @@ void run_plain(const float* x, const float* b, float* out, float2* wt,
                img_b, spec_b, sc, nullptr, ts, group_cap);
 }
 
-// FP32-only plans, ascending: lengths at most 1/8 apart, which with those of
-// toeplitz_ct.hip serve every width from 243 to 4096.
+// FP32-only plans, ascending.  With those of toeplitz_ct.hip the lengths are at
+// most 16 % apart, and every width from 243 to 4096 has one within 1/7 of the
+// smallest smooth length that it could use.
 #define TC_FOR_TOEPLITZ_PLAIN_1(X) X(486) X(512) X(576) X(648) X(864) X(972)
 #define TC_FOR_TOEPLITZ_PLAIN_2(X) X(1024) X(1152) X(1296) X(1536) X(1728)
 #define TC_FOR_TOEPLITZ_PLAIN_3(X) X(1944) X(2048) X(2592) X(3072) X(3456)

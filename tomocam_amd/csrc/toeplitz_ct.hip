@@ -146,11 +146,21 @@ static const ToeplitzPlainOps* find_plain(int M) {
   return nullptr;
 }
 
-// the smallest FP32-only plan length >= m (0: none)
-int toeplitz_plain_length(int m) {
-  for (const ToeplitzPlainOps* o : kPlain)
-    if (o->M >= m) return o->M;
-  return 0;
+// the length in [m, most] with the FP32 passes, of the plans with
+// mixed-precision forms and of the others, that has the least size x relative
+// time (0: none)
+int toeplitz_plan_length(int m, int most) {
+  int best = 0;
+  float best_cost = 0.f;
+  auto take = [&](int M, float cost) {
+    if (M < m || M > most || (best && M * cost >= best_cost)) return;
+    best = M;
+    best_cost = M * cost;
+  };
+  for (int i = 0; i < kToeplitzCtCount; ++i)
+    take(kToeplitzCtSizes[i], kToeplitzCtCost[i]);
+  for (const ToeplitzPlainOps* o : kPlain) take(o->M, 1.f);
+  return best;
 }
 
 // column-pass lines per workgroup (0: no compile-time plan for M)
@@ -190,13 +200,6 @@ bool toeplitz_ct_prepare(int M) {
       return o != nullptr;
     }
   }
-}
-
-// whether M has the mixed-precision forms
-bool toeplitz_ct_mixed(int M) {
-  for (int i = 0; i < kToeplitzCtCount; ++i)
-    if (kToeplitzCtSizes[i] == M) return true;
-  return false;
 }
 
 // FP16 column-pass scales per slice (0: no compile-time plan for M)
