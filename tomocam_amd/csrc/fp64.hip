@@ -734,11 +734,14 @@ spread_fixup_kernel(SpreadArgs a, const int4* __restrict__ fix,
 // and the columns are summed over the lanes in a fixed order.  (One thread per
 // point evaluated 32 exponentials and read single cells: 2 x 200^2 at 150 angles
 // 65 -> 15 us.)
+// The points are numbered from i0 on: a launch holds fewer than 2^32 threads
+// (what is beyond is dropped without an error).
 __global__ void __launch_bounds__(256)
-interp_kernel(GridArgs g, const double2* __restrict__ fine, double2* c) {
+interp_kernel(GridArgs g, const double2* __restrict__ fine, double2* c,
+              long i0) {
   const long J = (long)g.P * g.N;
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long i = t >> 4;
+  const long i = i0 + (t >> 4);
   const int b = (int)(t & 15);
   if (i >= J * g.S) return;  // all sixteen lanes of a point or none
   const int s = (int)(i / J);
@@ -841,23 +844,32 @@ void Nufft::type1(const double2* c, double2* f, double* fr, double rscale,
     }
   }
   lists_.fill(a.g);
-  a.c = c;
-  a.fine = fine;
-  a.S = S;
+  // Groups of sb slices, as many to a launch as have their split tiles' scratch
+  // slots in 1 GB, at most 65535.
   const int sb = S <= 2 ? 2 : 4;
-  const unsigned ng = cdiv(S, sb);
-  DevBuf scratch(sizeof(double2) * (size_t)std::max(lists_.nslots(), 1) * ng *
-                 sb * SP_T * SP_T);
+  const size_t group_bytes = sizeof(double2) *
+                             (size_t)std::max(lists_.nslots(), 1) * sb * SP_T *
+                             SP_T;
+  const int most = (int)std::max<size_t>(
+      1, std::min<size_t>(65535, (size_t(1) << 30) / group_bytes));
+  const int groups = std::min((int)cdiv(S, sb), most);
+  DevBuf scratch(group_bytes * groups);
   auto k = sb == 2 ? spread_kernel<2> : spread_kernel<4>;
-  hipLaunchKernelGGL(k, dim3((unsigned)lists_.nwork(), ng),
-                     dim3(64 * SP_WAVES), 0, s, a,
-                     lists_.work(), scratch.as<double2>());
-  TC_HIP(hipGetLastError());
-  if (lists_.nfix()) {
-    hipLaunchKernelGGL(spread_fixup_kernel,
-                       dim3((unsigned)lists_.nfix(), ng, 4 * sb), dim3(256), 0, s,
-                       a, lists_.fix(), scratch.as<double2>(), sb);
+  for (int s0 = 0; s0 < S; s0 += groups * sb) {
+    a.c = c + (long)s0 * P_ * N_;
+    a.fine = fine + s0 * fplane;
+    a.S = std::min(S - s0, groups * sb);
+    const unsigned ng = cdiv(a.S, sb);
+    hipLaunchKernelGGL(k, dim3((unsigned)lists_.nwork(), ng),
+                       dim3(64 * SP_WAVES), 0, s, a, lists_.work(),
+                       scratch.as<double2>());
     TC_HIP(hipGetLastError());
+    if (lists_.nfix()) {
+      hipLaunchKernelGGL(spread_fixup_kernel,
+                         dim3((unsigned)lists_.nfix(), ng, 4 * sb), dim3(256),
+                         0, s, a, lists_.fix(), scratch.as<double2>(), sb);
+      TC_HIP(hipGetLastError());
+    }
   }
   // only the columns of the modes are read back
   fft2(fine, S, nf_, nf_, +1, s, (nm_ + 1) / 2, nm_ / 2, false, true);
@@ -879,10 +891,13 @@ void Nufft::type2_real(const double* f, double2* c, int S, hipStream_t s) {
   // rows without a mode are zero
   fft2(fine, S, nf_, nf_, -1, s, (nm_ + 1) / 2, nm_ / 2, true, false);
   GridArgs g{cs_.as<double2>(), P_, N_, nf_, S};
-  const long npts = (long)S * P_ * N_;
-  hipLaunchKernelGGL(interp_kernel, dim3(cdiv(16 * npts, 256)), dim3(256), 0, s,
-                     g, fine, c);
-  TC_HIP(hipGetLastError());
+  const long npts = (long)S * P_ * N_, most = 1L << 27;
+  for (long i0 = 0; i0 < npts; i0 += most) {
+    hipLaunchKernelGGL(interp_kernel,
+                       dim3(cdiv(16 * std::min(most, npts - i0), 256)),
+                       dim3(256), 0, s, g, fine, c, i0);
+    TC_HIP(hipGetLastError());
+  }
 }
 
 // ---------------------------------------------------------------------------
