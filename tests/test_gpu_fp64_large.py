@@ -11,17 +11,18 @@ from conftest import announce
 pytestmark = pytest.mark.gpu
 
 
-def test_many_points(torch_cuda):
+# 2^28 points and some, in many slices and in one
+@pytest.mark.parametrize("S,N,P", [(256, 16, 65600), (1, 64, (1 << 22) + 64)])
+def test_many_points(torch_cuda, S, N, P):
     torch = torch_cuda
     from tomocam_amd import gpu
-    S, N, P = 256, 16, 65600  # 2^28 points and some
     announce(f"FP64 project S={S} N={N} P={P}")
     ang = np.arange(P) * (np.pi / P)
     g = torch.Generator(device="cuda").manual_seed(1)
     x = torch.rand((S, N, N), device="cuda", generator=g, dtype=torch.float64)
     got = gpu.project(x, ang)
     pick = [0, 1, P // 2, P - 2, P - 1]
-    for s in (0, 127, 128, 255):
+    for s in sorted({0, S // 2 - 1, S // 2, S - 1} & set(range(S))):
         ref = gpu.project(x[s:s + 1], ang[pick])
         assert torch.equal(got[s, pick], ref[0])
     del got

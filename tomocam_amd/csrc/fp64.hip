@@ -969,51 +969,75 @@ static std::shared_ptr<Nufft> nufft_plan(const double* h_angles, int P, int N,
   return nu;
 }
 
+// Slices that the projectors take at once: their grids and samples within about
+// 2 GB, in batches of one size.  The buffers are the calling thread's cached ones
+// and stay after the call, so they must not grow with the stack.  (16 x 1400^2,
+// 2.5 GB, gradient: 56.3 ms in two batches, 55.8 in one.)
+static int slice_batch(int S, int P, int N, const Nufft& nu) {
+  const double per = 16.0 * ((double)nu.nf() * nu.nf() + 2.0 * P * N);
+  const int most = (int)std::max(1.0, std::min((double)S, 2.0e9 / per));
+  const int n = (int)cdiv(S, most);
+  return (int)cdiv(S, n);
+}
+
 void project(const double* img, double* sino, int S, int N,
              const double* h_angles, int P, hipStream_t s) {
   TC_REQUIRE(S >= 1 && N >= 2 && P >= 1, "FP64 project: bad shape");
   auto nu = nufft_plan(h_angles, P, N, N);
-  const long ns = (long)S * P * N;
-  DevBuf c(sizeof(double2) * ns), v(sizeof(double2) * ns);
-  nu->type2_real(img, c.as<double2>(), S, s);
   const double2* tw = roots(N);
-  hipLaunchKernelGGL((ray_dft_kernel<false, 1, false>), dim3(cdiv(ns, 256)),
-                     dim3(256), 0, s, c.as<void>(), v.as<double2>(),
-                     (long)S * P, N, tw);
-  TC_HIP(hipGetLastError());
-  hipLaunchKernelGGL(real_part_kernel, dim3(cdiv(ns, 256)), dim3(256), 0, s,
-                     v.as<double2>(), sino, ns, 1.0 / ((double)N * N));
-  TC_HIP(hipGetLastError());
+  const int B = slice_batch(S, P, N, *nu);
+  const long rays = (long)P * N;  // samples of a slice
+  DevBuf c(sizeof(double2) * B * rays), v(sizeof(double2) * B * rays);
+  for (int s0 = 0; s0 < S; s0 += B) {
+    const int nb = std::min(B, S - s0);
+    const long ns = nb * rays;
+    nu->type2_real(img + (long)s0 * N * N, c.as<double2>(), nb, s);
+    hipLaunchKernelGGL((ray_dft_kernel<false, 1, false>), dim3(cdiv(ns, 256)),
+                       dim3(256), 0, s, c.as<void>(), v.as<double2>(),
+                       (long)nb * P, N, tw);
+    TC_HIP(hipGetLastError());
+    hipLaunchKernelGGL(real_part_kernel, dim3(cdiv(ns, 256)), dim3(256), 0, s,
+                       v.as<double2>(), sino + s0 * rays, ns,
+                       1.0 / ((double)N * N));
+    TC_HIP(hipGetLastError());
+  }
 }
 
 void backproject(const double* sino, double* img, int S, int P, int N,
                  const double* h_angles, bool fbp, hipStream_t s) {
   TC_REQUIRE(S >= 1 && N >= 2 && P >= 1, "FP64 backproject: bad shape");
   auto nu = nufft_plan(h_angles, P, N, N);
-  const long ns = (long)S * P * N;
-  DevBuf v(sizeof(double2) * ns);
   const double2* tw = roots(N);
-  if (fbp)
-    hipLaunchKernelGGL((ray_dft_kernel<true, -1, true>), dim3(cdiv(ns, 256)),
-                       dim3(256), 0, s, sino, v.as<double2>(), (long)S * P, N,
-                       tw);
-  else
-    hipLaunchKernelGGL((ray_dft_kernel<true, -1, false>), dim3(cdiv(ns, 256)),
-                       dim3(256), 0, s, sino, v.as<double2>(), (long)S * P, N,
-                       tw);
-  TC_HIP(hipGetLastError());
-  nu->type1(v.as<double2>(), nullptr, img, 1.0 / ((double)N * N), S, s);
+  const int B = slice_batch(S, P, N, *nu);
+  const long rays = (long)P * N;
+  DevBuf v(sizeof(double2) * B * rays);
+  auto dft = fbp ? ray_dft_kernel<true, -1, true>
+                 : ray_dft_kernel<true, -1, false>;
+  for (int s0 = 0; s0 < S; s0 += B) {
+    const int nb = std::min(B, S - s0);
+    hipLaunchKernelGGL(dft, dim3(cdiv(nb * rays, 256)), dim3(256), 0, s,
+                       (const void*)(sino + s0 * rays), v.as<double2>(),
+                       (long)nb * P, N, tw);
+    TC_HIP(hipGetLastError());
+    nu->type1(v.as<double2>(), nullptr, img + (long)s0 * N * N,
+              1.0 / ((double)N * N), nb, s);
+  }
 }
 
 void gradient_nufft(const double* x, const double* b, double* g, int S, int N,
                     const double* h_angles, int P, hipStream_t s) {
   TC_REQUIRE(S >= 1 && N >= 2 && P >= 1, "FP64 gradient: bad shape");
   auto nu = nufft_plan(h_angles, P, N, N);
-  const long ns = (long)S * P * N;
-  DevBuf c(sizeof(double2) * ns);
-  nu->type2_real(x, c.as<double2>(), S, s);
-  nu->type1(c.as<double2>(), nullptr, g, 1.0 / ((double)N * N * N), S, s);
-  if (b) axpby(g, b, g, (long)S * N * N, 1.0, -1.0, s);
+  const int B = slice_batch(S, P, N, *nu);
+  const long img = (long)N * N;
+  DevBuf c(sizeof(double2) * (size_t)B * P * N);
+  for (int s0 = 0; s0 < S; s0 += B) {
+    const int nb = std::min(B, S - s0);
+    nu->type2_real(x + s0 * img, c.as<double2>(), nb, s);
+    nu->type1(c.as<double2>(), nullptr, g + s0 * img,
+              1.0 / ((double)N * N * N), nb, s);
+  }
+  if (b) axpby(g, b, g, S * img, 1.0, -1.0, s);
 }
 
 // ---------------------------------------------------------------------------
