@@ -7,7 +7,7 @@
 //   twiddle  w_L^(r (j mod Ns) L/(Ns R)), from the stage's table [r - 1][k]
 //            of (R - 1) Ns values (k = j mod Ns)
 //   outputs  y[(j - j mod Ns) R + (j mod Ns) + r Ns]
-// Each radix-R DFT (R up to 27, composite radices by Cooley-Tukey in
+// Each radix-R DFT (R up to 36, composite radices by Cooley-Tukey in
 // registers) runs entirely in registers; consecutive stages exchange data
 // through one LDS line (write outputs, barrier, read inputs, barrier).
 // Stage-1 inputs t + i T + r L/R_1 and last-stage outputs t + i T + r L/R_S

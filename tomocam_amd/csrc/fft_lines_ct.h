@@ -75,12 +75,12 @@ struct LinePlan {
   }
 };
 
-// Line l of batch b starts at b * bstride + (l / lgroup) * lstride +
-// l % lgroup; element i at + i * estride.  Of a line, the elements [0, nin) and [L - nin_hi, L) are
-// read (the others are zero) and [0, nout) and [L - nout_hi, L) written.
-// COL: the workgroup's lines are adjacent columns, so consecutive threads
-// take consecutive lines (coalesced loads of a row); otherwise consecutive
-// threads take consecutive elements of one line.
+// Line l of batch b starts at b * bstride + (l / lgroup) * lstride + l %
+// lgroup; element i at + i * estride.  Of a line, the elements [0, nin) and [L
+// - nin_hi, L) are read (the others are zero) and [0, nout) and [L - nout_hi,
+// L) written.  COL: the workgroup's lines are adjacent columns, so consecutive
+// threads take consecutive lines (coalesced loads of a row); otherwise
+// consecutive threads take consecutive elements of one line.
 template <class P, int DIR, bool COL>
 __global__ void __launch_bounds__(P::NT)
 ct_lines_kernel(const float2* in, float2* out, const float2* __restrict__ tw,
@@ -531,7 +531,8 @@ struct LineOps {
 // Plans, ascending: length, elements per thread, lines per workgroup and
 // radices (each divides the elements per thread).  From 192 on the lengths are
 // at most 1/8 apart, but for 216 to 256, 324 to 384 and 648 to 768 (18.5 %), so
-// that a chirp length rounded up to one costs little; radices of 8 to 36 keep the LDS exchanges at one to three.
+// that a chirp length rounded up to one costs little; radices of 8 to 36 keep
+// the LDS exchanges at one to three.
 #define TC_FOR_LINE_LENGTHS_1(X) \
   X(64) X(96) X(128) X(144) X(192) X(216) X(256) X(288) X(324) X(384) X(432)
 #define TC_FOR_LINE_LENGTHS_2(X) \

@@ -48,8 +48,9 @@ __device__ __forceinline__ unsigned half_at(int L, int row, int col) {
   return (unsigned)(((col / HG_B) * L + row) * HG_B + col % HG_B);
 }
 
-// Rows of nm real modes <-> the half of an L x L Hermitian grid.  Mode index k stands for k - floor(nm/2); row k of
-// slice s is grid row (k - floor(nm/2)) mod L.
+// Rows of nm real modes <-> the half of an L x L Hermitian grid.  Mode index k
+// stands for k - floor(nm/2); row k of slice s is grid row (k - floor(nm/2))
+// mod L.
 //   r2c: half = forward row transforms of real_in, each value times
 //        corr[row] corr[column]; only the nm mode rows are written;
 //   c2r: real_out = scale corr corr times the inverse (exp(+i), unnormalised)

@@ -1,5 +1,5 @@
-// Polar-grid NUFFT (tile-owned LDS spreading, gather interpolation),
-// Bluestein ray DFT and the projectors built on them.
+// Polar-grid NUFFT (tile-owned spreading on the matrix cores, gather
+// interpolation), ray DFT (direct or Bluestein) and the projectors built on them.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -25,8 +25,9 @@ namespace tc {
 // Type 1 takes the exponent as -beta z^2 / (1 + sqrt(1 - z^2)): the difference
 // sqrt - 1 carries the root's rounding, times beta, into the weights near the
 // kernel's centre, a level error of up to 6e-7 of an image.  Type 2 keeps the
-// difference form (its weights are those of the earlier kernels, bit for bit),
-// because a residual P x - y amplifies any change of level in P x.
+// difference form.  The other would be more exact there too (the gradient of
+// 1/2 |P x - y|^2 at 8 x 512^2 is 2.3e-5 off 64 bits, 3.5e-6 with it), but that
+// gradient amplifies any change of P x's level, and would move by more than 2e-5.
 __device__ __forceinline__ float es_kernel(float z, float beta) {
   const float s = fmaf(-z, z, 1.0f);
   const float r = __builtin_amdgcn_sqrtf(fmaxf(s, 0.f)) + 1.0f;
@@ -327,9 +328,9 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
 // whose slots would be a long chain, one cell and sixteen slots at a time, four
 // workgroups a tile.  (All tiles that way: 22 instead of 11 us at 8 x 512^2,
 // where most tiles have few slots; none: 36 instead of 17 us at 8 x 2048^2, whose
-// centre has 211 slots.)  The order per cell is slot order.  The sums are FP64: the centre's cells add a value of the same sign
-// from every ray over many slots, and their rounding is a level error of the
-// whole image.
+// centre has 211 slots.)  The order per cell is slot order.  The sums are FP64:
+// the centre's cells add a value of the same sign from every ray over many
+// slots, and their rounding is a level error of the whole image.
 template <int PER, int U>
 __device__ __forceinline__ void spread_fixup(const SpreadArgs& a, int4 f, int s,
                                              const float2* base,
@@ -420,9 +421,9 @@ struct InterpArgs {
 // adjacent bytes a point (weights past the footprint are zero).  The loads
 // are bound by the cache lines they touch, about 10 a point and slice; one
 // column a lane, row by row, touched about 22 (8 x 1024^2 at 720 angles:
-// 117 -> 91 us; 8 x 512^2 at 360: 41 -> 27 us).  Where the three blocks reach past the stored half (near columns 0
-// and nf/2) the wave takes that form: lane b reads footprint column b of
-// every row, or its mirror image.
+// 117 -> 91 us; 8 x 512^2 at 360: 41 -> 27 us).  Where the three blocks reach
+// past the stored half (near columns 0 and nf/2) the wave takes that form: lane
+// b reads footprint column b of every row, or its mirror image.
 //
 // The eight lanes' sums are then added across the group for eight slices at
 // once by a transposing butterfly (exchange halves with lanes b^4, b^2, b^1:
@@ -599,6 +600,7 @@ PolarNufft::PolarNufft(const float* h_angles, int nproj, int npix, int nmodes)
     : P_(nproj), N_(npix), nm_(nmodes) {
   ArenaPause no_arena;  // cached plan, tables filled synchronously
   TC_REQUIRE(nproj >= 1 && npix >= 2 && nmodes >= 1, "NUFFT: bad geometry");
+  // (a limit of the FP32 entry points; the lists would take more)
   TC_REQUIRE(nproj <= 2048, "NUFFT: too many projection angles");
   TC_REQUIRE(npix < 65536, "NUFFT: too many samples per ray");
   nf_ = grid_length(std::max(2 * nmodes, 2 * NUFFT_W), true);
@@ -893,8 +895,11 @@ RayDft::RayDft(int N, int sign) : N_(N) {
   TC_REQUIRE(N >= 1, "ray DFT: N must be >= 1");
   direct_ = fft_lines_ct_has(N);
   if (direct_) fft_prepare(N);
-  // The chirp-z length: a planned FFT length where there is one (the planned
-  // kernel runs forward transform, multiply and inverse in registers)
+  // The chirp-z length.  Backward a planned FFT length where there is one (the
+  // planned kernel runs forward transform, multiply and inverse in registers).
+  // Forward the rule of the fine grids, whose lengths have a plan at about half of
+  // the widths: another length rounds P x differently, which residuals P x - y
+  // amplify (es_kernel above).
   if (sign < 0) {
     const int c = fft_lines_ct_length(2 * N - 1);
     L_ = c > 0 ? c : fft_next_smooth(2 * N - 1, false);

@@ -67,10 +67,11 @@ static std::pair<int, int> len_key(int n) {
 // the cheapest plan of any kind within 1/7 of the smallest even smooth length,
 // which every width from 243 to 4096 has (there without the mixed forms, see
 // has_mixed), else that length.  Runtime-plan kernels against the plan: 2 x 849^2
-// 98 and 54 us; 4 x 330^2, 672 and 768 points, 35 and 27 us; 2 x 1310^2, 2646 and 2916, 280
-// and 72 us; 2 x 2620^2, 5250 and 5832, 1003 and 293 us; 2 x 3000^2, 6000 and
-// 6144, 1279 and 425 us.  Shorter lengths have no plans: trial ones took 13.5
-// instead of 18.8 us at 1 x 128^2 and 21.1 instead of 23.9 at 1 x 181^2.
+// 98 and 54 us; 4 x 330^2, 672 and 768 points, 35 and 27 us; 2 x 1310^2, 2646
+// and 2916, 280 and 72 us; 2 x 2620^2, 5250 and 5832, 1003 and 293 us; 2 x
+// 3000^2, 6000 and 6144, 1279 and 425 us.  Shorter lengths have no plans: trial
+// ones took 13.5 instead of 18.8 us at 1 x 128^2 and 21.1 instead of 23.9 at 1
+// x 181^2.
 int toeplitz_fft_length(int n) {
   {
     // (no device query while nothing is tuned: the rule works without one)
