@@ -327,10 +327,11 @@ spread_kernel(SpreadArgs a, const int4* __restrict__ work, float2* scratch) {
 // slots, four slots at a time (16 loads in flight); of the first nheavy tiles,
 // whose slots would be a long chain, one cell and sixteen slots at a time, four
 // workgroups a tile.  (All tiles that way: 22 instead of 11 us at 8 x 512^2,
-// where most tiles have few slots; none: 36 instead of 17 us at 8 x 2048^2, whose
-// centre has 211 slots.)  The order per cell is slot order.  The sums are FP64:
-// the centre's cells add a value of the same sign from every ray over many
-// slots, and their rounding is a level error of the whole image.
+// where most tiles have few slots; none: 32 instead of 19 us at 8 x 2048^2,
+// whose centre has 211 slots, 14 instead of 12 at 8 x 512^2.)  The order per
+// cell is slot order.  The sums are FP64: the centre's cells add a value of the
+// same sign from every ray over many slots, and their rounding is a level error
+// of the whole image.
 template <int PER, int U>
 __device__ __forceinline__ void spread_fixup(const SpreadArgs& a, int4 f, int s,
                                              const float2* base,
