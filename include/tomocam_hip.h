@@ -120,9 +120,11 @@ int tc_psf_destroy(tc_psf p);
 int tc_psf_info(tc_psf p, int* n, int* fft_size);
 
 /* The FFT size M a PSF of width n would use (M >= 2n - 1; the reference
- * uses 2n - 1, src/toeplitz.h:57-60): the smallest length with compile-time
- * passes when within 10 % of the smallest even 2,3,5,7-smooth length, else
- * that.  No GPU needed. */
+ * uses 2n - 1, src/toeplitz.h:57-60): the cheapest length that has
+ * compile-time passes with mixed-precision forms and is within 10 % of the
+ * smallest even 2,3,5,7-smooth length; with none, for widths from 243 on the
+ * cheapest that has FP32 passes and is within 1/7 of it; else that length.
+ * No GPU needed. */
 int tc_toeplitz_fft_length(int n, int* fft_size);
 
 /* PointSpreadFunction::convolve (src/toeplitz.h:95-101):
@@ -171,7 +173,7 @@ int tc_psf_tune(tc_psf p, int nslices, int mixed, int* group, void* stream);
  * 768 for n = 350 ... 362, 2250 and 2304, 4500 and 4608), times one FP32
  * application of each on `nslices` slices of scratch data and rebuilds the
  * handle's spectrum at the faster one; the static rule's choice is kept
- * unless the other is at least 2 % faster.  The choice holds for this width
+ * unless the other is at least 5 % faster.  The choice holds for this width
  * for the rest of the process (later handles and tc_toeplitz_fft_length
  * use it).  *fft_size (optional) receives the handle's FFT length.
  * tc_mbir2 / tc_mbir2_mixed run it on first use of a width unless

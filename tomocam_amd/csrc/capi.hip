@@ -317,8 +317,9 @@ int tc_toeplitz_apply_mixed(tc_psf p, const float* d_x, float* d_out,
     TC_REQUIRE(d_x && d_out, "null argument");
     TC_REQUIRE(nslices >= 1, "Toeplitz: need at least one slice");
     TC_REQUIRE(P.has_mixed(), "mixed precision needs a compile-time FFT "
-                              "plan; FFT length " + std::to_string(P.M()) +
-                              " has none");
+                              "plan with FP16 forms; width " +
+                              std::to_string(P.n()) + " (FFT length " +
+                              std::to_string(P.M()) + ") has none");
     hipStream_t s = as_stream(stream);
     tc::DevBuf x16(tc::half_pair_bytes(nslices, P.n(), P.n()));
     tc::DevBuf gsc(sizeof(float) * (size_t)nslices);

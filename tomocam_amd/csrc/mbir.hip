@@ -922,8 +922,9 @@ Run2Stats run2_device(Psf& psf, const float* x0, const float* b, float* out,
   float *gsc = nullptr, *gsc_next = nullptr;
   if (opt.mixed) {
     TC_REQUIRE(psf.has_mixed(),
-               "mixed precision needs a compile-time FFT plan; FFT length " +
-                   std::to_string(psf.M()) + " has none");
+               "mixed precision needs a compile-time FFT plan with FP16 "
+               "forms; width " + std::to_string(psf.n()) + " (FFT length " +
+                   std::to_string(psf.M()) + ") has none");
     bg16.alloc(half_pair_bytes(S, n, n));
     bgsc.alloc(sizeof(float) * 2 * (size_t)S);
     bgmax.alloc(sizeof(float) * (size_t)qblk * QWAVES * qa.zchunk);

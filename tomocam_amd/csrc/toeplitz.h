@@ -1,8 +1,8 @@
 // Toeplitz (PSF-convolution) normal operator T x = sum_q x[q] PSF(a-q) / n^3.
 //
 // Reference: PointSpreadFunction<T> (src/toeplitz.h:33-160).  The PSF is
-// placed circularly on an M x M grid (M = smallest even 2,3,5,7-smooth size
-// >= 2n-1), whose spectrum is real and even.  One application is three
+// placed circularly on an M x M grid (M >= 2n-1 even and 2,3,5,7-smooth:
+// toeplitz_fft_length), whose spectrum is real and even.  One application is three
 // passes over HBM:
 //   A  pair-packed real row FFTs of the n non-zero rows -> Wt
 //      (k1 < H = M/2+1, stored k1-major so pass B reads whole columns);
@@ -138,6 +138,7 @@ class Psf {
                      int mode, double* dot_partials, float2* wt,
                      hipStream_t stream);
   int n_, M_, H_, rp_;
+  bool mixed_ = false;  // has_mixed
   DevBuf arr_;
   DevBuf spec_;
   DevBuf work_;

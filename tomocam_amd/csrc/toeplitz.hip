@@ -134,6 +134,9 @@ Psf::Psf(const float* d_psf, int n, hipStream_t stream) : n_(n) {
 void Psf::build_spectrum(int M, hipStream_t stream) {
   M_ = M;
   H_ = M_ / 2 + 1;
+  // the mixed forms serve the widths whose smooth length is within 10 %
+  const std::vector<int> c10 = toeplitz_ct_candidates(n_);
+  mixed_ = std::find(c10.begin(), c10.end(), M_) != c10.end();
   {
     ArenaPause no_arena;  // process-lifetime tables
     if (!toeplitz_ct_prepare(M_)) fft_length(M_);
@@ -526,11 +529,7 @@ bool Psf::run_half(const void* g16, const float* gsc, float* out,
 }
 
 bool Psf::has_fused() const { return toeplitz_ct_lpw(M_) > 0; }
-bool Psf::has_mixed() const {
-  // the mixed forms serve the widths whose smooth length is within 10 %
-  const std::vector<int> c = toeplitz_ct_candidates(n_);
-  return std::find(c.begin(), c.end(), M_) != c.end();
-}
+bool Psf::has_mixed() const { return mixed_; }
 
 void toeplitz_set_group(int H, int rp, int elem_bytes, int nslices,
                         int group);
