@@ -17,7 +17,8 @@ constexpr int SP_T = 32;  // tile edge (grid points)
 // random: a level error of the whole image or PSF (T x of 1454^2 at 720 angles
 // against 64 bits: 6.3e-7 with items of 1024 points there, 3.8e-6 with 4096).
 // The tiles that hold such cells are cut into items of SP_CENTRE_CHUNK points,
-// whose sums the fix-up adds in FP64: 6.4e-8.
+// whose sums the fix-up adds in FP64: 6.4e-8.  (FP32 lists only: FP64 sums need
+// no such care, and their angles have no limit that would bound the slots.)
 constexpr int SP_CENTRE = 8, SP_CENTRE_CHUNK = 128;
 
 struct TileGeom {
@@ -87,9 +88,9 @@ class TileLists {
   // Points per tile and every tile's segments, for kernel width W (8 or 16);
   // reads the counts back (one synchronisation).  g: ax .. umax filled in.
   void make_segments(const TileGeom& g, int W, hipStream_t stream);
-  // The work and fix-up lists for `chunk` points per item (the tiles about the
-  // centre: at most SP_CENTRE_CHUNK).  Synchronous copies: the caller has no
-  // kernel reading the previous lists in flight.
+  // The work and fix-up lists for `chunk_max` points per item (FP32: the tiles
+  // about the centre at most SP_CENTRE_CHUNK).  Synchronous copies: the caller
+  // has no kernel reading the previous lists in flight.
   void make_work(int chunk_max);
   void fill(TileGeom& g) const;  // the list pointers
 
@@ -113,7 +114,7 @@ class TileLists {
  private:
   int nwork_ = 0, nslots_ = 0, nfix_ = 0, nheavy_ = 0, chunk_ = 0;
   std::vector<int> counts_;      // polar points per tile
-  std::vector<char> centre_;     // whether it holds cells about the centre
+  std::vector<char> centre_;     // tiles cut into items of SP_CENTRE_CHUNK
   std::vector<int> tile_first_;  // first segment of each tile
   DevBuf seg_, seg_off_, tile_seg_;
   // two int4 per item: tile, first point, end point, scratch slot (-1: none);

@@ -150,7 +150,7 @@ void TileLists::make_segments(const TileGeom& geom, int W, hipStream_t stream) {
       return i * SP_T <= g.nf / 2 + SP_CENTRE &&
              (i + 1) * SP_T > g.nf / 2 - SP_CENTRE;
     };
-    centre_[t] = near(t / g.ntx) && near(t % g.ntx);
+    centre_[t] = W == 8 && near(t / g.ntx) && near(t % g.ntx);
   }
   tile_first_.assign(ntiles + 1, 0);
   for (int t = 0; t < ntiles; ++t)
@@ -167,7 +167,7 @@ void TileLists::make_segments(const TileGeom& geom, int W, hipStream_t stream) {
   TC_HIP(hipGetLastError());
 }
 
-// The work and fix-up lists for `chunk` points per item, uploaded to the
+// The work and fix-up lists for `chunk_max` points per item, uploaded to the
 // plan's buffers (synchronous copies: the caller has no kernel reading the
 // previous lists in flight).
 void TileLists::make_work(int chunk_max) {
