@@ -144,13 +144,13 @@ void TileLists::make_segments(const TileGeom& geom, int W, hipStream_t stream) {
                         hipMemcpyDeviceToHost, stream));
   TC_HIP(hipStreamSynchronize(stream));
   counts_.assign(h.begin(), h.begin() + ntiles);
-  centre_.resize(ntiles);
-  for (int t = 0; t < ntiles; ++t) {
-    auto near = [&](int i) {  // tile i along an axis
-      return i * SP_T <= g.nf / 2 + SP_CENTRE &&
-             (i + 1) * SP_T > g.nf / 2 - SP_CENTRE;
-    };
-    centre_[t] = W == 8 && near(t / g.ntx) && near(t % g.ntx);
+  centre_.assign(ntiles, 0);
+  if (W == 8) {
+    const int lo = std::max(0, (g.nf / 2 - SP_CENTRE) / SP_T);
+    const int hi = (g.nf / 2 + SP_CENTRE) / SP_T;
+    for (int ty = lo; ty <= std::min(hi, ntiles / g.ntx - 1); ++ty)
+      for (int tx = lo; tx <= std::min(hi, g.ntx - 1); ++tx)
+        centre_[ty * g.ntx + tx] = 1;
   }
   tile_first_.assign(ntiles + 1, 0);
   for (int t = 0; t < ntiles; ++t)
